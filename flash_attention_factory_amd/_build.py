@@ -8,6 +8,9 @@ _PKG = os.path.dirname(os.path.abspath(__file__))
 SOURCE = os.path.join(_PKG, "csrc", "fa_paged_attention.hip")
 LIBRARY = os.path.join(_PKG, "libfa_paged_attention.so")
 
+TORCH_OPS_SOURCE = os.path.join(_PKG, "csrc", "torch_ops.cpp")
+TORCH_OPS_LIBRARY = os.path.join(_PKG, "libfa_torch_ops.so")
+
 HIPCC_FLAGS = [
     "--offload-arch=gfx950", "-O3", "-std=c++17", "-fPIC", "-shared", "-fvisibility=hidden",
     # packed-fp32 instructions are kept out of the generated code on purpose
@@ -27,6 +30,23 @@ def build(verbose: bool = False, extra_flags=(), output: str = LIBRARY) -> str:
     res = subprocess.run(cmd, capture_output=True, text=True)
     if res.returncode != 0:
         raise RuntimeError(f"hipcc failed ({res.returncode}):\n{res.stdout}\n{res.stderr}")
+    return output
+
+
+def build_torch_ops(verbose: bool = False, output: str = TORCH_OPS_LIBRARY) -> str:
+    """The native operators of torch.ops.fa_amd (host code only)."""
+    import torch
+    root = os.path.dirname(torch.__file__)
+    cmd = [os.environ.get("CXX", "g++"), "-O2", "-std=c++17", "-fPIC", "-shared", "-Wall", "-fvisibility=hidden",
+           "-D__HIP_PLATFORM_AMD__=1", "-DUSE_ROCM=1", f"-D_GLIBCXX_USE_CXX11_ABI={int(torch._C._GLIBCXX_USE_CXX11_ABI)}",
+           "-isystem", os.path.join(root, "include"), "-isystem", os.path.join(root, "include", "torch", "csrc", "api", "include"),
+           "-isystem", "/opt/rocm/include", TORCH_OPS_SOURCE, "-o", output, "-L" + os.path.join(root, "lib"),
+           "-ltorch", "-ltorch_cpu", "-lc10", "-lc10_hip"]
+    if verbose:
+        print(" ".join(cmd), flush=True)
+    res = subprocess.run(cmd, capture_output=True, text=True)
+    if res.returncode != 0:
+        raise RuntimeError(f"{cmd[0]} failed ({res.returncode}):\n{res.stdout}\n{res.stderr}")
     return output
 
 

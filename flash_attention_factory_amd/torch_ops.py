@@ -36,19 +36,25 @@ explicit 0 checks nothing and warns of nothing.
 Caches are ``[blocks, block_size, kv_heads, head_size]`` views as in ``lib.*.run``; every
 output is an argument the operator mutates, nothing is allocated.  Importing this module
 registers the operators; there is no CPU implementation.
+
+The operators of ``torch.ops.fa_amd`` are native (csrc/torch_ops.cpp, ``libfa_torch_ops.so``).  The functions below
+are the same operators in Python, in the namespace ``fa_amd_py``: they say what a valid call is, and every call
+that the native ones do not launch -- an invalid one, above all -- ends there.
 """
 from __future__ import annotations
 
+import ctypes
 from typing import Optional
 
 import torch
 from torch import Tensor
 
+from . import _build, _cabi
 from .lib import (kv_cache_write as _kv_cache_write, paged_attention_fp8_loop as _fp8_loop,
                   paged_attention_fp8_reduce as _fp8_reduce, paged_attention_loop as _loop,
                   paged_attention_reduce as _reduce)
 
-_NS = "fa_amd"
+_NS = "fa_amd_py"
 
 
 def _group(query: Tensor, key_cache: Tensor) -> int:
@@ -143,7 +149,25 @@ def kv_cache_write(key: Tensor, value: Tensor, key_cache: Tensor, value_cache: T
                         k_scales=k_scales, v_scales=v_scales)
 
 
+_NAMES = ("paged_attention_loop", "paged_attention_fp8_loop", "paged_attention_reduce", "paged_attention_fp8_reduce",
+          "kv_cache_write")
+
+
+def _load_native() -> None:
+    torch.ops.load_library(_build.TORCH_OPS_LIBRARY)
+    L = _cabi.load()
+    entries = (L.fa_paged_attention_loop, L.fa_paged_attention_fp8_loop, L.fa_paged_attention_reduce,
+               L.fa_paged_attention_fp8_reduce, L.fa_kv_cache_write)
+    table = (ctypes.c_void_p * len(entries))(*(ctypes.cast(e, ctypes.c_void_p).value for e in entries))
+    bind = ctypes.CDLL(_build.TORCH_OPS_LIBRARY).fa_torch_ops_bind
+    bind.argtypes, bind.restype = [ctypes.c_void_p, ctypes.c_size_t], None
+    bind(table, len(entries))
+
+
+_load_native()
+
 # Shape propagation for tracing: every operator only writes into its arguments.
-for _op in (paged_attention_loop, paged_attention_fp8_loop, paged_attention_reduce, paged_attention_fp8_reduce,
-            kv_cache_write):
-    _op.register_fake(lambda *args, **kwargs: None)
+for _name in _NAMES:
+    globals()[_name].register_fake(lambda *args, **kwargs: None)
+    torch.library.register_fake(f"fa_amd::{_name}", lambda *args, **kwargs: None)
+    globals()[_name] = getattr(torch.ops.fa_amd, _name)
