@@ -41,6 +41,7 @@ EXPORTS = (
     "fa_paged_attention_kernel_status",
     "fa_paged_attention_reduce_plan",
     "fa_paged_attention_init",
+    "fa_paged_attention_loop_workspace_bytes",
 )
 
 ABI_REVISION = 8
@@ -121,6 +122,14 @@ class Options(_Versioned):
         ("schedule", ctypes.c_int32),
         ("spin_limit", ctypes.c_int32),
         ("segment_partitions", ctypes.c_int32),
+    ]
+
+
+class OptionsWorkspace(Options):
+    """Options with memory for the single-pass entries to work in (fa_paged_attention_options_workspace)."""
+    _fields_ = [
+        ("workspace", ctypes.c_void_p),
+        ("workspace_bytes", ctypes.c_int64),
     ]
 
 
@@ -215,6 +224,8 @@ def load() -> ctypes.CDLL:
         fn = getattr(L, name)
         fn.argtypes = common + [P, P, P] + tail
         fn.restype = ctypes.c_int32
+    L.fa_paged_attention_loop_workspace_bytes.argtypes = tail + [ctypes.c_int32]
+    L.fa_paged_attention_loop_workspace_bytes.restype = ctypes.c_int64
     L.fa_kv_cache_write.argtypes = [P, P, P, P, P, ctypes.POINTER(KvWriteShape), ctypes.POINTER(Options)]
     L.fa_kv_cache_write.restype = ctypes.c_int32
     L.fa_last_error.restype = ctypes.c_char_p

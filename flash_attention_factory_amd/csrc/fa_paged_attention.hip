@@ -24,7 +24,26 @@ FA_EXPORT int32_t fa_paged_attention_loop(void *out, const void *query, const vo
   const fa_status st = fa::read_call_structs(shape, options, &c);
   if (st != FA_OK) return st;
   return fa::dispatch_paged_attention_loop(out, query, key_cache, value_cache, block_tables,
-                                           context_lens, scale, max_context_len, &c.shape, c.options());
+                                           context_lens, scale, max_context_len, &c.shape, c.options(), c.workspace,
+                                           c.workspace_bytes);
+}
+
+FA_EXPORT int64_t fa_paged_attention_loop_workspace_bytes(const fa_paged_attention_shape *shape,
+                                                          const fa_paged_attention_options *options, int32_t kv_fp8) {
+  fa::CallStructs c;
+  if (fa::read_call_structs(shape, options, &c) != FA_OK) return 0;
+  // the checks of a call, made on placeholders: nothing is launched and no pointer is followed
+  static float placeholder[4] __attribute__((aligned(16)));
+  fa_paged_attention_options op = c.has_options ? c.options_storage : fa_paged_attention_options{};
+  op.struct_size = sizeof(op);
+  op.validate_only = 1;
+  void *any = placeholder;
+  const int32_t *ints = reinterpret_cast<const int32_t *>(placeholder);
+  fa::Resolved r;
+  if (fa::validate_and_resolve(any, any, any, any, ints, ints, 0, nullptr, nullptr, nullptr, &c.shape, &op, kv_fp8 != 0,
+                               /*split=*/false, &r) != FA_OK)
+    return 0;
+  return fa::row_merge_space(c.shape, r, 0).bytes;
 }
 
 FA_EXPORT int32_t fa_paged_attention_reduce(void *out, const void *query, const void *key_cache,
@@ -127,7 +146,7 @@ FA_EXPORT int32_t fa_paged_attention_fp8_loop(void *out, const void *query, cons
   if (st != FA_OK) return st;
   return fa::dispatch_paged_attention_fp8_loop(out, query, key_cache, value_cache, block_tables,
                                                context_lens, scale, max_context_len, &c.shape,
-                                               c.options());
+                                               c.options(), c.workspace, c.workspace_bytes);
 }
 
 FA_EXPORT int32_t fa_paged_attention_fp8_reduce(void *out, const void *query,

@@ -107,12 +107,22 @@ struct CallStructs {
   fa_paged_attention_shape shape;
   fa_paged_attention_options options_storage;
   bool has_options = false;
+  void *workspace = nullptr;  // of fa_paged_attention_options_workspace
+  int64_t workspace_bytes = 0;
   const fa_paged_attention_options *options() const { return has_options ? &options_storage : nullptr; }
 };
 
 inline fa_status read_options(const fa_paged_attention_options *options, CallStructs *c) {
   c->has_options = options != nullptr;
   if (!options) return FA_OK;
+  if (options->struct_size == sizeof(fa_paged_attention_options_workspace)) {
+    const auto *full = reinterpret_cast<const fa_paged_attention_options_workspace *>(options);
+    c->options_storage = full->options;
+    c->options_storage.struct_size = (uint32_t)sizeof(c->options_storage);
+    c->workspace = full->workspace;
+    c->workspace_bytes = full->workspace_bytes;
+    return FA_OK;
+  }
   return read_versioned(options, &c->options_storage, sizeof(uint32_t), "options");
 }
 
@@ -163,6 +173,10 @@ struct Resolved {
   float *elapsed_us;
   bool validate_only;
   const void *sinks;
+  int32_t max_context_len;  // as the caller passed it; 0: unknown
+  // loop entries: memory for the pieces of rows that the launch cuts (launch_kernels_loop.h); NULL: rows stay whole
+  void *workspace;
+  int64_t workspace_bytes;
   fa_split_plan *plan;  // non-NULL: the split launcher fills this in where it would launch, and launches nothing
 };
 
@@ -283,6 +297,9 @@ inline fa_status validate_and_resolve(const void *out, const void *query, const 
   r->validate_only = o && o->validate_only != 0;
   r->sinks = o ? o->sinks : nullptr;
   r->plan = nullptr;
+  r->max_context_len = max_context_len;
+  r->workspace = nullptr;
+  r->workspace_bytes = 0;
   r->status = nullptr;
   r->spin_limit = spin_limit_of(o);
   if (!r->validate_only) return kernel_status_of_current_device(&r->status);
@@ -367,6 +384,10 @@ inline PagedAttnParams make_params(void *out, float *exp_sums, float *max_logits
   p.kv_head_bytes = s.kv_head_stride * r.kv_elem_bytes;
   p.compute_units = 0;  // the split path's launcher fills it in
   p.final_out = nullptr;  // (and this, in the segment form)
+  p.merge_pieces = nullptr;  // (these, the loop path's launcher where rows are cut)
+  p.merge_flags = nullptr;
+  p.merge_nonce = 0;
+  p.merge_whole_partitions = 0;
   p.kv_rows_apart = s.kv_token_stride != s.head_size;
   p.segment_force = r.segment_partitions;
   p.pair_heads = 0;

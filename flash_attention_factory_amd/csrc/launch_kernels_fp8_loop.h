@@ -17,10 +17,11 @@ inline fa_status dispatch_paged_attention_fp8_loop(void *out, const void *query,
                                                    const int32_t *context_lens, float scale,
                                                    int32_t max_context_len,
                                                    const fa_paged_attention_shape *shape,
-                                                   const fa_paged_attention_options *options) {
+                                                   const fa_paged_attention_options *options, void *workspace,
+                                                   int64_t workspace_bytes) {
   return dispatch_paged_attention_loop_any<true>(out, query, key_cache, value_cache, block_tables,
                                                  context_lens, scale, max_context_len, shape,
-                                                 options);
+                                                 options, workspace, workspace_bytes);
 }
 
 }  // namespace fa

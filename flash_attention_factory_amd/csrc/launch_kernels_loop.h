@@ -8,6 +8,8 @@
 #pragma once
 
 #include <algorithm>
+#include <atomic>
+#include <chrono>
 
 #include "launch_common.h"
 
@@ -37,6 +39,86 @@
 
 namespace fa {
 
+// ---- rows cut into pieces -----------------------------------------------------------------------
+// A launch of few rows leaves most compute units idle, or waits for its longest row.  Given workspace, it cuts its
+// rows (paged_attention_row_merge.h) where that pays.  The host knows the number of rows and a bound on their length;
+// whether the rows at hand are worth it the device decides (cut_pays).  Back to back, us, whole -> cut:
+//   8 rows of 30011 keys 402 -> 32 (the split path's two kernels: 37), 24 rows of 900-4096 keys 49 -> 18, 110 rows
+//   of 622-5556 keys 53 -> 19, 64 rows of 8192-32768 keys 432 -> 113 (floor 103), 320 rows of 2698-5095 keys 146 -> 105
+// Beyond kRowMergeMaxItems rows units have two rows each and cutting gives little: 416 to 720 rows measured between
+// 0.91 and 1.02 of the whole rows' speed.  Rows that stay whole cost 0.1 to 1 us more here than in the persistent loop
+// kernel (16-bit cache 6.7 -> 6.9, byte cache 6.4 -> 7.2: the kernel is twice its size and starts cold), so a call whose
+// bound already says that they will be takes that kernel.
+#ifndef FA_ROW_MERGE_MAX_ITEMS
+#define FA_ROW_MERGE_MAX_ITEMS 384
+#endif
+#ifndef FA_ROW_MERGE_WHOLE_PARTITIONS
+#define FA_ROW_MERGE_WHOLE_PARTITIONS 5
+#endif
+#ifndef FA_ROW_MERGE_PIECE_BYTES
+#define FA_ROW_MERGE_PIECE_BYTES (128 << 10)
+#endif
+constexpr int kRowMergeMaxItems = FA_ROW_MERGE_MAX_ITEMS;
+// Pieces are a whole number of partitions of this many bytes of K and V, two at least; rows of up to
+// kRowMergeWholePartitions of them stay whole.
+constexpr int kRowMergePartitionBytes = FA_ROW_MERGE_PIECE_BYTES;
+constexpr int kRowMergeWholePartitions = FA_ROW_MERGE_WHOLE_PARTITIONS;
+
+// Wavefronts per work-group; wide where the launch without cuts would be (FA_PLOOP_WIDE).
+template <bool kWide>
+constexpr int kMergeWaves = kWide ? 8 : 4;
+
+struct RowMergeSpace {
+  int64_t flags = 0;  // words
+  int64_t bytes = 0;  // 0: the call would not cut its rows
+};
+
+// The most keys of a row that some query token sees, as far as the host knows.
+inline int64_t visible_row_bound(const fa_paged_attention_shape &shape, const Resolved &r, int32_t max_context_len) {
+  int64_t bound = (int64_t)shape.max_blocks_per_seq * shape.block_size;
+  if (max_context_len > 0) bound = std::min<int64_t>(bound, max_context_len);
+  if (r.mask_flags & FA_MASK_WINDOW) bound = std::min<int64_t>(bound, (int64_t)r.window_left + r.query_len);
+  return bound;
+}
+
+inline int row_merge_partition(int row_bytes) { return kRowMergePartitionBytes / (2 * row_bytes); }
+
+inline RowMergeSpace row_merge_space(const fa_paged_attention_shape &shape, const Resolved &r, int32_t max_context_len) {
+  RowMergeSpace space;
+  const int64_t heads = r.pair_heads ? shape.num_kv_heads / 2 : shape.num_kv_heads;
+  const int group = r.pair_heads ? 2 * r.group : r.group, head_size = r.pair_heads ? 128 : shape.head_size;
+  const int64_t items = shape.num_seqs * heads;
+  if (r.schedule != FA_SCHEDULE_AUTO || !kUsePersistentLoop || shape.num_pool_blocks <= 0 ||
+      shape.num_seqs > kLoopPersistentMaxSeqs || (int64_t)shape.max_blocks_per_seq * shape.block_size >= kSegmentMaxContext)
+    return space;
+  if (r.query_len > kMaxGroup / group) return space;  // (two column tiles per wavefront)
+  if (items > kRowMergeMaxItems || visible_row_bound(shape, r, max_context_len) <=
+                                       kRowMergeWholePartitions * row_merge_partition(head_size * r.kv_elem_bytes))
+    return space;
+  // one slice per wavefront, of four wavefronts or of eight (see the launch)
+  const int slices = head_size == 128 ? kMergeWaves<true> : kMergeWaves<false>;
+  const int cols = group * r.query_len;
+  space.flags = (kMergeWholePieces + items) * slices;  // (an even number of 8-byte words: what follows is aligned to 16)
+  space.bytes = space.flags * 8;
+  int64_t floats = 0;  // of a piece
+  for (int n : {kMergeWaves<false>, slices}) floats = std::max(floats, (int64_t)n * merge_slice_floats(cols, head_size / 4 / n));
+  space.bytes += (kMergeWholePieces + items) * floats * 4;
+  return space;
+}
+
+// A number that no other launch of this process has, and hardly one of another: the clock, mixed.
+inline uint64_t next_merge_nonce() {
+  static std::atomic<uint64_t> counter{(uint64_t)std::chrono::high_resolution_clock::now().time_since_epoch().count()};
+  uint64_t nonce;
+  do {
+    uint64_t x = counter.fetch_add(0x9e3779b97f4a7c15ull, std::memory_order_relaxed);
+    x = (x ^ (x >> 30)) * 0xbf58476d1ce4e5b9ull;
+    x = (x ^ (x >> 27)) * 0x94d049bb133111ebull;
+    nonce = x ^ (x >> 31);
+  } while (nonce == 0);
+  return nonce;
+}
+
 // The launches of one batch that a single kernel launch can take: persistent form for up to
 // kLoopPersistentMaxSeqs sequences, else grid (kv heads, 1, sequences) with NW wavefronts per
 // work-group.  Kernel time is ADDED to *total_us when the call is timed.
@@ -64,12 +146,37 @@ inline fa_status launch_paged_attn_loop_rows(void *out, const void *query, const
                           max_ctx < kLoopPersistentMaxContext;
   // One launch per group of query tokens that fit the MFMA columns (one launch for decode): 16
   // columns, or in the persistent form two tiles of 16 held by every wavefront.
+  const RowMergeSpace merge = r.workspace ? row_merge_space(shape, r, r.max_context_len) : RowMergeSpace{};
   const int per_tile = p.query_count;
   const int per_launch = (persistent && r.query_len > per_tile) ? 2 * per_tile : per_tile;
   for (int q0 = 0; q0 < r.query_len; q0 += per_launch) {
     p.query_first = q0;
     p.query_count = std::min(per_launch, r.query_len - q0);
-    if (persistent && r.schedule == FA_SCHEDULE_VALU) {
+    if (persistent && merge.bytes > 0) {
+      // few rows: cut into pieces, merged within the launch
+      constexpr int SW = kMergeWaves<false>, SO = SegmentSplit<KV8>::occ, TPC = Pipeline<KV8>::tiles_per_chunk;
+      auto kernel = ext ? paged_attn_segment_kernel<HEAD_SIZE, QT, KVF, SW, SO, TPC, true, 1, true, KROW>
+                        : paged_attn_segment_kernel<HEAD_SIZE, QT, KVF, SW, SO, TPC, false, 1, true, KROW>;
+      int waves = SW, resident = 0, cus = 0;
+      FA_HIP_CHECK(compute_units_of_current_device(&cus));
+      if constexpr (HEAD_SIZE == 128) {
+        if (FA_PLOOP_WIDE && !ext && 2 * items <= cus) {
+          waves = kMergeWaves<true>;
+          kernel = paged_attn_segment_kernel<HEAD_SIZE, QT, KVF, kMergeWaves<true>, SO, TPC, false, 1, true, KROW>;
+        }
+      }
+      FA_HIP_CHECK(resident_groups(kernel, waves * 64, &resident));
+      p.compute_units = cus;
+      p.segment_force = 0;
+      p.partition_size = row_merge_partition(HEAD_SIZE * (KV8 ? 1 : 2));
+      p.merge_whole_partitions = kRowMergeWholePartitions;
+      p.max_num_partitions = INT32_MAX;
+      p.merge_flags = static_cast<uint64_t *>(r.workspace);
+      p.merge_pieces = reinterpret_cast<float *>(p.merge_flags + merge.flags);
+      p.merge_nonce = next_merge_nonce();
+      const int64_t most = items * ((max_ctx + p.partition_size - 1) / p.partition_size);
+      FA_HIP_CHECK(timer.launch(kernel, dim3((unsigned)std::min<int64_t>(resident, most)), dim3(waves * 64), 0, p));
+    } else if (persistent && r.schedule == FA_SCHEDULE_VALU) {
       if constexpr (HEAD_SIZE == 128 && std::is_same<QT, F16>::value) {
         constexpr int VW = FA_VALU_WAVES;
         auto kernel = paged_attn_valu_persistent_kernel<KVF, VW, Pipeline<KV8>::stream_loads_loop, (KV8 ? FA_VALU_OCC_FP8 : FA_VALU_OCC_16)>;
@@ -251,12 +358,23 @@ inline fa_status dispatch_paged_attention_loop_any(void *out, const void *query,
                                                    const int32_t *context_lens, float scale,
                                                    int32_t max_context_len,
                                                    const fa_paged_attention_shape *shape,
-                                                   const fa_paged_attention_options *options) {
+                                                   const fa_paged_attention_options *options,
+                                                   void *workspace, int64_t workspace_bytes) {
   Resolved r;
   fa_status st = validate_and_resolve(out, query, key_cache, value_cache, block_tables, context_lens,
                                       max_context_len, nullptr, nullptr, nullptr, shape, options,
                                       KV8, /*split=*/false, &r);
-  if (st != FA_OK || r.validate_only) return st;
+  if (st != FA_OK) return st;
+  if (workspace) {
+    if ((uintptr_t)workspace % 16) return fail(FA_ERR_BAD_SHAPE, "workspace must be 16-byte aligned");
+    const RowMergeSpace space = row_merge_space(*shape, r, 0);
+    if (workspace_bytes < space.bytes)
+      return fail(FA_ERR_SCRATCH_TOO_SMALL, "workspace of %lld bytes, this call asks for %lld", (long long)workspace_bytes,
+                  (long long)space.bytes);
+    r.workspace = workspace;
+    r.workspace_bytes = workspace_bytes;
+  }
+  if (r.validate_only) return st;
   const bool bf16 = shape->q_dtype == FA_DTYPE_BF16;
 #define FA_LOOP_CASE(HS, QT)                                                                      \
   do {                                                                                            \
@@ -287,10 +405,11 @@ inline fa_status dispatch_paged_attention_loop(void *out, const void *query, con
                                                const int32_t *context_lens, float scale,
                                                int32_t max_context_len,
                                                const fa_paged_attention_shape *shape,
-                                               const fa_paged_attention_options *options) {
+                                               const fa_paged_attention_options *options, void *workspace,
+                                               int64_t workspace_bytes) {
   return dispatch_paged_attention_loop_any<false>(out, query, key_cache, value_cache, block_tables,
                                                   context_lens, scale, max_context_len, shape,
-                                                  options);
+                                                  options, workspace, workspace_bytes);
 }
 
 }  // namespace fa

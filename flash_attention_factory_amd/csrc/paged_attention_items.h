@@ -24,6 +24,12 @@ namespace fa {
 // ctx: the sequence's length
 struct WorkItem { int seq, kvh, ctx, c_lo, c_end, tok_end, part0, parts; };
 
+// An item of a launch that merges the pieces of a row itself: pieces of the item's row, `whole` of them of full
+// length; numbers, among all pieces of the launch, of this piece, of the row's first whole piece (the next ones
+// follow piece_step apart) and of the shorter piece that ends the row.  (Not part of WorkItem: the other kernels'
+// copies of the fields ended up in LDS and cost the segment kernel 7 us a launch.)
+struct MergeItem : WorkItem { int pieces, whole, piece, first_piece, piece_step, last_piece; };
+
 __device__ __forceinline__ int snake_position(int nth, int groups, int group) {
   return nth * groups + ((nth & 1) ? groups - 1 - group : group);
 }
@@ -113,9 +119,19 @@ struct LoopItems {
   }
 };
 
+// ROW_MERGE: for a launch that merges the pieces of a row itself (paged_attention_row_merge.h).  A row then begins
+// at the partition of its first key inside the local window, the length of a piece grows until there are no more
+// than kMergeWholePieces whole ones, part0 is the piece's number within the row, and pieces are numbered.
+template <bool ROW_MERGE = false>
 struct SegmentItems {
-  static constexpr int NQ = kSegmentMaxSeqs / 64;
+  static constexpr int NQ = (ROW_MERGE ? kMergeMaxSeqs : kSegmentMaxSeqs) / 64;
+  static constexpr int kIdTiles = ROW_MERGE ? 2 : 0;
   int ctxv[NQ], parts[NQ], incl[NQ], fullc[NQ], key[NQ];
+  // ROW_MERGE: first key of the row that is read; block ids of chunk `first_chunk` of every sequence, requested
+  // with the lengths, so that a work-group whose first item begins a row waits for one trip to memory, not two;
+  // whether rows are cut, and if not, whether every row has a work-group of its own
+  int base[ROW_MERGE ? NQ : 1], sid[ROW_MERGE ? NQ : 1][ROW_MERGE ? kIdTiles : 1];
+  bool one_row_each = false, have_first_ids = false;
   int S, Hk, m, seg_tokens, full_total, total_items, lane, key_top_bit, psize;
   int head_shift = -1;  // stack_affine_shift of the pool
   // even shares (m == 0): tape[j] = cost of all rows up to and including the lane's sequence's (row_cost);
@@ -129,25 +145,102 @@ struct SegmentItems {
   // heads_per_item: adjacent kv heads that one work-group takes together (its wavefronts in teams);
   // item_row_bytes: bytes of one token's K row (as of its V row) of an item
   __device__ __forceinline__ void build(const PagedAttnParams &p, int lane_, int groups, int heads_per_item,
-                                        int item_row_bytes) {
+                                        int item_row_bytes, [[maybe_unused]] int first_chunk = 0,
+                                        [[maybe_unused]] int chunk_tokens = 32) {
     lane = lane_;
     S = p.num_seqs;
     Hk = p.num_kv_heads / heads_per_item;
     head_shift = stack_affine_shift(p.kv_head_bytes * heads_per_item, Hk);
     const int max_ctx = p.max_blocks_per_seq << p.block_shift;
     psize = p.partition_size;
-    const int total_parts = count_partitions<NQ>(p.context_lens, S, max_ctx, p.partition_size, p.max_num_partitions, lane, ctxv, parts);
-    // (cost of the batch in steps of kShareTokens, from above: every partition full, every row a piece)
-    const long long steps_at_most = ((long long)total_parts * (psize >> kShareTokensLog2) + (long long)S * kSharePieceCost) * Hk;
-    even = p.segment_force == -1 && steps_at_most < (1 << 24);  // (a batch beyond that is cut into segments)
-    if (even) {
-      build_even_shares(groups, p.compute_units);
-      return;
+    if constexpr (ROW_MERGE) {
+      // (only the work-groups that have an item if rows stay whole: thousands of wavefronts asking for the same
+      // lines hold up the few that wait for them)
+      have_first_ids = (int)blockIdx.x < S * Hk;
+#pragma unroll
+      for (int j = 0; j < NQ; ++j)
+        if (have_first_ids && j * 64 < S) {  // (lanes past the batch ask for the last sequence's)
+          const int32_t *row = p.block_tables + (int64_t)min(lane + 64 * j, S - 1) * p.max_blocks_per_seq;
+#pragma unroll
+          for (int t = 0; t < kIdTiles; ++t)
+            sid[j][t] = row[min((first_chunk * chunk_tokens + t * kTileTokens) >> p.block_shift, p.max_blocks_per_seq - 1)];
+        }
     }
-    m = p.segment_force > 0 ? min(p.segment_force, kSegmentMaxPartitions)
-                            : partitions_per_segment<NQ>(ctxv, parts, total_parts, S, p.partition_size, Hk, groups,
-                                                         p.compute_units, p.kv_rows_apart != 0,
-                                                         2 * p.partition_size * item_row_bytes);
+    if constexpr (ROW_MERGE) {
+      // No row long enough to be cut and a work-group for each: known from the lengths alone, and as little code as
+      // can be until the first loads go out (a launch of short rows lasts 6 us, and its code comes from memory too).
+      int len[NQ];
+      bool any_long = false;
+#pragma unroll
+      for (int j = 0; j < NQ; ++j) len[j] = p.context_lens[min(lane + 64 * j, S - 1)];
+#pragma unroll
+      for (int j = 0; j < NQ; ++j) {
+        ctxv[j] = max(0, min(len[j], max_ctx));
+        base[j] = 0;
+        any_long |= ctxv[j] > p.merge_whole_partitions * psize;
+      }
+      one_row_each = !__any(any_long) && S * Hk <= groups;
+      if (one_row_each) return;
+    }
+    int total_parts = count_partitions<NQ>(p.context_lens, S, max_ctx, p.partition_size, p.max_num_partitions, lane, ctxv, parts);
+    if constexpr (ROW_MERGE) {
+      const bool window = p.mask_flags & kMaskWindow;
+#pragma unroll
+      for (int j = 0; j < NQ; ++j) base[j] = 0;
+      if (window) {  // (wave-uniform) rows from the partition of the earliest key that some query token sees
+        int local = 0;
+        const float inv = __builtin_amdgcn_rcpf((float)psize);
+#pragma unroll
+        for (int j = 0; j < NQ; ++j) {
+          int rem;
+          const int skip = quotient_below_2p24(max(0, ctxv[j] - p.query_len + p.query_first - p.window_left), psize, inv, rem);
+          base[j] = skip * psize;
+          ctxv[j] -= base[j];
+          parts[j] -= skip;
+          local += parts[j];
+        }
+        total_parts = wave_total(local);
+      }
+    }
+    if constexpr (!ROW_MERGE) {
+      // (cost of the batch in steps of kShareTokens, from above: every partition full, every row a piece)
+      const long long steps_at_most = ((long long)total_parts * (psize >> kShareTokensLog2) + (long long)S * kSharePieceCost) * Hk;
+      even = p.segment_force == -1 && steps_at_most < (1 << 24);  // (a batch beyond that is cut into segments)
+      if (even) {
+        build_even_shares(groups, p.compute_units);
+        return;
+      }
+    }
+    bool cut = true;
+    int longest = 0, live = 0;  // (ROW_MERGE) partitions of the longest row, rows per kv head
+    if constexpr (ROW_MERGE) {
+#pragma unroll
+      for (int j = 0; j < NQ; ++j) {
+        longest = max(longest, parts[j]);
+        if (j * 64 < S) live += __builtin_popcountll(__ballot(parts[j] > 0));
+      }
+      longest = __builtin_amdgcn_readfirstlane(__reduce_max_sync(~0ull, longest));
+      cut = cut_pays(longest, total_parts, live, Hk, p.compute_units, p.merge_whole_partitions);
+    }
+    if constexpr (ROW_MERGE) {
+      one_row_each = !cut && S * Hk <= groups;
+      if (one_row_each) return;  // nobody takes a second item, so the order of the rows is of no matter
+    }
+    if (!cut) m = max(longest, 1);
+    else
+      m = p.segment_force > 0 ? min(p.segment_force, kSegmentMaxPartitions)
+                              : partitions_per_segment<NQ>(ctxv, parts, total_parts, S, p.partition_size, Hk, groups,
+                                                           p.compute_units, p.kv_rows_apart != 0,
+                                                           2 * p.partition_size * item_row_bytes);
+    if constexpr (ROW_MERGE) {
+      m = max(m, 2);  // (a piece costs its merge whatever its length)
+      while (true) {  // ends: one whole piece per row at most once m spans the longest
+        int whole, all;
+        count_segments<NQ>(ctxv, parts, S, p.partition_size, m, whole, all);
+        if ((int64_t)whole * Hk <= kMergeWholePieces || (int64_t)m * psize >= max_ctx) break;
+        m *= 2;
+      }
+    }
     seg_tokens = m * p.partition_size;
     int running = 0, tails = 0;
 #pragma unroll
@@ -282,11 +375,46 @@ struct SegmentItems {
     }
     return 255 - (found & 255);
   }
+  // ROW_MERGE, uncut rows, at least as many work-groups as rows: row number `group`.
+  __device__ __forceinline__ bool row_of_group(int n, int group, int chunk_tokens, MergeItem &it) const {
+    if (n > 0 || group >= S * Hk) return false;
+    const int s = __builtin_amdgcn_readfirstlane(group / Hk);
+    int ctx_s = 0, base_s = 0;
+#pragma unroll
+    for (int j = 0; j < NQ; ++j)
+      if ((s >> 6) == j) {
+        ctx_s = __builtin_amdgcn_readlane(ctxv[j], s & 63);
+        base_s = __builtin_amdgcn_readlane(base[ROW_MERGE ? j : 0], s & 63);
+      }
+    it.seq = s;
+    it.kvh = stack_affine_head(group - s * Hk, head_shift);
+    it.ctx = it.tok_end = base_s + ctx_s;
+    it.c_lo = base_s / chunk_tokens;
+    it.c_end = (it.ctx + chunk_tokens - 1) / chunk_tokens;
+    it.part0 = 0;
+    it.parts = it.pieces = it.whole = 1;
+    it.piece = it.first_piece = it.last_piece = it.piece_step = 0;
+    return it.ctx > 0;
+  }
+  // ROW_MERGE: block id of tile t of chunk `first_chunk` of a sequence.
+  __device__ __forceinline__ int first_id(int t, int seq) const {
+    int id = 0;
+#pragma unroll
+    for (int j = 0; j < NQ; ++j)
+      if ((seq >> 6) == j) id = __builtin_amdgcn_readlane(sid[ROW_MERGE ? j : 0][ROW_MERGE ? t : 0], seq & 63);
+    return id;
+  }
   // n-th item of work-group `group`, asked for n = 0, 1, 2, ... in turn.  Segments: position in the
   // sorted list -> (sequence, segment, kv head), kv head fastest.
-  __device__ __forceinline__ bool at(int n, int groups, int group, int chunk_tokens, WorkItem &it) {
-    if (even) return next_of_share(chunk_tokens, it);
+  __device__ __forceinline__ bool at(int n, int groups, int group, int chunk_tokens,
+                                     std::conditional_t<ROW_MERGE, MergeItem, WorkItem> &it) {
+    if constexpr (!ROW_MERGE) {
+      if (even) return next_of_share(chunk_tokens, it);
+    }
     const int pos = snake_position(n, groups, group);
+    if constexpr (ROW_MERGE) {
+      if (one_row_each) return row_of_group(n, group, chunk_tokens, it);
+    }
     if (pos >= total_items) return false;
     const int q = __builtin_amdgcn_readfirstlane(pos / Hk);
     it.kvh = stack_affine_head(pos - q * Hk, head_shift);
@@ -300,15 +428,33 @@ struct SegmentItems {
       s = sequence_of_tail(q - full_total);
     }
     s = min(s, S - 1);
-    int inc_s = 0, full_s = 0, ctx_s = 0;
+    int inc_s = 0, full_s = 0, ctx_s = 0, base_s = 0;
 #pragma unroll
     for (int j = 0; j < NQ; ++j)
       if ((s >> 6) == j) {
         inc_s = __builtin_amdgcn_readlane(incl[j], s & 63);
         full_s = __builtin_amdgcn_readlane(fullc[j], s & 63);
         ctx_s = __builtin_amdgcn_readlane(ctxv[j], s & 63);
+        if constexpr (ROW_MERGE) base_s = __builtin_amdgcn_readlane(base[j], s & 63);
       }
     it.seq = __builtin_amdgcn_readfirstlane(s);
+    if constexpr (ROW_MERGE) {
+      const int seg = full ? q - (inc_s - full_s) : full_s;
+      const int tok_begin = base_s + seg * seg_tokens;
+      it.ctx = base_s + ctx_s;
+      it.tok_end = full ? tok_begin + seg_tokens : it.ctx;
+      it.c_lo = tok_begin / chunk_tokens;
+      it.c_end = (it.tok_end + chunk_tokens - 1) / chunk_tokens;
+      it.part0 = seg;
+      it.parts = 1;
+      it.whole = full_s;
+      it.pieces = full_s + (ctx_s > full_s * seg_tokens);
+      it.first_piece = (inc_s - full_s) * Hk + it.kvh;
+      it.piece_step = Hk;
+      it.last_piece = (full_total + s) * Hk + it.kvh;
+      it.piece = full ? it.first_piece + seg * Hk : it.last_piece;
+      return true;
+    }
     const int seg = full ? q - (inc_s - full_s) : full_s;
     it.part0 = seg * m;
     const int tok_begin = seg * seg_tokens;

@@ -36,6 +36,7 @@
 #include "paged_attention_items.h"
 #include "paged_attention_kernel.h"
 #include "paged_attention_loop_persistent_kernel.h"
+#include "paged_attention_row_merge.h"
 #include "paged_attention_segment_policy.h"
 
 // Builds that time what the stores of the partials cost (profiles/): 1 leaves out the rows of tmp_out,
@@ -46,13 +47,16 @@
 
 namespace fa {
 
-//
-template <int D, typename QT, int KVF, int NWG, int OCC, int TPC, bool EXT = false, int HPW = 1>
+// ROW_MERGE: the loop path's form of the kernel.  There is no reduce launch and no tmp_out: the pieces of a row are
+// merged by the wavefronts that finish it (paged_attention_row_merge.h) and p.out is the call's `out`.
+// KROW: how K tiles are loaded, as in the loop kernels.
+template <int D, typename QT, int KVF, int NWG, int OCC, int TPC, bool EXT = false, int HPW = 1, bool ROW_MERGE = false,
+          bool KROW = true>
 __global__ void __launch_bounds__(NWG * 64) __attribute__((amdgpu_waves_per_eu(OCC)))
 paged_attn_segment_kernel(const PagedAttnParams p) {
   constexpr int NW = NWG;       // wavefronts of the work-group
   constexpr int NT = NW / HPW;  // of which a team of NT shares a segment's chunks of one kv head and merges
-  using W = WaveAttn<D, QT, KVF, TPC, SegmentSplit<(KVF != 0)>::stream_loads, EXT>;
+  using W = WaveAttn<D, QT, KVF, TPC, SegmentSplit<(KVF != 0)>::stream_loads, EXT, KROW>;
   using Chunk = typename W::Chunk;
   using Ids = typename W::Ids;
   using ItemExt = typename W::ItemExt;
@@ -63,6 +67,7 @@ paged_attn_segment_kernel(const PagedAttnParams p) {
   constexpr int SL = NR / NT;
   static_assert(NT >= 1 && NW % HPW == 0 && NR % NT == 0 && SL >= 4 && SL % 4 == 0,
                 "each wavefront stores whole 16-byte pieces");
+  static_assert(!ROW_MERGE || (HPW == 1 && NT > 1), "rows are merged slice by slice, one kv head per work-group");
   // NT == 1: every wavefront has a kv head of its own and the whole of each item's chunks, so an item's
   // state never leaves its registers: no LDS, no waiting for the others.
 
@@ -80,9 +85,9 @@ paged_attn_segment_kernel(const PagedAttnParams p) {
   // The segment list (SegmentItems): all full segments, then the sequences' last, shorter segments
   // in order of length, dealt to the work-groups in snake order, so that the work-groups' totals
   // come out even although a work-group only gets a handful of segments.
-  using Item = WorkItem;  // c_lo .. c_end: the segment's chunks; ctx: the sequence's length (EXT)
-  SegmentItems items;
-  items.build(p, lane, G, HPW, W::ROWB * HPW);
+  using Item = std::conditional_t<ROW_MERGE, MergeItem, WorkItem>;  // c_lo .. c_end: the segment's chunks; ctx: the sequence's length (EXT)
+  SegmentItems<ROW_MERGE> items;
+  items.build(p, lane, G, HPW, W::ROWB * HPW, tw, CT);
   // n-th item of this work-group; with HPW > 1 an item is HPW adjacent kv heads of one segment, of
   // which this wavefront's team takes one (kvh is then the team's own head)
   auto item_at = [&](int nth, Item &it) {
@@ -127,7 +132,28 @@ paged_attn_segment_kernel(const PagedAttnParams p) {
   };
   // Store this wavefront's slice o[SL] of an item's merged, un-normalised output (maximum M in base-2
   // units, sum L) as the item's partial -- or, where the item is its row's only piece, as the row's result.
-  auto store_slice = [&](const Item &it, float M, float L, const float (&o)[SL], float out_mul) {
+  auto store_slice = [&](const Item &it, float M, float L, float (&o)[SL], float out_mul) {
+    if constexpr (ROW_MERGE) {
+      if (it.pieces > 1) {  // wave-uniform
+        const int cols = EXT ? p.query_count * p.group : p.group;
+        if (wa.col_valid) {
+          const MergeSlot slot = merge_slot(p, it.piece, tw, NT, cols, SL);
+#pragma unroll
+          for (int e = 0; e < SL; e += 2) share_pair(slot.pair(e >> 2, (e >> 1) & 1, r, i), o[e], o[e + 1]);
+          if (r == 0) share_pair(slot.scalars(i), M, L);
+        }
+        if (!merge_arrive(p, it, tw, NT, lane)) return;
+        merge_pieces<SL>(p, it, tw, NT, cols, r, i, M, L, o);
+      }
+      if (wa.col_valid && wa.keeps_output()) {
+        const int64_t row = EXT ? (int64_t)it.seq * p.query_len + wa.col_q : it.seq;
+        const int head = it.kvh * p.group + wa.col_g;
+        const float inv = !EXT ? p.out_scale / L : L > 0.f ? out_mul / L : 0.f;  // L = 0: the query token sees no key
+        W::template store_q<SL>(reinterpret_cast<char *>(p.out) + ((row * p.num_heads + head) * wa.out_row_elems() +
+                                                                   wa.out_elem(4 * r * NDT + tw * SL)) * 2, o, inv);
+      }
+      return;
+    }
     if (wa.col_valid && wa.keeps_output()) {
       const int head = it.kvh * p.group + wa.col_g;
       int64_t row = it.seq;
@@ -224,7 +250,17 @@ paged_attn_segment_kernel(const PagedAttnParams p) {
   TileScales ts = {}, nts = {}, nxt_ts = {};
   if constexpr (EXT) cur_ext = wa.fetch_item_ext(cur.kvh, p.block_tables + (int64_t)cur.seq * p.max_blocks_per_seq);
   if (armed) {
-    const Ids ids = wa.fetch_ids(p.block_tables + (int64_t)cur.seq * p.max_blocks_per_seq, cur.c_lo + tw, col_max);
+    Ids ids;
+    bool have_ids = false;
+    if constexpr (ROW_MERGE) {
+      static_assert(TPC == decltype(items)::kIdTiles, "the ids requested with the lengths are those of one chunk");
+      have_ids = items.have_first_ids && cur.c_lo == 0;
+      if (have_ids) {
+#pragma unroll
+        for (int t = 0; t < TPC; ++t) ids.v[t] = min((uint32_t)items.first_id(t, cur.seq), (uint32_t)p.max_block_id);
+      }
+    }
+    if (!have_ids) ids = wa.fetch_ids(p.block_tables + (int64_t)cur.seq * p.max_blocks_per_seq, cur.c_lo + tw, col_max);
     wa.load_q(cur.seq, cur.kvh);
     wa.issue_k(R, cur.kvh, cur.c_lo + tw, ids);
     wa.issue_v(R, cur.kvh, cur.c_lo + tw, ids);

@@ -30,6 +30,7 @@ struct Entries {
   decltype(&fa_paged_attention_loop) loop, fp8_loop;
   decltype(&fa_paged_attention_reduce) reduce, fp8_reduce;
   decltype(&fa_kv_cache_write) kv_cache_write;
+  decltype(&fa_paged_attention_loop_workspace_bytes) workspace_bytes;
 };
 Entries entries = {};
 
@@ -98,7 +99,8 @@ bool attend(const Tensor &out, const Scratch *scratch, const Tensor &query, cons
   sh.num_pool_blocks = (int32_t)blocks;
   sh.q_dtype = q_type == at::kBFloat16 ? FA_DTYPE_BF16 : FA_DTYPE_F16;
 
-  fa_paged_attention_options op = FA_PAGED_ATTENTION_OPTIONS_INIT;
+  fa_paged_attention_options_workspace full = FA_PAGED_ATTENTION_OPTIONS_WORKSPACE_INIT;
+  fa_paged_attention_options &op = full.options;
   op.sinks = sinks.has_value() ? sinks->const_data_ptr() : nullptr;
   op.softcap = (float)softcap;
   op.fp8_scale = (float)fp8_scale;
@@ -144,6 +146,12 @@ bool attend(const Tensor &out, const Scratch *scratch, const Tensor &query, cons
                o, q, k, v, tables, lens, (float)scale, (int32_t)max_context_len, static_cast<float *>(scratch->exp_sums.data_ptr()),
                static_cast<float *>(scratch->max_logits.data_ptr()), static_cast<float *>(scratch->tmp_out.data_ptr()), &sh,
                &op) == FA_OK;
+  Tensor space;
+  if (const int64_t need = entries.workspace_bytes(&sh, &op, fp8); need > 0) {  // see fa_paged_attention_options_workspace
+    space = at::empty({need}, query.options().dtype(at::kByte));
+    full.workspace = space.data_ptr();
+    full.workspace_bytes = need;
+  }
   return (fp8 ? entries.fp8_loop : entries.loop)(o, q, k, v, tables, lens, (float)scale, 0, &sh, &op) == FA_OK;
 }
 

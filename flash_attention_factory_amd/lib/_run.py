@@ -12,6 +12,7 @@ from __future__ import annotations
 
 import ctypes
 import warnings
+from contextlib import nullcontext
 from typing import List, Optional
 
 import torch
@@ -121,7 +122,7 @@ def run_impl(entry: str, split: bool, fp8: bool, max_logits, exp_sums, tem_outpu
         raise _cabi.PagedAttentionError(_cabi.FA_ERR_UNSUPPORTED_HEAD_OR_BLOCK_SIZE,
                                         "Unsupported head size or block size")
     elapsed = (ctypes.c_float * 2)(0.0, 0.0)
-    op = _cabi.Options()
+    op = _cabi.Options() if split else _cabi.OptionsWorkspace()
     op.sinks = sinks.data_ptr() if sinks is not None else None
     op.alibi_slopes = alibi_slopes.data_ptr() if alibi_slopes is not None else None
     op.softcap = softcap
@@ -164,7 +165,15 @@ def run_impl(entry: str, split: bool, fp8: bool, max_logits, exp_sums, tem_outpu
             raise _cabi.PagedAttentionError(_cabi.FA_ERR_UNSUPPORTED_DTYPE,
                                             "max_logits/exp_sums must be contiguous fp32")
         args += [exp_sums.data_ptr(), max_logits.data_ptr(), tmp.data_ptr()]
-    with torch.cuda.device(query.device):
+    if not split:
+        # few rows: memory in which they can be shared among more work-groups (from PyTorch's stream-ordered
+        # allocator, so that calls that overlap on other streams, and graphs, have memory of their own)
+        need = L.fa_paged_attention_loop_workspace_bytes(ctypes.byref(sh), ctypes.byref(op), int(fp8))
+        if need > 0:
+            space = torch.empty(need, dtype=torch.uint8, device=query.device)
+            op.workspace, op.workspace_bytes = space.data_ptr(), need
+    # (entering torch.cuda.device costs 2 us also where the device is the current one)
+    with nullcontext() if query.device.index == torch.cuda.current_device() else torch.cuda.device(query.device):
         _cabi.check(fn(*args, ctypes.byref(sh), ctypes.byref(op)))
     if not timed:
         return []

@@ -34,8 +34,9 @@ block_size``: if the scratch arrays hold fewer tokens than that, a RuntimeWarnin
 explicit 0 checks nothing and warns of nothing.
 
 Caches are ``[blocks, block_size, kv_heads, head_size]`` views as in ``lib.*.run``; every
-output is an argument the operator mutates, nothing is allocated.  Importing this module
-registers the operators; there is no CPU implementation.
+output is an argument the operator mutates.  Nothing is allocated, but for a few MB of workspace from PyTorch's
+stream-ordered allocator where a loop operator shares the rows of a small batch among more work-groups.
+Importing this module registers the operators; there is no CPU implementation.
 
 The operators of ``torch.ops.fa_amd`` are native (csrc/torch_ops.cpp, ``libfa_torch_ops.so``).  The functions below
 are the same operators in Python, in the namespace ``fa_amd_py``: they say what a valid call is, and every call
@@ -157,7 +158,7 @@ def _load_native() -> None:
     torch.ops.load_library(_build.TORCH_OPS_LIBRARY)
     L = _cabi.load()
     entries = (L.fa_paged_attention_loop, L.fa_paged_attention_fp8_loop, L.fa_paged_attention_reduce,
-               L.fa_paged_attention_fp8_reduce, L.fa_kv_cache_write)
+               L.fa_paged_attention_fp8_reduce, L.fa_kv_cache_write, L.fa_paged_attention_loop_workspace_bytes)
     table = (ctypes.c_void_p * len(entries))(*(ctypes.cast(e, ctypes.c_void_p).value for e in entries))
     bind = ctypes.CDLL(_build.TORCH_OPS_LIBRARY).fa_torch_ops_bind
     bind.argtypes, bind.restype = [ctypes.c_void_p, ctypes.c_size_t], None

@@ -212,6 +212,26 @@ int32_t fa_paged_attention_loop(void *out, const void *query, const void *key_ca
                                 const fa_paged_attention_shape *shape,
                                 const fa_paged_attention_options *options);
 
+/* The single-pass entries with memory to work in.  A batch of few (sequence, kv head) rows leaves most of the
+ * GPU idle if every row is one work-group's, and a batch of unequal ones waits for the longest: given a
+ * workspace, such a call cuts long rows into pieces that several work-groups take, merged within the same
+ * launch.  `out` is the same up to the order of fp32 sums.
+ * fa_paged_attention_loop_workspace_bytes: what a call asks for, from its shape and options (the fields that say
+ * what is computed; pointers are not followed, no GPU is needed); 0 if it would not use any, or is not a valid
+ * call.  kv_fp8: byte caches (fa_paged_attention_fp8_loop).
+ * The workspace goes with the options: a caller passes &x.options of the struct below, whose
+ * options.struct_size is the size of the whole.  workspace: device memory, 16-byte aligned, contents of no matter
+ * before and after; calls that may overlap on the GPU (other streams) need one each.  NULL: none.  Less than the
+ * call asks for: FA_ERR_SCRATCH_TOO_SMALL.  Entries other than the two single-pass ones do not look at it. */
+typedef struct fa_paged_attention_options_workspace {
+  fa_paged_attention_options options;
+  void *workspace;
+  int64_t workspace_bytes;
+} fa_paged_attention_options_workspace;
+#define FA_PAGED_ATTENTION_OPTIONS_WORKSPACE_INIT {{(uint32_t)sizeof(fa_paged_attention_options_workspace)}}
+int64_t fa_paged_attention_loop_workspace_bytes(const fa_paged_attention_shape *shape,
+                                                const fa_paged_attention_options *options, int32_t kv_fp8);
+
 /* Split-context kernel followed by the reduce kernel.  exp_sums, max_logits and tmp_out are
  * scratch the two kernels hand partial softmax states through; every slot either holds what
  * upstream stores there for its partition -- or nothing: for batches with many

@@ -1,0 +1,172 @@
+"""Loop path with workspace: rows cut into pieces that several work-groups take, merged inside the launch
+(csrc/paged_attention_row_merge.h), against the CPU oracle at the sizes where it can go wrong: rows around the
+length from which they are cut, more pieces than a wavefront has lanes, every number of MFMA columns, empty rows,
+windows, sinks, several query tokens; workspace of any contents; replays of a HIP graph; two streams at once.
+
+Tolerance: results are rounded to fp16 / bf16 (2^-11, 2^-8 of the value) from probabilities rounded to the same
+type before P.V; 1e-2 of the largest value, as in the repository's other comparisons with the oracle."""
+import ctypes
+
+import pytest
+import torch
+
+from flash_attention_factory_amd import _cabi, runner, workloads as W
+from flash_attention_factory_amd.lib import paged_attention_fp8_loop, paged_attention_loop
+
+pytestmark = pytest.mark.gpu
+
+
+def _workload(lens, hk, group, d, fp8=None, block=16, bf16=False, sinks=False, seed=0):
+    w = W.make_test_shaped(batch_size=len(lens), nheads=hk * group, nheads_k=hk, d=d, seqlen_k=max(lens), varlen=False,
+                           has_sinks=sinks, fp8=fp8 is not None, block_size=block, seed=seed,
+                           dtype=torch.bfloat16 if bf16 else torch.float16, layout=W.HEAD_MAJOR if bf16 else W.TOKEN_MAJOR,
+                           **({"fp8_dtype": fp8} if fp8 is not None else {}))
+    w.context_lens.copy_(torch.tensor(lens, dtype=torch.int32))
+    return w
+
+
+def _run(w, dev, query=None, out=None, **kw):
+    wd = w.to(dev)
+    q = wd.query if query is None else query.to(dev)
+    out = torch.full_like(q, 7.0) if out is None else out
+    head = (None, None, None, out, None, q, runner.logical_cache_view(wd, wd.key_cache),
+            runner.logical_cache_view(wd, wd.value_cache), wd.block_tables, wd.context_lens,
+            w.num_heads // w.num_kv_heads, w.scale)
+    tail = (w.block_size, 0, kw.pop("alibi", None), wd.sinks, kw.pop("softcap", 0.0))
+    if w.is_fp8:
+        paged_attention_fp8_loop.run(*head, w.fp8_scale, *tail, timed=False, **kw)
+    else:
+        paged_attention_loop.run(*head, *tail, timed=False, **kw)
+    return out
+
+
+def _needs(w, query_len=1):
+    """Bytes the call asks for: > 0 says that it takes the path under test."""
+    sh, op = _cabi.Shape(), _cabi.Options()
+    sh.num_seqs, sh.num_heads, sh.head_size = w.query.shape[0], w.num_heads, w.query.shape[-1]
+    sh.num_kv_heads, sh.block_size, sh.max_blocks_per_seq = w.num_kv_heads, w.block_size, w.block_tables.shape[1]
+    sh.max_num_partitions, sh.num_pool_blocks = 1, w.key_cache.shape[0]
+    sh.kv_block_stride, sh.kv_token_stride, sh.kv_head_stride = w.kv_strides()
+    sh.q_dtype = _cabi.FA_DTYPE_BF16 if w.query.dtype == torch.bfloat16 else _cabi.FA_DTYPE_F16
+    op.query_len = query_len
+    return _cabi.load().fa_paged_attention_loop_workspace_bytes(ctypes.byref(sh), ctypes.byref(op), int(w.is_fp8))
+
+
+def _check(oracle, w, out, **kw):
+    query = kw.pop("query", w.query)
+    ref = oracle.attention_ref(query, w.key_cache, w.value_cache, w.block_tables, w.context_lens, scale=w.scale,
+                               block_size=w.block_size, kv_strides=w.kv_strides(), num_kv_heads=w.num_kv_heads, sinks=w.sinks,
+                               fp8_scale=w.fp8_scale, want_f32=True, **kw)[1]
+    live = w.context_lens > 0
+    unit = ref[live].abs().max()
+    torch.testing.assert_close(out.float().cpu()[live] / unit, ref[live] / unit, atol=1e-2, rtol=1e-2)
+    assert (out.cpu()[~live] == 7.0).all(), "rows without keys are not written"
+
+
+E5M2, E4M3 = torch.float8_e5m2, torch.float8_e4m3fn
+
+
+@pytest.mark.parametrize("lens, hk, group, d, fp8, block, bf16", [
+    # 5 partitions of 256 keys stay whole; one key more, and rows beside it that do
+    ([1281, 1280, 1, 0, 257], 2, 4, 128, None, 16, False),
+    ([1536, 1537, 511, 512, 513], 1, 1, 128, None, 64, True),
+    # more pieces than lanes; an empty row between
+    ([50001, 0, 700], 1, 2, 128, None, 16, True),
+    # 16-bit rows of 128 bytes, byte rows of 128 and of 64 bytes (partitions of 512, 512, 1024 keys)
+    ([5000, 2561, 2560], 4, 3, 64, None, 32, False),
+    ([5121, 2559, 9000], 2, 5, 128, E5M2, 16, False),
+    ([2700, 6001], 2, 16, 128, E4M3, 16, True),
+    # kv heads in pairs (byte rows of 64 bytes that lie next to each other)
+    ([9001, 5121, 40], 2, 4, 64, E5M2, 64, False),
+    ([7000, 100], 3, 7, 64, E4M3, 32, True),
+    # many short rows and one long
+    ([300] * 7 + [12000], 2, 8, 128, None, 16, False),
+])
+@pytest.mark.parametrize("sinks", [False, True])
+def test_against_the_oracle(oracle, lens, hk, group, d, fp8, block, bf16, sinks):
+    w = _workload(lens, hk, group, d, fp8, block, bf16, sinks)
+    assert _needs(w) > 0
+    dev = torch.device("cuda:0")
+    out = _run(w, dev)
+    again = _run(w, dev)
+    torch.cuda.synchronize()
+    assert torch.equal(out, again), "the order of arrival shows in the result"
+    _check(oracle, w, out)
+
+
+@pytest.mark.parametrize("window", [0, 1300, 2048, 100000])
+@pytest.mark.parametrize("query_len, group", [(1, 4), (3, 4), (2, 8)])
+def test_windows_modifiers_and_query_tokens(oracle, window, query_len, group):
+    w = _workload([4100, 1500, 2817, 5], 2, group, 128, sinks=True)
+    dev = torch.device("cuda:0")
+    H = 2 * group
+    g = torch.Generator().manual_seed(3)
+    query = torch.randn((4, query_len, H, 128), generator=g).to(torch.float16) if query_len > 1 else w.query
+    alibi = torch.linspace(0.001, 0.01, H)
+    assert _needs(w, query_len) > 0
+    out = _run(w, dev, query=query, alibi=alibi.to(dev), softcap=20.0, apply_alibi=True, apply_softcap=True, window_left=window)
+    torch.cuda.synchronize()
+    _check(oracle, w, out, query=query, alibi_slopes=alibi, softcap=20.0, window_left=window)
+
+
+@pytest.mark.parametrize("fill", [0x00, 0xFF, 0x7F])
+def test_contents_of_the_workspace_do_not_matter(oracle, fill):
+    """Through the C ABI, twice on the same memory, without clearing it in between."""
+    w = _workload([6000, 1400, 3000], 2, 4, 128)
+    dev = torch.device("cuda:0")
+    need = _needs(w)
+    space = torch.full((need,), fill, dtype=torch.uint8, device=dev)
+    wd = w.to(dev)
+    L, sh, op = _cabi.load(), _cabi.Shape(), _cabi.OptionsWorkspace()
+    op.workspace, op.workspace_bytes = space.data_ptr(), need
+    sh.num_seqs, sh.num_heads, sh.head_size, sh.num_kv_heads = 3, 8, 128, 2
+    sh.block_size, sh.max_blocks_per_seq, sh.max_num_partitions = w.block_size, w.block_tables.shape[1], 1
+    sh.kv_block_stride, sh.kv_token_stride, sh.kv_head_stride = w.kv_strides()
+    sh.num_pool_blocks, sh.q_dtype = w.key_cache.shape[0], _cabi.FA_DTYPE_F16
+    op.stream = torch.cuda.current_stream().cuda_stream
+    outs = []
+    for _ in range(2):
+        out = torch.full_like(wd.query, 7.0)
+        _cabi.check(L.fa_paged_attention_loop(
+            out.data_ptr(), wd.query.data_ptr(), wd.key_cache.data_ptr(), wd.value_cache.data_ptr(), wd.block_tables.data_ptr(),
+            wd.context_lens.data_ptr(), w.scale, 0, ctypes.byref(sh), ctypes.byref(op)))
+        outs.append(out)
+    torch.cuda.synchronize()
+    assert torch.equal(*outs)
+    _check(oracle, w, outs[0])
+
+
+def test_graph_replays_and_overlapping_streams(oracle):
+    from flash_attention_factory_amd import torch_ops  # noqa: F401
+    dev = torch.device("cuda:0")
+    w = _workload([6000, 1400, 3000], 4, 4, 128)
+    wd = w.to(dev)
+    query, lens, out = wd.query.clone(), wd.context_lens.clone(), torch.zeros_like(wd.query)
+
+    def op(o, q, n):
+        torch.ops.fa_amd.paged_attention_loop(o, q, wd.key_cache, wd.value_cache, wd.block_tables, n, w.scale)
+
+    eager = torch.zeros_like(out)
+    op(eager, query, lens)
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        op(out, query, lens)
+        op(out, query, lens)
+    streams = [torch.cuda.Stream(), torch.cuda.Stream()]
+    for it in range(4):
+        query.copy_(torch.randn_like(query))
+        lens.copy_(torch.tensor([6000 - 977 * it, 1400 + 700 * it, 3000 - it], dtype=torch.int32))
+        op(eager, query, lens)
+        out.zero_()
+        torch.randn(1 << 20, device=dev).sum()
+        graph.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(out, eager), f"replay {it}"
+        others = [torch.zeros_like(out) for _ in range(8)]
+        torch.cuda.synchronize()
+        for k, o in enumerate(others):
+            with torch.cuda.stream(streams[k & 1]):
+                op(o, query, lens)
+        torch.cuda.synchronize()
+        assert all(torch.equal(o, eager) for o in others), f"streams {it}"

@@ -1,0 +1,60 @@
+"""fa_paged_attention_loop_workspace_bytes and the checks of the workspace that goes with the options
+(validate_only launches nothing, so no GPU is needed)."""
+import ctypes
+
+import pytest
+
+from flash_attention_factory_amd import _cabi
+
+
+def _call(seqs=3, kv_heads=8, group=4, d=128, blocks=256, block=16, **opts):
+    sh, op = _cabi.Shape(), _cabi.Options()
+    sh.num_seqs, sh.num_heads, sh.num_kv_heads, sh.head_size = seqs, kv_heads * group, kv_heads, d
+    sh.block_size, sh.max_blocks_per_seq, sh.max_num_partitions = block, blocks, 1
+    sh.kv_block_stride, sh.kv_token_stride, sh.kv_head_stride = block * kv_heads * d, d, block * d
+    sh.num_pool_blocks = 4096
+    for k, v in opts.items():
+        setattr(op, k, v)
+    return sh, op
+
+
+def _bytes(fp8=0, **kw):
+    sh, op = _call(**kw)
+    return _cabi.load().fa_paged_attention_loop_workspace_bytes(ctypes.byref(sh), ctypes.byref(op), fp8)
+
+
+def test_who_asks_for_workspace():
+    assert _bytes() > 0
+    assert _bytes(seqs=48) > 0 and _bytes(seqs=49) == 0              # 384 rows, 392
+    assert _bytes(blocks=80) == 0 and _bytes(blocks=81) > 0          # 1280 keys stay whole
+    assert _bytes(fp8=1, blocks=160) == 0 and _bytes(fp8=1, blocks=161) > 0
+    assert _bytes(schedule=_cabi.FA_SCHEDULE_GRID) == 0
+    assert _bytes(query_len=4) > 0 and _bytes(query_len=5) == 0      # 16 columns, 20
+    assert _bytes(mask_flags=_cabi.FA_MASK_WINDOW, window_left=1000) == 0
+    assert _bytes(mask_flags=_cabi.FA_MASK_WINDOW, window_left=2000) > 0
+    assert _bytes(d=96) == 0                                         # not a valid call
+    assert _bytes() <= 16 << 20
+
+
+@pytest.mark.parametrize("fp8", [0, 1])
+def test_argument_checks(fp8):
+    L = _cabi.load()
+    sh, _ = _call(blocks=1024)
+    need = _bytes(fp8=fp8, blocks=1024)
+    full = _cabi.OptionsWorkspace()
+    assert ctypes.sizeof(full) == full.struct_size == 120 and _cabi.OptionsWorkspace.workspace.offset == 104
+    full.validate_only = 1
+    room = (ctypes.c_char * 64)()
+    p = (ctypes.addressof(room) + 15) // 16 * 16
+    entry = L.fa_paged_attention_fp8_loop if fp8 else L.fa_paged_attention_loop
+
+    def call(space, size):
+        full.workspace, full.workspace_bytes = space, size
+        return entry(p, p, p, p, p, p, 1.0, 0, ctypes.byref(sh), ctypes.byref(full))
+
+    assert call(p, need) == _cabi.FA_OK
+    assert call(None, 0) == _cabi.FA_OK
+    assert call(p, need - 1) == _cabi.FA_ERR_SCRATCH_TOO_SMALL and b"asks for" in L.fa_last_error()
+    assert call(p + 8, need) == _cabi.FA_ERR_BAD_SHAPE
+    full.struct_size = 112  # half of the workspace's fields
+    assert call(p, need) == _cabi.FA_ERR_BAD_SHAPE and b"options.struct_size" in L.fa_last_error()
