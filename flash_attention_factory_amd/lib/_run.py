@@ -12,12 +12,13 @@ from __future__ import annotations
 
 import ctypes
 import warnings
-from contextlib import nullcontext
 from typing import List, Optional
 
 import torch
 
 from .. import _cabi
+
+_Times = ctypes.c_float * 2
 
 _scratch = {}
 _warned_scratch = False
@@ -121,7 +122,6 @@ def run_impl(entry: str, split: bool, fp8: bool, max_logits, exp_sums, tem_outpu
     if key_cache.size(1) != block_size:
         raise _cabi.PagedAttentionError(_cabi.FA_ERR_UNSUPPORTED_HEAD_OR_BLOCK_SIZE,
                                         "Unsupported head size or block size")
-    elapsed = (ctypes.c_float * 2)(0.0, 0.0)
     op = _cabi.Options() if split else _cabi.OptionsWorkspace()
     op.sinks = sinks.data_ptr() if sinks is not None else None
     op.alibi_slopes = alibi_slopes.data_ptr() if alibi_slopes is not None else None
@@ -149,7 +149,9 @@ def run_impl(entry: str, split: bool, fp8: bool, max_logits, exp_sums, tem_outpu
     # bytes are E5M2 as upstream fixes them (paged_attention_fp8_loop.cpp:43) unless the tensor says E4M3
     op.kv_fp8_format = _cabi.FA_FP8_E4M3 if key_cache.dtype == torch.float8_e4m3fn else _cabi.FA_FP8_E5M2
     op.stream = torch.cuda.current_stream(query.device).cuda_stream
-    op.elapsed_us = ctypes.cast(elapsed, ctypes.POINTER(ctypes.c_float)) if timed else None
+    if timed:
+        elapsed = _Times(0.0, 0.0)
+        op.elapsed_us = elapsed
     fn = getattr(L, entry)
     args = [output.data_ptr(), query.data_ptr(), key_cache.data_ptr(), value_cache.data_ptr(),
             block_tables.data_ptr(), context_lens.data_ptr(), float(sm_scale), int(max_context_len)]
@@ -172,8 +174,7 @@ def run_impl(entry: str, split: bool, fp8: bool, max_logits, exp_sums, tem_outpu
         if need > 0:
             space = torch.empty(need, dtype=torch.uint8, device=query.device)
             op.workspace, op.workspace_bytes = space.data_ptr(), need
-    # (entering torch.cuda.device costs 2 us also where the device is the current one)
-    with nullcontext() if query.device.index == torch.cuda.current_device() else torch.cuda.device(query.device):
+    with torch.cuda.device(query.device):
         _cabi.check(fn(*args, ctypes.byref(sh), ctypes.byref(op)))
     if not timed:
         return []
