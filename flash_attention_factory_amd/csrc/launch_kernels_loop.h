@@ -146,7 +146,9 @@ inline fa_status launch_paged_attn_loop_rows(void *out, const void *query, const
                           max_ctx < kLoopPersistentMaxContext;
   // One launch per group of query tokens that fit the MFMA columns (one launch for decode): 16
   // columns, or in the persistent form two tiles of 16 held by every wavefront.
-  const RowMergeSpace merge = r.workspace ? row_merge_space(shape, r, r.max_context_len) : RowMergeSpace{};
+  // (a sub-batch of a batch that asked for no workspace has none: what is cut here was sized by the whole call)
+  RowMergeSpace merge = r.workspace ? row_merge_space(shape, r, r.max_context_len) : RowMergeSpace{};
+  if (merge.bytes > r.workspace_bytes) merge = RowMergeSpace{};
   const int per_tile = p.query_count;
   const int per_launch = (persistent && r.query_len > per_tile) ? 2 * per_tile : per_tile;
   for (int q0 = 0; q0 < r.query_len; q0 += per_launch) {
@@ -371,8 +373,10 @@ inline fa_status dispatch_paged_attention_loop_any(void *out, const void *query,
     if (workspace_bytes < space.bytes)
       return fail(FA_ERR_SCRATCH_TOO_SMALL, "workspace of %lld bytes, this call asks for %lld", (long long)workspace_bytes,
                   (long long)space.bytes);
-    r.workspace = workspace;
-    r.workspace_bytes = workspace_bytes;
+    if (space.bytes > 0) {  // (else the launches, sub-batches of this call among them, have none)
+      r.workspace = workspace;
+      r.workspace_bytes = workspace_bytes;
+    }
   }
   if (r.validate_only) return st;
   const bool bf16 = shape->q_dtype == FA_DTYPE_BF16;

@@ -170,3 +170,35 @@ def test_graph_replays_and_overlapping_streams(oracle):
                 op(o, query, lens)
         torch.cuda.synchronize()
         assert all(torch.equal(o, eager) for o in others), f"streams {it}"
+
+
+def test_a_call_that_asks_for_none_leaves_the_workspace_alone(oracle):
+    """130 sequences ask for no workspace and run as sub-batches of 65, a number that would ask for some: whatever
+    workspace comes with the call, of any size, is not touched.  (The memory behind it is this test's own: 8 MB, more
+    than the 2.7 MB that 65 sequences would ask for.)"""
+    lens = [1700, 40] * 65
+    w = _workload(lens, 2, 2, 128)
+    wide = torch.zeros((130, 256), dtype=torch.int32)
+    wide[:, :w.block_tables.shape[1]] = w.block_tables
+    w.block_tables = wide
+    assert _needs(w) == 0
+    whole, w.query = w.query, w.query[:65]
+    assert _needs(w) > 0
+    w.query = whole
+    dev = torch.device("cuda:0")
+    wd = w.to(dev)
+    memory = torch.full((8 << 20,), 0x5A, dtype=torch.uint8, device=dev)
+    L, sh, op = _cabi.load(), _cabi.Shape(), _cabi.OptionsWorkspace()
+    op.workspace, op.workspace_bytes = memory.data_ptr(), 16
+    sh.num_seqs, sh.num_heads, sh.head_size, sh.num_kv_heads = 130, 4, 128, 2
+    sh.block_size, sh.max_blocks_per_seq, sh.max_num_partitions = w.block_size, 256, 1
+    sh.kv_block_stride, sh.kv_token_stride, sh.kv_head_stride = w.kv_strides()
+    sh.num_pool_blocks, sh.q_dtype = w.key_cache.shape[0], _cabi.FA_DTYPE_F16
+    op.stream = torch.cuda.current_stream().cuda_stream
+    out = torch.full_like(wd.query, 7.0)
+    _cabi.check(L.fa_paged_attention_loop(
+        out.data_ptr(), wd.query.data_ptr(), wd.key_cache.data_ptr(), wd.value_cache.data_ptr(), wd.block_tables.data_ptr(),
+        wd.context_lens.data_ptr(), w.scale, 0, ctypes.byref(sh), ctypes.byref(op)))
+    torch.cuda.synchronize()
+    assert (memory == 0x5A).all()
+    _check(oracle, w, out)
