@@ -360,7 +360,9 @@ inline PagedAttnParams make_params(void *out, float *exp_sums, float *max_logits
   p.mask_flags = r.mask_flags;
   p.alibi_slopes = r.alibi_slopes;
   p.softcap = r.softcap;
-  p.window_left = r.window_left;
+  // A window beyond the block table masks nothing more than one as wide as the table; cut to that, a position less
+  // the window (the kernels' first visible key) stays within 32 bits for every window the caller may ask for.
+  p.window_left = (int32_t)std::min<int64_t>(r.window_left, (int64_t)s.max_blocks_per_seq * s.block_size);
   p.query_len = r.query_len;
   p.query_first = 0;
   p.query_count = std::min(r.query_len, kMaxGroup / r.group);

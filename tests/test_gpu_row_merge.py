@@ -202,3 +202,20 @@ def test_a_call_that_asks_for_none_leaves_the_workspace_alone(oracle):
     torch.cuda.synchronize()
     assert (memory == 0x5A).all()
     _check(oracle, w, out)
+
+
+@pytest.mark.parametrize("query_len", [2, 3])
+@pytest.mark.parametrize("hk", [2, 12])
+@pytest.mark.parametrize("fp8", [None, E5M2])
+def test_the_widest_window_is_none(oracle, hk, query_len, fp8):
+    """window_left = 2^31 - 1 masks nothing: the bits of the call without a window, also where a context is shorter
+    than the query tokens."""
+    w = _workload([4100, 1500, 2817, 2], hk, 4, 128, fp8)
+    dev = torch.device("cuda:0")
+    query = torch.randn((4, query_len, 4 * hk, 128), generator=torch.Generator().manual_seed(4)).to(torch.float16)
+    assert _needs(w, query_len) > 0
+    out = _run(w, dev, query=query, window_left=2**31 - 1)
+    without = _run(w, dev, query=query)
+    torch.cuda.synchronize()
+    assert torch.equal(out, without)
+    _check(oracle, w, out, query=query)
