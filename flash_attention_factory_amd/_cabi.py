@@ -195,6 +195,14 @@ def require_same_device(anchor_name: str, anchor, named_tensors) -> None:
                                       f"must live on the device of {anchor_name}")
 
 
+def require_value_pool(key_cache, value_cache) -> None:
+    """Block ids, heads and rows are checked against key_cache alone, so value_cache (of the same strides) has to
+    hold at least as much."""
+    if value_cache.shape != key_cache.shape and any(v < k for v, k in zip(value_cache.shape, key_cache.shape)):
+        raise PagedAttentionError(FA_ERR_BAD_SHAPE, f"value_cache {tuple(value_cache.shape)} is smaller than key_cache "
+                                                    f"{tuple(key_cache.shape)}")
+
+
 class PagedAttentionError(RuntimeError):
     def __init__(self, code: int, message: str):
         super().__init__(f"[fa_status {code}] {message}")

@@ -39,6 +39,13 @@ bool fits_int32(int64_t v) { return v >= std::numeric_limits<int32_t>::min() && 
 bool is_16bit(at::ScalarType t) { return t == at::kHalf || t == at::kBFloat16; }
 bool is_byte_cache(at::ScalarType t) { return t == at::kFloat8_e5m2 || t == at::kFloat8_e4m3fn || t == at::kByte; }
 
+// Block ids, heads and rows are checked against key_cache alone, so value_cache has to hold at least as much.
+bool covers(const Tensor &value_cache, const Tensor &key_cache) {
+  for (int64_t d = 0; d < key_cache.dim(); ++d)
+    if (value_cache.size(d) < key_cache.size(d)) return false;
+  return true;
+}
+
 bool same_device(const Tensor &anchor, const Tensor &t) { return t.device() == anchor.device(); }
 bool same_device(const Tensor &anchor, const OptTensor &t) { return !t.has_value() || t->device() == anchor.device(); }
 
@@ -75,6 +82,7 @@ bool attend(const Tensor &out, const Scratch *scratch, const Tensor &query, cons
   if (block_tables.scalar_type() != at::kInt || context_lens.scalar_type() != at::kInt) return false;
   if ((fp8 ? !is_byte_cache(kv_type) : kv_type != q_type) || value_cache.scalar_type() != kv_type) return false;
   if (key_cache.dim() != 4 || key_cache.stride(3) != 1 || value_cache.strides() != key_cache.strides()) return false;
+  if (!covers(value_cache, key_cache)) return false;
   if ((query.dim() != 3 && query.dim() != 4) || out.sizes() != query.sizes()) return false;
   const int64_t S = query.size(0), QL = query.dim() == 4 ? query.size(1) : 1, H = query.size(-2), D = query.size(-1);
   const int64_t blocks = key_cache.size(0), block_size = key_cache.size(1), kv_heads = key_cache.size(2);
@@ -166,7 +174,7 @@ bool append(const Tensor &key, const Tensor &value, const Tensor &key_cache, con
   const bool fp8 = is_byte_cache(kv_type);
   if ((!fp8 && kv_type != type) || value_cache.scalar_type() != kv_type) return false;
   if (key_cache.dim() != 4 || key_cache.stride(3) != 1 || value_cache.strides() != key_cache.strides() ||
-      key_cache.size(2) != key.size(1) || key_cache.size(3) != key.size(2))
+      !covers(value_cache, key_cache) || key_cache.size(2) != key.size(1) || key_cache.size(3) != key.size(2))
     return false;
   if (slot_mapping.scalar_type() != at::kLong || !slot_mapping.is_contiguous() || slot_mapping.numel() != key.size(0)) return false;
   for (int64_t v : {key.size(0), key.size(1), key.size(2), key_cache.size(1)})

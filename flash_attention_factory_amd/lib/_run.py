@@ -89,6 +89,7 @@ def run_impl(entry: str, split: bool, fp8: bool, max_logits, exp_sums, tem_outpu
         raise _cabi.PagedAttentionError(_cabi.FA_ERR_BAD_SHAPE,
                                         "caches must be 4-D [blocks, block_size, kv_heads, head_size] "
                                         "views with a contiguous last dimension and equal strides")
+    _cabi.require_value_pool(key_cache, value_cache)
     # [S, H, D], or [S, query_len, H, D]: several query tokens per sequence (causal among themselves)
     if query.dim() == 4:
         S, QL, H, D = query.shape

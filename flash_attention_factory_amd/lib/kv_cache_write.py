@@ -46,6 +46,7 @@ def run(key: torch.Tensor, value: torch.Tensor, key_cache: torch.Tensor, value_c
         raise _cabi.PagedAttentionError(_cabi.FA_ERR_BAD_SHAPE,
                                         "caches must be 4-D [blocks, block_size, kv_heads, head_size] views "
                                         "matching key/value, with equal strides")
+    _cabi.require_value_pool(key_cache, value_cache)
     if slot_mapping.dtype != torch.int64 or not slot_mapping.is_contiguous() or slot_mapping.numel() != key.size(0):
         raise _cabi.PagedAttentionError(_cabi.FA_ERR_BAD_SHAPE, "slot_mapping must be contiguous int64 [tokens]")
     sh = _cabi.KvWriteShape()

@@ -182,3 +182,27 @@ def test_versions_streams_and_inference_mode():
         except Exception as e:  # noqa: BLE001
             outcomes.append((type(e), str(e)))
     assert outcomes[0] == outcomes[1]
+
+
+@pytest.mark.parametrize("ns", ["fa_amd", "fa_amd_py"])
+@pytest.mark.parametrize("fp8", [False, True])
+@pytest.mark.parametrize("smaller", [lambda t: t[:-1], lambda t: t[:, :8], lambda t: t[:, :, :1], lambda t: t[..., :64]],
+                         ids=["blocks", "block size", "kv heads", "head size"])
+def test_a_value_pool_smaller_than_the_key_pool_is_refused(smaller, fp8, ns):
+    """Block ids, heads and rows are checked against the key pool, so a smaller value pool would be read, and
+    written, beyond its end.  A larger one is as good as an equal one."""
+    st = _state(fp8)
+    st["value_cache"] = smaller(st["value_cache"])
+    for split in (False, True):
+        with pytest.raises(RuntimeError, match="smaller than key_cache"):
+            _call(ns, st, fp8, split)
+    key, slots = st["query"][:, :HK].contiguous(), torch.tensor([5, -1, 77], device="cuda:0")
+    with pytest.raises(RuntimeError, match="smaller than key_cache"):
+        getattr(torch.ops, ns).kv_cache_write(key, key.clone(), st["key_cache"], st["value_cache"], slots)
+    st, fewer = _state(fp8), _state(fp8)
+    st["block_tables"].clamp_(max=NB - 2)
+    fewer.update(block_tables=st["block_tables"], key_cache=fewer["key_cache"][:-1])
+    for t in (st, fewer):
+        _call(ns, t, fp8, False)
+    torch.cuda.synchronize()
+    assert torch.equal(st["out"], fewer["out"])
