@@ -22,6 +22,7 @@
 #include "../../include/fa_paged_attention.h"
 #include "paged_attention_kernel.h"
 #include "paged_attention_lds_kernel.h"
+#include "paged_attention_loop_cut_kernel.h"
 #include "paged_attention_loop_persistent_kernel.h"
 #include "paged_attention_loop_two_tile_kernel.h"
 #include "paged_attention_policy.h"
@@ -389,7 +390,6 @@ inline PagedAttnParams make_params(void *out, float *exp_sums, float *max_logits
   p.merge_pieces = nullptr;  // (these, the loop path's launcher where rows are cut)
   p.merge_flags = nullptr;
   p.merge_nonce = 0;
-  p.merge_whole_partitions = 0;
   p.kv_rows_apart = s.kv_token_stride != s.head_size;
   p.segment_force = r.segment_partitions;
   p.pair_heads = 0;

@@ -46,23 +46,21 @@ namespace fa {
 //   8 rows of 30011 keys 402 -> 32 (the split path's two kernels: 37), 24 rows of 900-4096 keys 49 -> 18, 110 rows
 //   of 622-5556 keys 53 -> 19, 64 rows of 8192-32768 keys 432 -> 113 (floor 103), 320 rows of 2698-5095 keys 146 -> 105
 // Beyond kRowMergeMaxItems rows units have two rows each and cutting gives little: 416 to 720 rows measured between
-// 0.91 and 1.02 of the whole rows' speed.  Rows that stay whole cost 0.1 to 1 us more here than in the persistent loop
-// kernel (16-bit cache 6.7 -> 6.9, byte cache 6.4 -> 7.2: the kernel is twice its size and starts cold), so a call whose
-// bound already says that they will be takes that kernel.
+// 0.91 and 1.02 of the whole rows' speed.  Rows that stay whole take as long as in the persistent loop kernel (0.4 to
+// 0.6 us more where some are long: paged_attention_loop_cut_kernel.h); a call whose bound already says that all are
+// short takes that kernel.
 #ifndef FA_ROW_MERGE_MAX_ITEMS
 #define FA_ROW_MERGE_MAX_ITEMS 384
-#endif
-#ifndef FA_ROW_MERGE_WHOLE_PARTITIONS
-#define FA_ROW_MERGE_WHOLE_PARTITIONS 5
 #endif
 #ifndef FA_ROW_MERGE_PIECE_BYTES
 #define FA_ROW_MERGE_PIECE_BYTES (128 << 10)
 #endif
 constexpr int kRowMergeMaxItems = FA_ROW_MERGE_MAX_ITEMS;
 // Pieces are a whole number of partitions of this many bytes of K and V, two at least; rows of up to
-// kRowMergeWholePartitions of them stay whole.
+// kMergeWholePartitions of them stay whole.
 constexpr int kRowMergePartitionBytes = FA_ROW_MERGE_PIECE_BYTES;
-constexpr int kRowMergeWholePartitions = FA_ROW_MERGE_WHOLE_PARTITIONS;
+static_assert((kRowMergePartitionBytes & (kRowMergePartitionBytes - 1)) == 0, "MergeRows::cut shifts");
+static_assert(kMergeMaxSeqs == kLoopPersistentMaxSeqs, "a launch takes as many rows whole as in pieces");
 
 // Wavefronts per work-group; wide where the launch without cuts would be (FA_PLOOP_WIDE).
 template <bool kWide>
@@ -93,7 +91,7 @@ inline RowMergeSpace row_merge_space(const fa_paged_attention_shape &shape, cons
     return space;
   if (r.query_len > kMaxGroup / group) return space;  // (two column tiles per wavefront)
   if (items > kRowMergeMaxItems || visible_row_bound(shape, r, max_context_len) <=
-                                       kRowMergeWholePartitions * row_merge_partition(head_size * r.kv_elem_bytes))
+                                       kMergeWholePartitions * row_merge_partition(head_size * r.kv_elem_bytes))
     return space;
   // one slice per wavefront, of four wavefronts or of eight (see the launch)
   const int slices = head_size == 128 ? kMergeWaves<true> : kMergeWaves<false>;
@@ -156,28 +154,28 @@ inline fa_status launch_paged_attn_loop_rows(void *out, const void *query, const
     p.query_count = std::min(per_launch, r.query_len - q0);
     if (persistent && merge.bytes > 0) {
       // few rows: cut into pieces, merged within the launch
-      constexpr int SW = kMergeWaves<false>, SO = SegmentSplit<KV8>::occ, TPC = Pipeline<KV8>::tiles_per_chunk;
-      auto kernel = ext ? paged_attn_segment_kernel<HEAD_SIZE, QT, KVF, SW, SO, TPC, true, 1, true, KROW>
-                        : paged_attn_segment_kernel<HEAD_SIZE, QT, KVF, SW, SO, TPC, false, 1, true, KROW>;
+      constexpr int SW = kMergeWaves<false>, SO = PersistentLoop<KV8>::occ, TPC = Pipeline<KV8>::tiles_per_chunk;
+      auto kernel = ext ? paged_attn_loop_cut_kernel<HEAD_SIZE, QT, KVF, SW, SO, TPC, true, KROW>
+                        : paged_attn_loop_cut_kernel<HEAD_SIZE, QT, KVF, SW, SO, TPC, false, KROW>;
       int waves = SW, resident = 0, cus = 0;
       FA_HIP_CHECK(compute_units_of_current_device(&cus));
       if constexpr (HEAD_SIZE == 128) {
         if (FA_PLOOP_WIDE && !ext && 2 * items <= cus) {
           waves = kMergeWaves<true>;
-          kernel = paged_attn_segment_kernel<HEAD_SIZE, QT, KVF, kMergeWaves<true>, SO, TPC, false, 1, true, KROW>;
+          kernel = paged_attn_loop_cut_kernel<HEAD_SIZE, QT, KVF, kMergeWaves<true>, SO, TPC, false, KROW>;
         }
       }
       FA_HIP_CHECK(resident_groups(kernel, waves * 64, &resident));
       p.compute_units = cus;
       p.segment_force = 0;
       p.partition_size = row_merge_partition(HEAD_SIZE * (KV8 ? 1 : 2));
-      p.merge_whole_partitions = kRowMergeWholePartitions;
-      p.max_num_partitions = INT32_MAX;
       p.merge_flags = static_cast<uint64_t *>(r.workspace);
       p.merge_pieces = reinterpret_cast<float *>(p.merge_flags + merge.flags);
       p.merge_nonce = next_merge_nonce();
       const int64_t most = items * ((max_ctx + p.partition_size - 1) / p.partition_size);
-      FA_HIP_CHECK(timer.launch(kernel, dim3((unsigned)std::min<int64_t>(resident, most)), dim3(waves * 64), 0, p));
+      // (a work-group for every row at least, resident or not: nobody waits for another)
+      const int64_t groups = std::max(items, std::min<int64_t>(resident, most));
+      FA_HIP_CHECK(timer.launch(kernel, dim3((unsigned)groups), dim3(waves * 64), 0, p));
     } else if (persistent && r.schedule == FA_SCHEDULE_VALU) {
       if constexpr (HEAD_SIZE == 128 && std::is_same<QT, F16>::value) {
         constexpr int VW = FA_VALU_WAVES;

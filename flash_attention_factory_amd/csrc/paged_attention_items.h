@@ -53,14 +53,17 @@ struct LoopItems {
     head_shift = stack_affine_shift(p.kv_head_bytes * heads_per_item, Hk);
     const int max_ctx = p.max_blocks_per_seq << p.block_shift;
     const int col_max = p.max_blocks_per_seq - 1;
+    // (both lengths are asked for before either is looked at)
+    if (lane < S) len0 = p.context_lens[lane];
+    if (S > 64 && lane + 64 < S) len1 = p.context_lens[lane + 64];
     if (lane < S) {
-      len0 = max(0, min(p.context_lens[lane], max_ctx));
       const int32_t *row = p.block_tables + (int64_t)lane * p.max_blocks_per_seq;
 #pragma unroll
       for (int t = 0; t < TPC; ++t) sid0[t] = row[min((wave * chunk_tokens + t * kTileTokens) >> p.block_shift, col_max)];
+      len0 = max(0, min(len0, max_ctx));
     }
     if (S > 64 && lane + 64 < S) {
-      len1 = max(0, min(p.context_lens[lane + 64], max_ctx));
+      len1 = max(0, min(len1, max_ctx));
       const int32_t *row = p.block_tables + (int64_t)(lane + 64) * p.max_blocks_per_seq;
 #pragma unroll
       for (int t = 0; t < TPC; ++t) sid1[t] = row[min((wave * chunk_tokens + t * kTileTokens) >> p.block_shift, col_max)];
@@ -119,19 +122,47 @@ struct LoopItems {
   }
 };
 
+// The rows of a launch that may cut them and merge the pieces itself (paged_attention_row_merge.h), before the
+// decision: lane holds sequences lane and lane + 64.
+struct MergeRows {
+  int base[2];   // first key that is read: the partition of the row's earliest key inside the local window
+  int keys[2];   // keys from there on
+  int parts[2];  // partitions of them
+  int total;     // of all sequences
+
+  // Whether the launch cuts its rows.  len0, len1: lengths as LoopItems has them (negative: no sequence).  Every
+  // wavefront goes through this before its first load of keys, at the speed at which instructions arrive from memory:
+  // partitions are a power of two long (row_merge_partition) and everything fits 32 bits (rows below 2^23 keys and
+  // 2^15 partitions, at most 2^9 of them).
+  __device__ __forceinline__ bool cut(const PagedAttnParams &p, int len0, int len1) {
+    const int log2 = 31 - __builtin_clz(p.partition_size);
+    const int len[2] = {max(len0, 0), max(len1, 0)};
+    int longest = 0, live = 0, sum = 0;
+#pragma unroll
+    for (int j = 0; j < 2; ++j) {
+      base[j] = 0;
+      if (p.mask_flags & kMaskWindow)
+        base[j] = max(0, len[j] - p.query_len + p.query_first - p.window_left) >> log2 << log2;
+      keys[j] = len[j] - base[j];
+      parts[j] = (keys[j] + p.partition_size - 1) >> log2;
+      longest = max(longest, parts[j]);
+      sum += parts[j];
+      live += __builtin_popcountll(__ballot(parts[j] > 0));
+    }
+    total = wave_total(sum);
+    longest = __builtin_amdgcn_readfirstlane(__reduce_max_sync(~0ull, longest));
+    return cut_pays(longest, total, live, p.num_kv_heads, p.compute_units);
+  }
+};
+
 // ROW_MERGE: for a launch that merges the pieces of a row itself (paged_attention_row_merge.h).  A row then begins
 // at the partition of its first key inside the local window, the length of a piece grows until there are no more
 // than kMergeWholePieces whole ones, part0 is the piece's number within the row, and pieces are numbered.
 template <bool ROW_MERGE = false>
 struct SegmentItems {
   static constexpr int NQ = (ROW_MERGE ? kMergeMaxSeqs : kSegmentMaxSeqs) / 64;
-  static constexpr int kIdTiles = ROW_MERGE ? 2 : 0;
   int ctxv[NQ], parts[NQ], incl[NQ], fullc[NQ], key[NQ];
-  // ROW_MERGE: first key of the row that is read; block ids of chunk `first_chunk` of every sequence, requested
-  // with the lengths, so that a work-group whose first item begins a row waits for one trip to memory, not two;
-  // whether rows are cut, and if not, whether every row has a work-group of its own
-  int base[ROW_MERGE ? NQ : 1], sid[ROW_MERGE ? NQ : 1][ROW_MERGE ? kIdTiles : 1];
-  bool one_row_each = false, have_first_ids = false;
+  int base[ROW_MERGE ? NQ : 1];  // ROW_MERGE: first key of the row that is read
   int S, Hk, m, seg_tokens, full_total, total_items, lane, key_top_bit, psize;
   int head_shift = -1;  // stack_affine_shift of the pool
   // even shares (m == 0): tape[j] = cost of all rows up to and including the lane's sequence's (row_cost);
@@ -145,107 +176,59 @@ struct SegmentItems {
   // heads_per_item: adjacent kv heads that one work-group takes together (its wavefronts in teams);
   // item_row_bytes: bytes of one token's K row (as of its V row) of an item
   __device__ __forceinline__ void build(const PagedAttnParams &p, int lane_, int groups, int heads_per_item,
-                                        int item_row_bytes, [[maybe_unused]] int first_chunk = 0,
-                                        [[maybe_unused]] int chunk_tokens = 32) {
+                                        int item_row_bytes) {
+    static_assert(!ROW_MERGE);
+    begin(p, lane_, heads_per_item);
+    const int max_ctx = p.max_blocks_per_seq << p.block_shift;
+    const int total_parts = count_partitions<NQ>(p.context_lens, S, max_ctx, p.partition_size, p.max_num_partitions, lane, ctxv, parts);
+    // (cost of the batch in steps of kShareTokens, from above: every partition full, every row a piece)
+    const long long steps_at_most = ((long long)total_parts * (psize >> kShareTokensLog2) + (long long)S * kSharePieceCost) * Hk;
+    even = p.segment_force == -1 && steps_at_most < (1 << 24);  // (a batch beyond that is cut into segments)
+    if (even) {
+      build_even_shares(groups, p.compute_units);
+      return;
+    }
+    m = p.segment_force > 0 ? min(p.segment_force, kSegmentMaxPartitions)
+                            : partitions_per_segment<NQ>(ctxv, parts, total_parts, S, p.partition_size, Hk, groups,
+                                                         p.compute_units, p.kv_rows_apart != 0,
+                                                         2 * p.partition_size * item_row_bytes);
+    cut_rows();
+  }
+  // ROW_MERGE: rows as cut_pays saw them
+  __device__ __forceinline__ void build(const PagedAttnParams &p, const MergeRows &rows, int lane_, int groups, int item_row_bytes) {
+    static_assert(ROW_MERGE);
+    begin(p, lane_, 1);
+#pragma unroll
+    for (int j = 0; j < NQ; ++j) {
+      ctxv[j] = rows.keys[j];
+      parts[j] = rows.parts[j];
+      base[j] = rows.base[j];
+    }
+    m = partitions_per_segment<NQ>(ctxv, parts, rows.total, S, p.partition_size, Hk, groups, p.compute_units,
+                                   p.kv_rows_apart != 0, 2 * p.partition_size * item_row_bytes);
+    m = max(m, 2);  // (a piece costs its merge whatever its length)
+    const int max_ctx = p.max_blocks_per_seq << p.block_shift;
+    while (true) {  // ends: one whole piece per row at most once m spans the longest
+      int whole, all;
+      count_segments<NQ>(ctxv, parts, S, p.partition_size, m, whole, all);
+      if ((int64_t)whole * Hk <= kMergeWholePieces || (int64_t)m * psize >= max_ctx) break;
+      m *= 2;
+    }
+    cut_rows();
+  }
+  __device__ __forceinline__ void begin(const PagedAttnParams &p, int lane_, int heads_per_item) {
     lane = lane_;
     S = p.num_seqs;
     Hk = p.num_kv_heads / heads_per_item;
     head_shift = stack_affine_shift(p.kv_head_bytes * heads_per_item, Hk);
-    const int max_ctx = p.max_blocks_per_seq << p.block_shift;
     psize = p.partition_size;
-    if constexpr (ROW_MERGE) {
-      // (only the work-groups that have an item if rows stay whole: thousands of wavefronts asking for the same
-      // lines hold up the few that wait for them)
-      have_first_ids = (int)blockIdx.x < S * Hk;
-#pragma unroll
-      for (int j = 0; j < NQ; ++j)
-        if (have_first_ids && j * 64 < S) {  // (lanes past the batch ask for the last sequence's)
-          const int32_t *row = p.block_tables + (int64_t)min(lane + 64 * j, S - 1) * p.max_blocks_per_seq;
-#pragma unroll
-          for (int t = 0; t < kIdTiles; ++t)
-            sid[j][t] = row[min((first_chunk * chunk_tokens + t * kTileTokens) >> p.block_shift, p.max_blocks_per_seq - 1)];
-        }
-    }
-    if constexpr (ROW_MERGE) {
-      // No row long enough to be cut and a work-group for each: known from the lengths alone, and as little code as
-      // can be until the first loads go out (a launch of short rows lasts 6 us, and its code comes from memory too).
-      int len[NQ];
-      bool any_long = false;
-#pragma unroll
-      for (int j = 0; j < NQ; ++j) len[j] = p.context_lens[min(lane + 64 * j, S - 1)];
-#pragma unroll
-      for (int j = 0; j < NQ; ++j) {
-        ctxv[j] = max(0, min(len[j], max_ctx));
-        base[j] = 0;
-        any_long |= ctxv[j] > p.merge_whole_partitions * psize;
-      }
-      one_row_each = !__any(any_long) && S * Hk <= groups;
-      if (one_row_each) return;
-    }
-    int total_parts = count_partitions<NQ>(p.context_lens, S, max_ctx, p.partition_size, p.max_num_partitions, lane, ctxv, parts);
-    if constexpr (ROW_MERGE) {
-      const bool window = p.mask_flags & kMaskWindow;
-#pragma unroll
-      for (int j = 0; j < NQ; ++j) base[j] = 0;
-      if (window) {  // (wave-uniform) rows from the partition of the earliest key that some query token sees
-        int local = 0;
-        const float inv = __builtin_amdgcn_rcpf((float)psize);
-#pragma unroll
-        for (int j = 0; j < NQ; ++j) {
-          int rem;
-          const int skip = quotient_below_2p24(max(0, ctxv[j] - p.query_len + p.query_first - p.window_left), psize, inv, rem);
-          base[j] = skip * psize;
-          ctxv[j] -= base[j];
-          parts[j] -= skip;
-          local += parts[j];
-        }
-        total_parts = wave_total(local);
-      }
-    }
-    if constexpr (!ROW_MERGE) {
-      // (cost of the batch in steps of kShareTokens, from above: every partition full, every row a piece)
-      const long long steps_at_most = ((long long)total_parts * (psize >> kShareTokensLog2) + (long long)S * kSharePieceCost) * Hk;
-      even = p.segment_force == -1 && steps_at_most < (1 << 24);  // (a batch beyond that is cut into segments)
-      if (even) {
-        build_even_shares(groups, p.compute_units);
-        return;
-      }
-    }
-    bool cut = true;
-    int longest = 0, live = 0;  // (ROW_MERGE) partitions of the longest row, rows per kv head
-    if constexpr (ROW_MERGE) {
-#pragma unroll
-      for (int j = 0; j < NQ; ++j) {
-        longest = max(longest, parts[j]);
-        if (j * 64 < S) live += __builtin_popcountll(__ballot(parts[j] > 0));
-      }
-      longest = __builtin_amdgcn_readfirstlane(__reduce_max_sync(~0ull, longest));
-      cut = cut_pays(longest, total_parts, live, Hk, p.compute_units, p.merge_whole_partitions);
-    }
-    if constexpr (ROW_MERGE) {
-      one_row_each = !cut && S * Hk <= groups;
-      if (one_row_each) return;  // nobody takes a second item, so the order of the rows is of no matter
-    }
-    if (!cut) m = max(longest, 1);
-    else
-      m = p.segment_force > 0 ? min(p.segment_force, kSegmentMaxPartitions)
-                              : partitions_per_segment<NQ>(ctxv, parts, total_parts, S, p.partition_size, Hk, groups,
-                                                           p.compute_units, p.kv_rows_apart != 0,
-                                                           2 * p.partition_size * item_row_bytes);
-    if constexpr (ROW_MERGE) {
-      m = max(m, 2);  // (a piece costs its merge whatever its length)
-      while (true) {  // ends: one whole piece per row at most once m spans the longest
-        int whole, all;
-        count_segments<NQ>(ctxv, parts, S, p.partition_size, m, whole, all);
-        if ((int64_t)whole * Hk <= kMergeWholePieces || (int64_t)m * psize >= max_ctx) break;
-        m *= 2;
-      }
-    }
-    seg_tokens = m * p.partition_size;
+  }
+  __device__ __forceinline__ void cut_rows() {
+    seg_tokens = m * psize;
     int running = 0, tails = 0;
 #pragma unroll
     for (int j = 0; j < NQ; ++j) {
-      const int cut = min(ctxv[j], parts[j] * p.partition_size);  // what the scratch arrays can hold
+      const int cut = min(ctxv[j], parts[j] * psize);  // what the scratch arrays can hold
       ctxv[j] = cut;
       fullc[j] = cut / seg_tokens;
       const int rem = cut - fullc[j] * seg_tokens;
@@ -375,35 +358,6 @@ struct SegmentItems {
     }
     return 255 - (found & 255);
   }
-  // ROW_MERGE, uncut rows, at least as many work-groups as rows: row number `group`.
-  __device__ __forceinline__ bool row_of_group(int n, int group, int chunk_tokens, MergeItem &it) const {
-    if (n > 0 || group >= S * Hk) return false;
-    const int s = __builtin_amdgcn_readfirstlane(group / Hk);
-    int ctx_s = 0, base_s = 0;
-#pragma unroll
-    for (int j = 0; j < NQ; ++j)
-      if ((s >> 6) == j) {
-        ctx_s = __builtin_amdgcn_readlane(ctxv[j], s & 63);
-        base_s = __builtin_amdgcn_readlane(base[ROW_MERGE ? j : 0], s & 63);
-      }
-    it.seq = s;
-    it.kvh = stack_affine_head(group - s * Hk, head_shift);
-    it.ctx = it.tok_end = base_s + ctx_s;
-    it.c_lo = base_s / chunk_tokens;
-    it.c_end = (it.ctx + chunk_tokens - 1) / chunk_tokens;
-    it.part0 = 0;
-    it.parts = it.pieces = it.whole = 1;
-    it.piece = it.first_piece = it.last_piece = it.piece_step = 0;
-    return it.ctx > 0;
-  }
-  // ROW_MERGE: block id of tile t of chunk `first_chunk` of a sequence.
-  __device__ __forceinline__ int first_id(int t, int seq) const {
-    int id = 0;
-#pragma unroll
-    for (int j = 0; j < NQ; ++j)
-      if ((seq >> 6) == j) id = __builtin_amdgcn_readlane(sid[ROW_MERGE ? j : 0][ROW_MERGE ? t : 0], seq & 63);
-    return id;
-  }
   // n-th item of work-group `group`, asked for n = 0, 1, 2, ... in turn.  Segments: position in the
   // sorted list -> (sequence, segment, kv head), kv head fastest.
   __device__ __forceinline__ bool at(int n, int groups, int group, int chunk_tokens,
@@ -412,9 +366,6 @@ struct SegmentItems {
       if (even) return next_of_share(chunk_tokens, it);
     }
     const int pos = snake_position(n, groups, group);
-    if constexpr (ROW_MERGE) {
-      if (one_row_each) return row_of_group(n, group, chunk_tokens, it);
-    }
     if (pos >= total_items) return false;
     const int q = __builtin_amdgcn_readfirstlane(pos / Hk);
     it.kvh = stack_affine_head(pos - q * Hk, head_shift);

@@ -51,10 +51,19 @@ constexpr int kLoopPersistentSpinLimit = 1 << 24;
 // What a kernel leaves in the status word (PagedAttnParams::status) when it gave up such a wait.
 constexpr int32_t kStatusSpinLimit = 1;
 
-//
-template <int D, typename QT, int KVF, int NWG, int OCC, int TPC, bool EXT = false, bool KROW = true, int HPW = 1>
-__global__ void __launch_bounds__(NWG * 64) __attribute__((amdgpu_waves_per_eu(OCC)))
-paged_attn_loop_persistent_kernel(const PagedAttnParams p) {
+// The LDS of a work-group of NW wavefronts whose states have NR values a lane: partial states of two items in
+// flight, item n in buffer n & 1.
+template <int NW, int NR>
+struct ItemStates {
+  float m[2][NW][16];
+  float l[2][NW][16];
+  float acc[2][NW][NR][64];
+  int arrived[2];  // wavefronts that have published into the buffer, ever
+};
+
+// Work-group `wg` of the G that share out `items`.
+template <int D, typename QT, int KVF, int NWG, int TPC, bool EXT, bool KROW, int HPW, typename States>
+__device__ __forceinline__ void walk_loop_items(const PagedAttnParams &p, LoopItems<TPC> &items, const int G, States &sm) {
   constexpr int NW = NWG;       // wavefronts of the work-group
   constexpr int NT = NW / HPW;  // of which a team of NT shares the chunks of one kv head of an item and merges
   using W = WaveAttn<D, QT, KVF, TPC, Pipeline<(KVF != 0)>::stream_loads_loop, EXT, KROW>;
@@ -68,13 +77,10 @@ paged_attn_loop_persistent_kernel(const PagedAttnParams p) {
   constexpr int SL = NR / NT;
   static_assert(NT > 1 && NW % HPW == 0 && NR % NT == 0 && SL >= 2, "merge slices the output across wavefronts");
 
-  FA_TIMELINE_STAMP(0);
-  FA_TIMELINE_WHERE();
   const int lane = threadIdx.x & 63;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int team = HPW == 1 ? 0 : wave / NT;   // which of the item's HPW adjacent kv heads
   const int tw = HPW == 1 ? wave : wave % NT;  // wavefront within the team
-  const int G = gridDim.x;
   const int wg = blockIdx.x;
   [[maybe_unused]] int timeline_chunks = 0;
   [[maybe_unused]] bool timeline_first = true;
@@ -83,8 +89,6 @@ paged_attn_loop_persistent_kernel(const PagedAttnParams p) {
   // The items, (sequence, kv head) pairs with the longest sequences first, dealt in snake order;
   // c_lo: first chunk to read (0 unless EXT)
   using Item = WorkItem;
-  LoopItems<TPC> items;
-  items.build(p, lane, tw, G, CT, HPW);
   // with HPW > 1 an item is HPW adjacent kv heads of a sequence, of which this wavefront's team
   // takes one (kvh is then the team's own head)
   auto item_at = [&](int n, Item &it) -> bool {
@@ -92,12 +96,6 @@ paged_attn_loop_persistent_kernel(const PagedAttnParams p) {
     if constexpr (HPW > 1) it.kvh = it.kvh * HPW + team;
     return there;
   };
-
-  // Partial states of two items in flight: item n goes to buffer n & 1.
-  __shared__ float sm_m[2][NW][16];
-  __shared__ float sm_l[2][NW][16];
-  __shared__ float sm_acc[2][NW][NR][64];
-  __shared__ int sm_arrived[2];  // wavefronts that have published into the buffer, ever
 
   W wa(p, lane);
   const int r = wa.r, i = wa.i;
@@ -108,7 +106,7 @@ paged_attn_loop_persistent_kernel(const PagedAttnParams p) {
   if (!item_at(0, cur)) return;  // the same for every wavefront of the work-group
   FA_TIMELINE_STAMP(1);
   if constexpr (EXT) cur.c_lo = wa.first_visible_chunk(cur.ctx, 0);
-  if (threadIdx.x < 2) sm_arrived[threadIdx.x] = 0;
+  if (threadIdx.x < 2) sm.arrived[threadIdx.x] = 0;
   __syncthreads();  // the only barrier: wavefronts meet through the counters from here on
 
   // A wavefront's state of item n goes to LDS and the wavefront moves on; nobody waits here.
@@ -117,14 +115,14 @@ paged_attn_loop_persistent_kernel(const PagedAttnParams p) {
     wa.settle();
     wa.l = rows_sum(wa.l);
     if (r == 0) {
-      sm_m[b][wave][i] = wa.m;
-      sm_l[b][wave][i] = wa.l;
+      sm.m[b][wave][i] = wa.m;
+      sm.l[b][wave][i] = wa.l;
     }
 #pragma unroll
-    for (int k = 0; k < NR; ++k) sm_acc[b][wave][k][lane] = wa.acc_at(k);
+    for (int k = 0; k < NR; ++k) sm.acc[b][wave][k][lane] = wa.acc_at(k);
     __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup");
     if (lane == 0)
-      __hip_atomic_fetch_add(&sm_arrived[b], 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+      __hip_atomic_fetch_add(&sm.arrived[b], 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
   };
   // Merge the NW published states of an item, normalise, store this wavefront's slice.
   // Called one chunk into the following item (or after the last item), when the other
@@ -138,7 +136,7 @@ paged_attn_loop_persistent_kernel(const PagedAttnParams p) {
     const int target = NW * ((item >> 1) + 1);
     bool arrived = false;
     for (int spin = 0; spin < p.spin_limit; ++spin) {
-      const int seen = __hip_atomic_load(&sm_arrived[b], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+      const int seen = __hip_atomic_load(&sm.arrived[b], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
       if (__builtin_amdgcn_readfirstlane(seen) >= target) {
         arrived = true;
         break;
@@ -152,21 +150,21 @@ paged_attn_loop_persistent_kernel(const PagedAttnParams p) {
     const int w0 = team * NT;  // the team's wavefronts: w0 .. w0 + NT - 1
     float M = -INFINITY;
 #pragma unroll
-    for (int u = 0; u < NT; ++u) M = fmaxf(M, sm_m[b][w0 + u][i]);
+    for (int u = 0; u < NT; ++u) M = fmaxf(M, sm.m[b][w0 + u][i]);
     float f[NT];
     float L = 0.f;
 #pragma unroll
     for (int u = 0; u < NT; ++u) {
-      const float mw = sm_m[b][w0 + u][i];
+      const float mw = sm.m[b][w0 + u][i];
       f[u] = (mw == -INFINITY) ? 0.f : fast_exp2(mw - M);  // a wavefront without chunks
-      L += f[u] * sm_l[b][w0 + u][i];
+      L += f[u] * sm.l[b][w0 + u][i];
     }
     float o[SL];
 #pragma unroll
     for (int k = 0; k < SL; ++k) {
       float a = 0.f;
 #pragma unroll
-      for (int u = 0; u < NT; ++u) a += f[u] * sm_acc[b][w0 + u][tw * SL + k][lane];
+      for (int u = 0; u < NT; ++u) a += f[u] * sm.acc[b][w0 + u][tw * SL + k][lane];
       o[k] = a;
     }
     if (wa.col_valid && wa.keeps_output()) {
@@ -302,6 +300,19 @@ paged_attn_loop_persistent_kernel(const PagedAttnParams p) {
   finish(n, cur.seq, cur.kvh, EXT ? cur_ext.out_mul : 1.f);
   FA_TIMELINE_STAMP(4);
   FA_TIMELINE_PUT(5, timeline_chunks);
+}
+
+template <int D, typename QT, int KVF, int NWG, int OCC, int TPC, bool EXT = false, bool KROW = true, int HPW = 1>
+__global__ void __launch_bounds__(NWG * 64) __attribute__((amdgpu_waves_per_eu(OCC)))
+paged_attn_loop_persistent_kernel(const PagedAttnParams p) {
+  using W = WaveAttn<D, QT, KVF, TPC, Pipeline<(KVF != 0)>::stream_loads_loop, EXT, KROW>;
+  FA_TIMELINE_STAMP(0);
+  FA_TIMELINE_WHERE();
+  __shared__ ItemStates<NWG, W::NR> sm;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  LoopItems<TPC> items;
+  items.build(p, threadIdx.x & 63, wave % (NWG / HPW), gridDim.x, W::CT, HPW);
+  walk_loop_items<D, QT, KVF, NWG, TPC, EXT, KROW, HPW>(p, items, gridDim.x, sm);
 }
 
 }  // namespace fa

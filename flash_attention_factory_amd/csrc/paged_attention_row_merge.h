@@ -1,4 +1,4 @@
-// Loop path, rows cut into pieces (paged_attn_segment_kernel<..., ROW_MERGE = true>): how the
+// Loop path, rows cut into pieces (paged_attn_loop_cut_kernel, walk_segment_items<..., ROW_MERGE = true>): how the
 // work-groups that share a (sequence, kv head) row hand their softmax states to whichever of them is
 // last, inside one launch.
 //

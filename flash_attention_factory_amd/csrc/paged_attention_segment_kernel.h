@@ -47,13 +47,11 @@
 
 namespace fa {
 
-// ROW_MERGE: the loop path's form of the kernel.  There is no reduce launch and no tmp_out: the pieces of a row are
-// merged by the wavefronts that finish it (paged_attention_row_merge.h) and p.out is the call's `out`.
-// KROW: how K tiles are loaded, as in the loop kernels.
-template <int D, typename QT, int KVF, int NWG, int OCC, int TPC, bool EXT = false, int HPW = 1, bool ROW_MERGE = false,
-          bool KROW = true>
-__global__ void __launch_bounds__(NWG * 64) __attribute__((amdgpu_waves_per_eu(OCC)))
-paged_attn_segment_kernel(const PagedAttnParams p) {
+// The segments that `items` gives this work-group.  ROW_MERGE: the loop path's form (paged_attention_loop_cut_kernel.h).
+// There is no reduce launch and no tmp_out: the pieces of a row are merged by the wavefronts that finish it
+// (paged_attention_row_merge.h) and p.out is the call's `out`.  KROW: how K tiles are loaded, as in the loop kernels.
+template <int D, typename QT, int KVF, int NWG, int TPC, bool EXT, int HPW, bool ROW_MERGE, bool KROW, typename States>
+__device__ __forceinline__ void walk_segment_items(const PagedAttnParams &p, SegmentItems<ROW_MERGE> &items, States &sm) {
   constexpr int NW = NWG;       // wavefronts of the work-group
   constexpr int NT = NW / HPW;  // of which a team of NT shares a segment's chunks of one kv head and merges
   using W = WaveAttn<D, QT, KVF, TPC, SegmentSplit<(KVF != 0)>::stream_loads, EXT, KROW>;
@@ -71,8 +69,6 @@ paged_attn_segment_kernel(const PagedAttnParams p) {
   // NT == 1: every wavefront has a kv head of its own and the whole of each item's chunks, so an item's
   // state never leaves its registers: no LDS, no waiting for the others.
 
-  FA_TIMELINE_STAMP(0);
-  FA_TIMELINE_WHERE();
   const int lane = threadIdx.x & 63;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int team = HPW == 1 ? 0 : wave / NT;   // which of the item's HPW adjacent kv heads
@@ -86,8 +82,6 @@ paged_attn_segment_kernel(const PagedAttnParams p) {
   // in order of length, dealt to the work-groups in snake order, so that the work-groups' totals
   // come out even although a work-group only gets a handful of segments.
   using Item = std::conditional_t<ROW_MERGE, MergeItem, WorkItem>;  // c_lo .. c_end: the segment's chunks; ctx: the sequence's length (EXT)
-  SegmentItems<ROW_MERGE> items;
-  items.build(p, lane, G, HPW, W::ROWB * HPW, tw, CT);
   // n-th item of this work-group; with HPW > 1 an item is HPW adjacent kv heads of one segment, of
   // which this wavefront's team takes one (kvh is then the team's own head)
   auto item_at = [&](int nth, Item &it) {
@@ -96,16 +90,10 @@ paged_attn_segment_kernel(const PagedAttnParams p) {
     return there;
   };
 
-  // Partial states of two items in flight: the n-th item of this work-group goes to buffer n & 1.
-  __shared__ float sm_m[2][NW][16];
-  __shared__ float sm_l[2][NW][16];
-  __shared__ float sm_acc[2][NW][NR][64];
-  __shared__ int sm_arrived[2];  // wavefronts that have published into the buffer, ever
-
   Item cur;
   if (!item_at(0, cur)) return;  // the same for every wavefront of the work-group
   FA_TIMELINE_STAMP(1);
-  if (threadIdx.x < 2) sm_arrived[threadIdx.x] = 0;
+  if (threadIdx.x < 2) sm.arrived[threadIdx.x] = 0;
   __syncthreads();  // the only barrier: wavefronts meet through the counters from here on
 
   W wa(p, lane);
@@ -121,14 +109,14 @@ paged_attn_segment_kernel(const PagedAttnParams p) {
     wa.settle();
     wa.l = rows_sum(wa.l);
     if (r == 0) {
-      sm_m[b][wave][i] = wa.m;
-      sm_l[b][wave][i] = wa.l;
+      sm.m[b][wave][i] = wa.m;
+      sm.l[b][wave][i] = wa.l;
     }
 #pragma unroll
-    for (int e = 0; e < NR; ++e) sm_acc[b][wave][e][lane] = wa.acc_at(e);
+    for (int e = 0; e < NR; ++e) sm.acc[b][wave][e][lane] = wa.acc_at(e);
     __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup");
     if (lane == 0)
-      __hip_atomic_fetch_add(&sm_arrived[b], 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+      __hip_atomic_fetch_add(&sm.arrived[b], 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
   };
   // Store this wavefront's slice o[SL] of an item's merged, un-normalised output (maximum M in base-2
   // units, sum L) as the item's partial -- or, where the item is its row's only piece, as the row's result.
@@ -207,7 +195,7 @@ paged_attn_segment_kernel(const PagedAttnParams p) {
     const int target = NW * ((n >> 1) + 1);
     bool arrived = false;
     for (int spin = 0; spin < p.spin_limit; ++spin) {
-      const int seen = __hip_atomic_load(&sm_arrived[b], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+      const int seen = __hip_atomic_load(&sm.arrived[b], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
       if (__builtin_amdgcn_readfirstlane(seen) >= target) {
         arrived = true;
         break;
@@ -221,21 +209,21 @@ paged_attn_segment_kernel(const PagedAttnParams p) {
     const int w0 = team * NT;  // the team's wavefronts: w0 .. w0 + NT - 1
     float M = -INFINITY;
 #pragma unroll
-    for (int u = 0; u < NT; ++u) M = fmaxf(M, sm_m[b][w0 + u][i]);
+    for (int u = 0; u < NT; ++u) M = fmaxf(M, sm.m[b][w0 + u][i]);
     float f[NT];
     float L = 0.f;
 #pragma unroll
     for (int u = 0; u < NT; ++u) {
-      const float mw = sm_m[b][w0 + u][i];
+      const float mw = sm.m[b][w0 + u][i];
       f[u] = (mw == -INFINITY) ? 0.f : fast_exp2(mw - M);  // a wavefront without chunks
-      L += f[u] * sm_l[b][w0 + u][i];
+      L += f[u] * sm.l[b][w0 + u][i];
     }
     float o[SL];
 #pragma unroll
     for (int e = 0; e < SL; ++e) {
       float a = 0.f;
 #pragma unroll
-      for (int u = 0; u < NT; ++u) a += f[u] * sm_acc[b][w0 + u][tw * SL + e][lane];
+      for (int u = 0; u < NT; ++u) a += f[u] * sm.acc[b][w0 + u][tw * SL + e][lane];
       o[e] = a;
     }
     store_slice(it, M, L, o, out_mul);
@@ -250,17 +238,7 @@ paged_attn_segment_kernel(const PagedAttnParams p) {
   TileScales ts = {}, nts = {}, nxt_ts = {};
   if constexpr (EXT) cur_ext = wa.fetch_item_ext(cur.kvh, p.block_tables + (int64_t)cur.seq * p.max_blocks_per_seq);
   if (armed) {
-    Ids ids;
-    bool have_ids = false;
-    if constexpr (ROW_MERGE) {
-      static_assert(TPC == decltype(items)::kIdTiles, "the ids requested with the lengths are those of one chunk");
-      have_ids = items.have_first_ids && cur.c_lo == 0;
-      if (have_ids) {
-#pragma unroll
-        for (int t = 0; t < TPC; ++t) ids.v[t] = min((uint32_t)items.first_id(t, cur.seq), (uint32_t)p.max_block_id);
-      }
-    }
-    if (!have_ids) ids = wa.fetch_ids(p.block_tables + (int64_t)cur.seq * p.max_blocks_per_seq, cur.c_lo + tw, col_max);
+    const Ids ids = wa.fetch_ids(p.block_tables + (int64_t)cur.seq * p.max_blocks_per_seq, cur.c_lo + tw, col_max);
     wa.load_q(cur.seq, cur.kvh);
     wa.issue_k(R, cur.kvh, cur.c_lo + tw, ids);
     wa.issue_v(R, cur.kvh, cur.c_lo + tw, ids);
@@ -366,6 +344,18 @@ paged_attn_segment_kernel(const PagedAttnParams p) {
   finish(n, cur, EXT ? cur_ext.out_mul : 1.f);
   FA_TIMELINE_STAMP(4);
   FA_TIMELINE_PUT(5, timeline_chunks);
+}
+
+template <int D, typename QT, int KVF, int NWG, int OCC, int TPC, bool EXT = false, int HPW = 1>
+__global__ void __launch_bounds__(NWG * 64) __attribute__((amdgpu_waves_per_eu(OCC)))
+paged_attn_segment_kernel(const PagedAttnParams p) {
+  using W = WaveAttn<D, QT, KVF, TPC, SegmentSplit<(KVF != 0)>::stream_loads, EXT, true>;
+  FA_TIMELINE_STAMP(0);
+  FA_TIMELINE_WHERE();
+  __shared__ ItemStates<NWG, W::NR> sm;
+  SegmentItems<> items;
+  items.build(p, threadIdx.x & 63, gridDim.x, HPW, W::ROWB * HPW);
+  walk_segment_items<D, QT, KVF, NWG, TPC, EXT, HPW, false, true>(p, items, sm);
 }
 
 }  // namespace fa

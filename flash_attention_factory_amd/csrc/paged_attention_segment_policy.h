@@ -27,6 +27,11 @@ constexpr int kSegmentMaxPartitions = FA_SEGMENT_MAX_PARTS;
 // Launches that merge the pieces of a row themselves (paged_attention_row_merge.h): whole pieces that a launch may cut, over all its rows; what is left of a row behind its whole pieces is
 // one more.  The length of a piece grows until that holds.
 constexpr int kMergeWholePieces = 1024;
+// Rows of up to this many partitions stay whole.
+#ifndef FA_MERGE_WHOLE_PARTITIONS
+#define FA_MERGE_WHOLE_PARTITIONS 5
+#endif
+constexpr int kMergeWholePartitions = FA_MERGE_WHOLE_PARTITIONS;
 // Where work-groups share a compute unit and each should have work throughout (see `halves` below):
 // bytes of K and V that a unit must have per segment it is given.
 #ifndef FA_SEGMENT_BYTES_WORTH_CUTTING
@@ -248,17 +253,17 @@ __device__ __forceinline__ int partitions_per_segment(const int (&ctxv)[NQ], con
 // the launch lasts as long as its longest row takes one work-group, or as long as the memory takes for all rows;
 // a cut costs some 4 us (the pieces through memory, flags, merge), as much as two partitions (a partition is
 // 128 KiB of K and V: row_merge_partition).  Measured with rows cut always (us, whole -> cut):
-//   rows of up to `whole` partitions lose: 11 to 296 rows 7.7 -> 11.1, 10.6 -> 16.0, 16.8 -> 17.6, 14.0 -> 24.2
+//   rows of up to kMergeWholePartitions lose: 11 to 296 rows 7.7 -> 11.1, 10.6 -> 16.0, 16.8 -> 17.6, 14.0 -> 24.2
 //   up to one row per unit: a work-group alone on its unit streams 1 / 160 of what the memory gives 256 units, so
 //     cutting pays where the longest row exceeds that share of all rows.  Unequal rows: 24 rows 49 -> 18, 110 rows
 //     53 -> 19, 168 rows 39 -> 31; equal ones, whose sum already keeps the memory busy: 176 rows 30 -> 44, 192 rows
 //     114 -> 119, 208 rows 39 -> 43 (and 119 rows 152 -> 96, 8 rows 402 -> 32)
 //   more rows than units: a unit has two rows or one, and unequal rows meet badly.  268 rows 66 -> 46, 288 rows
 //     118 -> 94, 320 rows 147 -> 105; equal rows 384: 76 -> 88
-__device__ __forceinline__ bool cut_pays(int longest, int total, int live, int num_kv_heads, int units, int whole) {
-  if (longest <= whole) return false;
-  if (live * num_kv_heads <= units) return (long long)(longest - 2) * (units * 5 >> 3) > (long long)total * num_kv_heads;
-  return (long long)4 * longest * live > (long long)5 * total;
+__device__ __forceinline__ bool cut_pays(int longest, int total, int live, int num_kv_heads, int units) {
+  if (longest <= kMergeWholePartitions) return false;
+  if (live * num_kv_heads <= units) return (longest - 2) * (units * 5 >> 3) > total * num_kv_heads;
+  return 4 * longest * live > 5 * total;
 }
 
 // Live partitions of all sequences, as every wavefront of an attention launch computes them:

@@ -91,11 +91,10 @@ struct PagedAttnParams {
   // kernel leaves such rows alone.  NULL: every partial goes to tmp_out.
   void *final_out;
   // Loop path with rows cut into pieces (paged_attention_row_merge.h): slots of the pieces, a flag per
-  // (piece, output slice), and what a flag is set to; rows of up to merge_whole_partitions partitions stay whole.
+  // (piece, output slice), and what a flag is set to.
   float *merge_pieces;
   uint64_t *merge_flags;
   uint64_t merge_nonce;
-  int32_t merge_whole_partitions;
 };
 
 constexpr int kMaskAlibi = 1, kMaskSoftcap = 2, kMaskWindow = 4;  // = fa_mask of the C ABI

@@ -219,3 +219,28 @@ def test_the_widest_window_is_none(oracle, hk, query_len, fp8):
     torch.cuda.synchronize()
     assert torch.equal(out, without)
     _check(oracle, w, out, query=query)
+
+
+@pytest.mark.parametrize("lens, hk, group, d, fp8, kw", [
+    ([200, 900, 5, 0, 1280], 2, 4, 128, None, {}),
+    ([300, 1, 64] * 33 + [0], 2, 1, 64, None, {}),             # more than 64 sequences
+    ([2560, 7, 700], 8, 4, 128, E5M2, {}),
+    ([1500] * 20, 8, 1, 128, None, {}),                        # long enough for cuts, not worth them
+    ([2700] * 40, 8, 2, 128, E4M3, {}),                        # the same with more rows than units
+    ([1500] * 20, 8, 1, 128, None, dict(softcap=20.0, apply_softcap=True)),
+    ([2700, 3000] * 20, 8, 1, 128, E5M2, dict(window_left=2600)),
+], ids=str)
+def test_rows_that_stay_whole_are_the_persistent_loop_kernels(oracle, monkeypatch, lens, hk, group, d, fp8, kw):
+    """Given workspace, rows that the device does not cut give the bits of the call without workspace."""
+    w = _workload(lens, hk, group, d, fp8)
+    wide = torch.zeros((len(lens), 4096), dtype=torch.int32)
+    wide[:, :w.block_tables.shape[1]] = w.block_tables
+    w.block_tables = wide
+    assert _needs(w) > 0
+    dev = torch.device("cuda:0")
+    out = _run(w, dev, **dict(kw))
+    monkeypatch.setattr(_cabi.load(), "fa_paged_attention_loop_workspace_bytes", lambda *args: 0)
+    without = _run(w, dev, **dict(kw))
+    torch.cuda.synchronize()
+    assert torch.equal(out, without)
+    _check(oracle, w, out, **{k: v for k, v in kw.items() if not k.startswith("apply")})
