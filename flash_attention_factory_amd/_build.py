@@ -56,3 +56,5 @@ if __name__ == "__main__":
     ap.add_argument("--output", default=LIBRARY)
     args, flags = ap.parse_known_args()  # everything else goes to hipcc (-DFA_TIMELINE ...)
     print(build(verbose=True, extra_flags=flags, output=os.path.abspath(args.output)))
+    if not flags and os.path.abspath(args.output) == LIBRARY:
+        print(build_torch_ops(verbose=True))

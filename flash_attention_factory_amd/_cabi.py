@@ -210,6 +210,19 @@ class PagedAttentionError(RuntimeError):
 
 
 _lib = None
+_when_loaded = []
+
+
+def when_loaded(then) -> None:
+    """Call then(library) once the library is loaded: now, if it can be (else whoever loads it is told why not)."""
+    _when_loaded.append(then)
+    if _lib is not None:
+        then(_lib)
+        return
+    try:
+        load()
+    except (RuntimeError, OSError):
+        pass
 
 
 def load() -> ctypes.CDLL:
@@ -250,6 +263,8 @@ def load() -> ctypes.CDLL:
         raise RuntimeError(f"{LIBRARY} has ABI revision {L.fa_paged_attention_abi_version()}, this binding is "
                            f"written for {ABI_REVISION}: rebuild the library")
     _lib = L
+    for then in _when_loaded:
+        then(L)
     return L
 
 

@@ -25,7 +25,7 @@ namespace {
 using at::Tensor;
 using OptTensor = std::optional<Tensor>;
 
-// The C ABI's entry points, as the process has loaded them (fa_torch_ops_bind).
+// The C ABI's entry points, as the process has loaded them (fa_torch_ops_bind); null until then.
 struct Entries {
   decltype(&fa_paged_attention_loop) loop, fp8_loop;
   decltype(&fa_paged_attention_reduce) reduce, fp8_reduce;
@@ -72,7 +72,7 @@ bool attend(const Tensor &out, const Scratch *scratch, const Tensor &query, cons
             const Tensor &block_tables, const Tensor &context_lens, double scale, bool fp8, double fp8_scale,
             int64_t partition_size, const OptTensor &sinks, const OptTensor &alibi_slopes, double softcap, int64_t window_left,
             const OptTensor &k_scales, const OptTensor &v_scales, int64_t max_context_len) {
-  if (!query.is_cuda()) return false;
+  if (!entries.loop || !query.is_cuda()) return false;
   for (const Tensor *t : {&out, &key_cache, &value_cache, &block_tables, &context_lens})
     if (!same_device(query, *t)) return false;
   if (!same_device(query, sinks) || !same_device(query, alibi_slopes)) return false;
@@ -165,7 +165,7 @@ bool attend(const Tensor &out, const Scratch *scratch, const Tensor &query, cons
 
 bool append(const Tensor &key, const Tensor &value, const Tensor &key_cache, const Tensor &value_cache, const Tensor &slot_mapping,
             double fp8_scale, const OptTensor &k_scales, const OptTensor &v_scales) {
-  if (!key.is_cuda()) return false;
+  if (!entries.loop || !key.is_cuda()) return false;
   for (const Tensor *t : {&value, &key_cache, &value_cache, &slot_mapping})
     if (!same_device(key, *t)) return false;
   const auto type = key.scalar_type(), kv_type = key_cache.scalar_type();

@@ -154,9 +154,8 @@ _NAMES = ("paged_attention_loop", "paged_attention_fp8_loop", "paged_attention_r
           "kv_cache_write")
 
 
-def _load_native() -> None:
-    torch.ops.load_library(_build.TORCH_OPS_LIBRARY)
-    L = _cabi.load()
+def _bind(L: ctypes.CDLL) -> None:
+    """The C ABI's entry points, for the native operators."""
     entries = (L.fa_paged_attention_loop, L.fa_paged_attention_fp8_loop, L.fa_paged_attention_reduce,
                L.fa_paged_attention_fp8_reduce, L.fa_kv_cache_write, L.fa_paged_attention_loop_workspace_bytes)
     table = (ctypes.c_void_p * len(entries))(*(ctypes.cast(e, ctypes.c_void_p).value for e in entries))
@@ -165,7 +164,30 @@ def _load_native() -> None:
     bind(table, len(entries))
 
 
-_load_native()
+def _load_native():
+    """The native operators.  Importing this module asks for neither library: without the C ABI's library a call ends
+    in the Python operators, which say what is missing, and without the operators' own (or with one that was built
+    against another PyTorch) the calls say that."""
+    try:
+        torch.ops.load_library(_build.TORCH_OPS_LIBRARY)
+    except OSError as e:
+        why = (f"{_build.TORCH_OPS_LIBRARY} does not load: {e}: build it, against this PyTorch, with "
+               "`python -c 'import __graft_entry__ as g; g.build()'`")
+
+        def unavailable(*args, **kwargs):
+            raise RuntimeError(why)
+
+        fragment = torch.library.Library("fa_amd", "FRAGMENT")
+        for name in _NAMES:
+            op = getattr(torch.ops.fa_amd_py, name).default
+            fragment.define(str(op._schema).partition("::")[2], tags=tuple(op.tags))
+            fragment.impl(name, unavailable, "CompositeExplicitAutograd")
+        return fragment
+    _cabi.when_loaded(_bind)
+    return None
+
+
+_fragment = _load_native()
 
 # Shape propagation for tracing: every operator only writes into its arguments.
 for _name in _NAMES:
