@@ -15,6 +15,7 @@
 #include <c10/hip/HIPStream.h>
 #include <torch/library.h>
 
+#include <atomic>
 #include <limits>
 
 #include "../../include/fa_kv_cache.h"
@@ -33,6 +34,10 @@ struct Entries {
   decltype(&fa_paged_attention_loop_workspace_bytes) workspace_bytes;
 };
 Entries entries = {};
+
+// The Python operators have given their one warning of scratch that a wide table could outgrow
+// (fa_torch_ops_capacity_warned): from then on such a call has nothing to say and is launched here.
+std::atomic<bool> capacity_warned{false};
 
 bool fits_int32(int64_t v) { return v >= std::numeric_limits<int32_t>::min() && v <= std::numeric_limits<int32_t>::max(); }
 
@@ -136,9 +141,10 @@ bool attend(const Tensor &out, const Scratch *scratch, const Tensor &query, cons
         scratch->tmp_out.numel() != slots * D)
       return false;
     sh.max_num_partitions = (int32_t)partitions;
-    if (max_context_len < 0) {  // unknown: the Python operator warns where the scratch arrays may be too small
+    if (max_context_len < 0) {  // unknown: the Python operator warns, once, where the scratch arrays may be too small
       const int64_t size = partition_size > 0 ? partition_size : (D == 64 ? 256 : 512);
-      if (scratch->exp_sums.size(-1) * size < block_tables.size(1) * block_size) return false;
+      if (scratch->exp_sums.size(-1) * size < block_tables.size(1) * block_size && !capacity_warned.load(std::memory_order_relaxed))
+        return false;
       max_context_len = 0;
     }
   }
@@ -293,6 +299,8 @@ extern "C" __attribute__((visibility("default"))) void fa_torch_ops_bind(void *c
   TORCH_CHECK(count * sizeof(void *) == sizeof(Entries), "fa_torch_ops_bind: ", count, " entry points");
   memcpy(&entries, table, sizeof(Entries));
 }
+
+extern "C" __attribute__((visibility("default"))) void fa_torch_ops_capacity_warned() { capacity_warned.store(true); }
 
 TORCH_LIBRARY_FRAGMENT(fa_amd, m) {
   const std::vector<at::Tag> tags = {at::Tag::pt2_compliant_tag};

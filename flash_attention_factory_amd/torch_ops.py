@@ -63,6 +63,7 @@ def _group(query: Tensor, key_cache: Tensor) -> int:
 
 
 _warned_capacity = False
+_native = None  # libfa_torch_ops.so, once it has the entry points
 
 
 def _checked_context_len(max_context_len: int, exp_sums: Tensor, partition_size: int, query: Tensor,
@@ -76,6 +77,8 @@ def _checked_context_len(max_context_len: int, exp_sums: Tensor, partition_size:
         size = partition_size if partition_size > 0 else (256 if query.size(-1) == 64 else 512)
         if exp_sums.size(-1) * size < block_tables.size(1) * key_cache.size(1):
             _warned_capacity = True
+            if _native is not None:
+                _native.fa_torch_ops_capacity_warned()
             import warnings
             warnings.warn(f"the scratch arrays hold {exp_sums.size(-1)} partitions of {size} tokens, the block table "
                           f"{block_tables.size(1)} blocks of {key_cache.size(1)}: a context beyond "
@@ -159,9 +162,13 @@ def _bind(L: ctypes.CDLL) -> None:
     entries = (L.fa_paged_attention_loop, L.fa_paged_attention_fp8_loop, L.fa_paged_attention_reduce,
                L.fa_paged_attention_fp8_reduce, L.fa_kv_cache_write, L.fa_paged_attention_loop_workspace_bytes)
     table = (ctypes.c_void_p * len(entries))(*(ctypes.cast(e, ctypes.c_void_p).value for e in entries))
-    bind = ctypes.CDLL(_build.TORCH_OPS_LIBRARY).fa_torch_ops_bind
-    bind.argtypes, bind.restype = [ctypes.c_void_p, ctypes.c_size_t], None
-    bind(table, len(entries))
+    global _native
+    _native = ctypes.CDLL(_build.TORCH_OPS_LIBRARY)
+    _native.fa_torch_ops_bind.argtypes, _native.fa_torch_ops_bind.restype = [ctypes.c_void_p, ctypes.c_size_t], None
+    _native.fa_torch_ops_capacity_warned.argtypes, _native.fa_torch_ops_capacity_warned.restype = [], None
+    _native.fa_torch_ops_bind(table, len(entries))
+    if _warned_capacity:
+        _native.fa_torch_ops_capacity_warned()
 
 
 def _load_native():

@@ -206,3 +206,29 @@ def test_a_value_pool_smaller_than_the_key_pool_is_refused(smaller, fp8, ns):
         _call(ns, t, fp8, False)
     torch.cuda.synchronize()
     assert torch.equal(st["out"], fewer["out"])
+
+
+@pytest.mark.parametrize("fp8", [False, True])
+def test_scratch_that_a_wide_table_could_outgrow_is_warned_of_once(fp8, monkeypatch):
+    """The default max_context_len with scratch for the rows at hand and a wider table: the Python operator is there
+    for the one warning of the process, not for every call."""
+    import warnings
+    st = _state(fp8)
+    st["block_tables"] = torch.cat([st["block_tables"]] * 8, 1)   # 2560 tokens, the scratch arrays hold 1024
+    with warnings.catch_warnings():
+        warnings.simplefilter("ignore")
+        _call("fa_amd", st, fp8, True, max_context_len=-1)
+    torch.cuda.synchronize()
+    want = st["out"].clone()
+
+    def never(*args, **kwargs):
+        raise AssertionError("the Python operator was called")
+
+    for module in (torch_ops._reduce, torch_ops._fp8_reduce):
+        monkeypatch.setattr(module, "run", never)
+    st["out"].fill_(7.0)
+    with warnings.catch_warnings():
+        warnings.simplefilter("error")
+        _call("fa_amd", st, fp8, True, max_context_len=-1)
+    torch.cuda.synchronize()
+    assert torch.equal(st["out"], want)
