@@ -162,9 +162,12 @@ bool attend(const Tensor &out, const Scratch *scratch, const Tensor &query, cons
                &op) == FA_OK;
   Tensor space;
   if (const int64_t need = entries.workspace_bytes(&sh, &op, fp8); need > 0) {  // see fa_paged_attention_options_workspace
-    space = at::empty({need}, query.options().dtype(at::kByte));
-    full.workspace = space.data_ptr();
-    full.workspace_bytes = need;
+    try {
+      space = at::empty({need}, query.options().dtype(at::kByte));
+      full.workspace = space.data_ptr();
+      full.workspace_bytes = need;
+    } catch (const c10::OutOfMemoryError &) {  // the call needs none
+    }
   }
   return (fp8 ? entries.fp8_loop : entries.loop)(o, q, k, v, tables, lens, (float)scale, 0, &sh, &op) == FA_OK;
 }

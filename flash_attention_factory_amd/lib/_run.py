@@ -173,8 +173,11 @@ def run_impl(entry: str, split: bool, fp8: bool, max_logits, exp_sums, tem_outpu
         # allocator, so that calls that overlap on other streams, and graphs, have memory of their own)
         need = L.fa_paged_attention_loop_workspace_bytes(ctypes.byref(sh), ctypes.byref(op), int(fp8))
         if need > 0:
-            space = torch.empty(need, dtype=torch.uint8, device=query.device)
-            op.workspace, op.workspace_bytes = space.data_ptr(), need
+            try:
+                space = torch.empty(need, dtype=torch.uint8, device=query.device)
+                op.workspace, op.workspace_bytes = space.data_ptr(), need
+            except torch.OutOfMemoryError:
+                pass  # the call needs none
     with torch.cuda.device(query.device):
         _cabi.check(fn(*args, ctypes.byref(sh), ctypes.byref(op)))
     if not timed:

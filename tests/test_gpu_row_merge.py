@@ -244,3 +244,33 @@ def test_rows_that_stay_whole_are_the_persistent_loop_kernels(oracle, monkeypatc
     torch.cuda.synchronize()
     assert torch.equal(out, without)
     _check(oracle, w, out, **{k: v for k, v in kw.items() if not k.startswith("apply")})
+
+
+def test_a_full_gpu_leaves_rows_whole(oracle):
+    """No memory for the workspace (PyTorch's allocator is held to what it has): the call runs without."""
+    from flash_attention_factory_amd import torch_ops  # noqa: F401
+    w = _workload([6000, 1400, 3000], 2, 4, 128)
+    need = _needs(w)
+    dev = torch.device("cuda:0")
+    wd = w.to(dev)
+    outs = [torch.full_like(wd.query, 7.0) for _ in range(2)]
+    torch.cuda.empty_cache()
+    torch.cuda.set_per_process_memory_fraction(1e-9)
+    held = []
+    try:
+        for size in (need, need // 8, need // 64):  # what the allocator has left in blocks of its own
+            try:
+                while True:
+                    held.append(torch.empty(size, dtype=torch.uint8, device=dev))
+            except torch.OutOfMemoryError:
+                pass
+        with pytest.raises(torch.OutOfMemoryError):
+            torch.empty(need, dtype=torch.uint8, device=dev)
+        _run(wd, dev, out=outs[0])
+        torch.ops.fa_amd.paged_attention_loop(outs[1], wd.query, wd.key_cache, wd.value_cache, wd.block_tables, wd.context_lens, w.scale)
+    finally:
+        torch.cuda.set_per_process_memory_fraction(1.0)
+        held.clear()
+    torch.cuda.synchronize()
+    for out in outs:
+        _check(oracle, w, out)
