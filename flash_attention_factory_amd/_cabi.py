@@ -243,6 +243,9 @@ def load() -> ctypes.CDLL:
             f"{LIBRARY} is missing: build it with `python -c 'import __graft_entry__ as g; g.build()'` "
             "(there is no CPU or PyTorch fallback for the paged-attention kernels)")
     L = ctypes.CDLL(LIBRARY)
+    missing = [name for name in EXPORTS if not hasattr(L, name)]
+    if missing:
+        raise RuntimeError(f"{LIBRARY} lacks {', '.join(missing)}: it was built from older sources, rebuild the library")
     P = ctypes.c_void_p
     common = [P, P, P, P, P, P, ctypes.c_float, ctypes.c_int32]
     tail = [ctypes.POINTER(Shape), ctypes.POINTER(Options)]

@@ -113,6 +113,12 @@ struct CallStructs {
   const fa_paged_attention_options *options() const { return has_options ? &options_storage : nullptr; }
 };
 
+// The struct with workspace is told from the options alone by its size, 120 bytes.  Whoever appends fields to the
+// options moves its workspace fields, too: from then on 120 bytes are an earlier header's struct, to be read as such
+// and never as options that have grown to that size.
+static_assert(sizeof(fa_paged_attention_options) == 104 && sizeof(fa_paged_attention_options_workspace) == 120,
+              "read_options has to tell this header's options with workspace (120 bytes) from longer options");
+
 inline fa_status read_options(const fa_paged_attention_options *options, CallStructs *c) {
   c->has_options = options != nullptr;
   if (!options) return FA_OK;

@@ -55,7 +55,10 @@
  * takes every later field as zero, its default, so a caller built against an older revision of
  * this header keeps working when fields are appended; a size of 0, one that is not a multiple of
  * 4, one smaller than the fields a struct cannot do without (the shapes: all fields of revision 8;
- * the options: struct_size alone) or one larger than the library knows is FA_ERR_BAD_SHAPE.
+ * the options: struct_size alone) or one larger than the library knows is FA_ERR_BAD_SHAPE.  The options
+ * also come with workspace behind them (fa_paged_attention_options_workspace), told by the size of the whole.
+ * An entry point that a later header of the same revision adds is missing from an older library: a caller
+ * that loads the library at run time looks for it.
  */
 #ifndef FA_PAGED_ATTENTION_H_
 #define FA_PAGED_ATTENTION_H_
@@ -80,7 +83,8 @@ typedef enum fa_status {
   FA_ERR_BAD_SHAPE = 6,          /* non-positive sizes, misaligned strides or pointers */
   FA_ERR_RUNTIME = 7,            /* a HIP call failed; see fa_last_error() */
   FA_ERR_SCRATCH_TOO_SMALL = 8   /* fa_paged_attention_reduce_static_scratch: the call needs more
-                                    scratch than FA_STATIC_SCRATCH_BYTES */
+                                    scratch than FA_STATIC_SCRATCH_BYTES; single-pass entries: the
+                                    workspace is smaller than the call asks for */
 } fa_status;
 
 typedef enum fa_dtype { FA_DTYPE_F16 = 0, FA_DTYPE_BF16 = 1 } fa_dtype;

@@ -49,3 +49,17 @@ def test_timeline_percentiles_skip_empty_slots():
     dt = importlib.import_module("flash_attention_factory_amd.debug_timeline")
     assert dt._pct([1.0, float("nan"), 3.0], (0, 50, 100)) == [1.0, 2.0, 3.0]
     assert all(np.isnan(v) for v in dt._pct([float("nan")] * 3))
+
+
+def test_a_library_of_older_sources_says_so(tmp_path):
+    """FA_PAGED_ATTENTION_LIBRARY names a library of the same ABI revision without the latest entry point."""
+    from flash_attention_factory_amd import _cabi
+    source, library = tmp_path / "older.c", tmp_path / "older.so"
+    names = [n for n in _cabi.EXPORTS if n != "fa_paged_attention_loop_workspace_bytes"]
+    source.write_text("\n".join(f"int {n}(void) {{ return {_cabi.ABI_REVISION}; }}" for n in names))
+    subprocess.run(["gcc", "-shared", "-fPIC", str(source), "-o", str(library)], check=True)
+    env = dict(os.environ, FA_PAGED_ATTENTION_LIBRARY=str(library), PYTHONPATH=ROOT)
+    res = subprocess.run([sys.executable, "-c", "from flash_attention_factory_amd import _cabi; _cabi.load()"],
+                         env=env, capture_output=True, text=True)
+    assert res.returncode != 0 and "RuntimeError" in res.stderr and "rebuild the library" in res.stderr
+    assert "lacks fa_paged_attention_loop_workspace_bytes" in res.stderr
