@@ -38,25 +38,44 @@ constexpr int kSplitFullGpuBelowTokens = 2048;
 
 // Upper bound on the keys of a row as far as the host knows it; the scratch arrays hold
 // max_num_partitions * partition_size of them, and a call whose rows could exceed that is left to
-// the split kernels (which cut such a row to what the arrays hold).  With a local window (and one query token) the bound is on
-// the keys that it sees: the loop kernel starts a row at the first of them, where the split
-// kernels also take the segments that lie before the window, to store partials of nothing, and choose the
-// length of a segment by whole rows.  Measured on 40 batches of up to 128
-// sequences with windows of 511 and 1023: the loop kernel is faster in 33 (1.02 to 1.79 times: 62 sequences of up to
-// 5351 keys 49 -> 28 us, 127 of 9006 in a byte cache 60 -> 34, 8 of 9049 17 -> 10), slower by 3 to 6 % in four, with few
-// rows of 1024 keys.
-inline int64_t split_row_bound(const fa_paged_attention_shape &shape, int32_t partition_size, int32_t max_context_len,
-                               int64_t visible) {
+// the split kernels (which cut such a row to what the arrays hold).
+inline int64_t split_row_bound(const fa_paged_attention_shape &shape, int32_t partition_size, int32_t max_context_len) {
   const int64_t table = (int64_t)shape.max_blocks_per_seq * shape.block_size;
   const int64_t known = max_context_len > 0 ? std::min<int64_t>(max_context_len, table) : table;
   const int64_t scratch = (int64_t)shape.max_num_partitions * partition_size;
-  return known <= scratch ? std::min(known, visible) : INT64_MAX;
+  return known <= scratch ? known : INT64_MAX;
 }
 
 // rows: (sequence, kv head) items as the loop kernel deals them (pairs or teams of kv heads count once)
 inline bool split_call_runs_as_loop(int64_t row_bound, int64_t rows, int compute_units) {
   if (row_bound <= kSplitNeverBelowTokens) return true;
   return row_bound <= kSplitFullGpuBelowTokens && rows >= compute_units;
+}
+
+// The same with a local window (and one query token) that sees `visible` keys of rows of up to `row_bound`.  The loop
+// kernel starts a row at the first key that is seen, but a work-group streams the rest alone; the split kernels share a
+// row, but also take the segments that lie before the window, to store partials of nothing, and choose the length of a
+// segment by whole rows.  Measured on 851 batches with windows of 255 to 2047 keys (profiles/), in us split -> loop:
+//   up to 768 keys                   the loop kernel is faster in 296 of 302 (17.9 -> 8.8) and 4 % slower in two
+//   up to 1024                       few rows share the work better than one work-group each can do it: 16 rows of
+//                                    16-bit keys with heads of 128 (512 bytes a key) 15.8 -> 18.9, other caches 11.4 -> 12.7.
+//                                    The loop kernel wins from half a row per unit on (224 rows 43 -> 25), where the
+//                                    rows are long in sum (40 of 11554 keys 25.8 -> 19.6) and with fewer bytes a key also
+//                                    from 3 rows for 16 units or 4096 keys a row on (48 of 1803 14.6 -> 13.6, 4 of 12239 15.7 -> 14.3)
+//   up to 2048, a row for every unit the loop kernel is faster by 15 % in the mean (480 rows 53 -> 33), but with 512 bytes a key
+//                                    only where the window saves two thirds of a row or units have two rows (372 rows of 3002
+//                                    keys 33 -> 42)
+// rows: as split_call_runs_as_loop counts them; all_rows: (sequence, kv head) rows, pairs of kv heads once.
+constexpr int kSplitWindowNeverBelowTokens = 768;
+inline bool window_call_runs_as_loop(int64_t row_bound, int64_t visible, int64_t rows, int64_t all_rows, int key_bytes,
+                                     int compute_units) {
+  const bool heavy = key_bytes >= 512;
+  if (visible > kSplitNeverBelowTokens)
+    return visible <= kSplitFullGpuBelowTokens && rows >= compute_units &&
+           (!heavy || row_bound >= 3 * visible || rows >= 2 * compute_units);
+  if (visible <= kSplitWindowNeverBelowTokens || 2 * all_rows >= compute_units || all_rows * row_bound >= 1600LL * compute_units)
+    return true;
+  return !heavy && (row_bound >= 4096 || 16 * all_rows >= 3 * compute_units);
 }
 
 // (sequence, kv head) items of a batch as the persistent loop kernel deals them.
@@ -81,12 +100,17 @@ enum SplitForm { kSplitFormGrid = 0, kSplitFormSegment = 1, kSplitFormLoop = 2 }
 inline SplitForm split_form_of(const fa_paged_attention_shape &shape, const Resolved &r, bool kv8,
                                int32_t max_context_len, int compute_units) {
   if (r.schedule != FA_SCHEDULE_AUTO) return kSplitFormGrid;
-  const int64_t visible = (r.mask_flags & FA_MASK_WINDOW) && r.query_len == 1 ? (int64_t)r.window_left + 1 : INT64_MAX;
   const bool loop_persistent = loop_persistent_fits(shape) && shape.num_seqs <= kLoopPersistentMaxSeqs;
-  if (loop_persistent && r.segment_partitions == 0 && !r.keep_split &&
-      split_call_runs_as_loop(split_row_bound(shape, r.partition_size, max_context_len, visible), loop_rows_of(shape, r, kv8),
-                              compute_units))
-    return kSplitFormLoop;
+  if (loop_persistent && r.segment_partitions == 0 && !r.keep_split) {
+    const int64_t bound = split_row_bound(shape, r.partition_size, max_context_len), rows = loop_rows_of(shape, r, kv8);
+    if (split_call_runs_as_loop(bound, rows, compute_units)) return kSplitFormLoop;
+    const int64_t visible = (int64_t)r.window_left + 1;
+    const int key_bytes = (r.pair_heads ? 4 : 2) * shape.head_size * r.kv_elem_bytes;
+    if ((r.mask_flags & FA_MASK_WINDOW) && r.query_len == 1 && bound != INT64_MAX && visible < bound &&
+        window_call_runs_as_loop(bound, visible, rows, (int64_t)shape.num_seqs * shape.num_kv_heads / (r.pair_heads ? 2 : 1),
+                                 key_bytes, compute_units))
+      return kSplitFormLoop;
+  }
   const bool segment = (kv8 ? SegmentSplit<true>::use : SegmentSplit<false>::use) && shape.num_pool_blocks > 0 &&
                        r.partition_size < kSegmentMaxContext &&
                        (int64_t)shape.max_blocks_per_seq * shape.block_size < kSegmentMaxContext;

@@ -318,7 +318,9 @@ const char *fa_last_error(void);
  *   FA_SPLIT_FORM_LOOP     the rows are too short for splitting to pay -- at most 1024 keys, or at most
  *                          2048 with a (sequence, kv head) row for every compute unit, by what
  *                          max_context_len (0 = unknown), the block table's width and the scratch
- *                          arrays' capacity say: the call is the single-pass kernel, one launch; the
+ *                          arrays' capacity say -- or, with a local window and one query token, too few
+ *                          of a row's keys are seen (up to 768; up to 1024 or 2048 by the number and the
+ *                          length of the rows): the call is the single-pass kernel, one launch; the
  *                          scratch arrays stay untouched and the second kernel time is 0
  * compute_units > 0: of the GPU in question; the plan is then made without a device and work_groups
  * stays 0.  compute_units = 0: the current device's, and work_groups is filled in.  Launches nothing.
