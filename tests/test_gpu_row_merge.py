@@ -274,3 +274,25 @@ def test_a_full_gpu_leaves_rows_whole(oracle):
     torch.cuda.synchronize()
     for out in outs:
         _check(oracle, w, out)
+
+
+@pytest.mark.parametrize("fp8, d, lens, query_len, window", [
+    (E5M2, 128, [6000, 2561, 9001, 30], 1, None),
+    (E4M3, 128, [5121, 700, 2600], 2, None),
+    (E5M2, 128, [9000, 4000, 41], 1, 3000),
+    (E4M3, 64, [5200, 11000, 9], 1, None),
+    (E5M2, 64, [12001, 5121], 3, 7000),
+])
+@pytest.mark.parametrize("per_block", [False, True], ids=["head", "block"])
+def test_scales_of_byte_caches_in_cut_rows(oracle, per_block, fp8, d, lens, query_len, window):
+    w = _workload(lens, 2, 4, d, fp8, 16, sinks=True)
+    dev = torch.device("cuda:0")
+    g = torch.Generator().manual_seed(9)
+    shape = (w.key_cache.shape[0], 2) if per_block else (2,)
+    ks, vs = (torch.exp2(4.0 * torch.rand(shape, generator=g) - 2.0) for _ in range(2))  # 1/4 .. 4
+    query = torch.randn((len(lens), query_len, 8, d), generator=g).to(torch.float16) if query_len > 1 else w.query
+    assert _needs(w, query_len) > 0
+    kw = dict(window_left=window) if window else {}
+    out = _run(w, dev, query=query, k_scales=ks.to(dev), v_scales=vs.to(dev), **kw)
+    torch.cuda.synchronize()
+    _check(oracle, w, out, query=query, k_scales=ks, v_scales=vs, **kw)
