@@ -104,7 +104,8 @@ inline RowMergeSpace row_merge_space(const fa_paged_attention_shape &shape, cons
   return space;
 }
 
-// A number that no other launch of this process has, and hardly one of another: the clock, mixed.
+// A number that no other launch of this process has, and hardly one of another: SplitMix64 (Steele, Lea and Flood,
+// "Fast splittable pseudorandom number generators", 2014), begun at the clock.
 inline uint64_t next_merge_nonce() {
   static std::atomic<uint64_t> counter{(uint64_t)std::chrono::high_resolution_clock::now().time_since_epoch().count()};
   uint64_t nonce;
@@ -306,7 +307,6 @@ template <int HEAD_SIZE, typename QT, int KVF>
 inline fa_status launch_paged_attn_loop(void *out, const void *query, const void *key_cache,
                                         const void *value_cache, const int32_t *block_tables,
                                         const int32_t *context_lens, float scale,
-                                        int32_t /*max_context_len: validation only*/,
                                         const fa_paged_attention_shape &shape, const Resolved &r) {
   float total_us = 0.f;
   // most sequences one launch takes: what the persistent kernel ranks, or what the grid's third
@@ -325,7 +325,7 @@ inline fa_status launch_paged_attn_loop(void *out, const void *query, const void
       dot.schedule = FA_SCHEDULE_GRID_VALU;
   }
   if (dot.schedule != r.schedule) return launch_paged_attn_loop<HEAD_SIZE, QT, KVF>(out, query, key_cache, value_cache, block_tables,
-                                                                                    context_lens, scale, 0, shape, dot);
+                                                                                    context_lens, scale, shape, dot);
   const bool persistent_pieces = PersistentLoop<(KVF != kKv16)>::sub_batches && r.schedule == FA_SCHEDULE_AUTO &&
                                  loop_persistent_fits(shape) && shape.num_seqs > kLoopPersistentMaxSeqs;
   const int most = persistent_pieces ? kLoopPersistentMaxSeqs : kGridMaxSeqs;
@@ -382,15 +382,13 @@ inline fa_status dispatch_paged_attention_loop_any(void *out, const void *query,
   do {                                                                                            \
     if (!KV8)                                                                                     \
       return launch_paged_attn_loop<HS, QT, kKv16>(out, query, key_cache, value_cache,            \
-                                                   block_tables, context_lens, scale,             \
-                                                   max_context_len, *shape, r);                   \
+                                                   block_tables, context_lens, scale, *shape, r); \
     if (r.e4m3)                                                                                   \
       return launch_paged_attn_loop<HS, QT, kKvE4M3>(out, query, key_cache, value_cache,          \
-                                                     block_tables, context_lens, scale,           \
-                                                     max_context_len, *shape, r);                 \
+                                                     block_tables, context_lens, scale, *shape,   \
+                                                     r);                                          \
     return launch_paged_attn_loop<HS, QT, kKvE5M2>(out, query, key_cache, value_cache,            \
-                                                   block_tables, context_lens, scale,             \
-                                                   max_context_len, *shape, r);                   \
+                                                   block_tables, context_lens, scale, *shape, r); \
   } while (0)
   if (shape->head_size == 128) {
     if (bf16) FA_LOOP_CASE(128, BF16);

@@ -342,7 +342,7 @@ inline fa_status launch_paged_attn_v2(void *out, const void *query, const void *
   }
   if (form == kSplitFormLoop) {
     const fa_status st = launch_paged_attn_loop<HEAD_SIZE, QT, KVF>(out, query, key_cache, value_cache, block_tables,
-                                                                    context_lens, scale, max_context_len, shape, r);
+                                                                    context_lens, scale, shape, r);
     if (r.elapsed_us) r.elapsed_us[1] = 0.f;
     return st;
   }

@@ -5,11 +5,11 @@
 // A wavefront of a work-group owns one slice of the output of every piece its work-group takes (the
 // slice it merges out of LDS), and wavefront `tw` owns the same slice in every work-group.  So the
 // pieces of a row meet per slice: the wavefront writes its slice of the piece -- un-normalised sums with
-// their maximum and total, fp32 -- to the piece's slot of the workspace, counts itself in on the
-// (row, slice)'s arrival word, and the wavefront that completes the count reads the other pieces' slices
-// and stores the result.  Nobody waits for anybody: there is no spin and no order among work-groups that
-// the launch depends on.  Pieces are merged in the order of their keys whoever merges them, so the result
-// does not depend on the arrival order.
+// their maximum and total, fp32 -- to the piece's slot of the workspace, sets the flag of that slice of
+// the piece, and if it then finds the flags of all the row's pieces set, reads their slices, its own
+// among them, and stores the result.  Nobody waits for anybody: there is no spin and no order among
+// work-groups that the launch depends on.  Pieces are merged in the order of their keys whoever merges
+// them, so the result does not depend on the arrival order.
 //
 // How the last one is found: a wavefront sets the flag of its slice of its piece and then looks at the flags of
 // that slice of all the row's pieces, 64 at a time.  Whoever's flag is last in memory sees them all and merges; so

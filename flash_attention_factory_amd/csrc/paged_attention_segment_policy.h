@@ -24,8 +24,9 @@ constexpr int kSegmentMaxContext = 1 << 23;  // lengths are packed into 23 bits 
 #define FA_SEGMENT_MAX_PARTS 64
 #endif
 constexpr int kSegmentMaxPartitions = FA_SEGMENT_MAX_PARTS;
-// Launches that merge the pieces of a row themselves (paged_attention_row_merge.h): whole pieces that a launch may cut, over all its rows; what is left of a row behind its whole pieces is
-// one more.  The length of a piece grows until that holds.
+// Launches that merge the pieces of a row themselves (paged_attention_row_merge.h): whole pieces that a launch may
+// cut, over all its rows; what is left of a row behind its whole pieces is one more.  The length of a piece grows
+// until that holds.
 constexpr int kMergeWholePieces = 1024;
 // Rows of up to this many partitions stay whole.
 #ifndef FA_MERGE_WHOLE_PARTITIONS
