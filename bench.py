@@ -48,6 +48,9 @@ kv_cache_write  the step before the path (scatter of new K/V rows into the pools
              rounding): kernel time by the same events, read + written bytes against the
              HBM peak, and its CPU oracle on a bounded sample; random slots, and under
              kv_cache_write_prefill the slots a prefill writes (consecutive per sequence)
+
+stdout has one JSON line: the headline, its roofline, and configs_summary with the figures of every
+configuration.  All that is listed above goes to stderr, in one JSON line of its own.
 """
 from __future__ import annotations
 
@@ -723,9 +726,8 @@ def main():
                 print(child.stderr, file=sys.stderr)
                 return child.returncode
             line["large_batches"].append(json.loads(child.stdout.strip().splitlines()[-1]))
-    # Every configuration's figures once more, compact and LAST in the line (and inside `config`), so
-    # that whoever keeps only the head or the tail of it keeps them: microseconds per call, the dominant
-    # kernel's duration and fraction of the HBM peak, measured traffic.
+    # Every configuration's figures once more, compact: microseconds per call, the dominant kernel's duration
+    # and fraction of the HBM peak, measured traffic.
     summary = [_summary_of("config1: " + args.layout, main_res["us_per_call"], line["roofline"])]
     for r in others:
         summary.append(_summary_of(r["workload"], r["us_per_call"], r["roofline"], r.get("kernel_us_mean")))
@@ -736,9 +738,13 @@ def main():
         if r.get("form") is None or "forced" not in r["form"]:
             summary.append(dict(w=("recipe_e5m2_" if "E5M2" in r["workload"] else "recipe_fp16_") + r["kernel"],
                                 us=round(r["us_per_call"], 2), frac=round(r["hbm_frac"], 4), form=r.get("form")))
-    line["config"]["configs_summary"] = summary
+    # The one line on stdout is short, so that whoever keeps only the end of the output keeps all of it; what was
+    # measured beside the headline goes to stderr whole.
     line["configs_summary"] = summary
-    print(json.dumps(line), flush=True)
+    print(json.dumps(line), file=sys.stderr, flush=True)
+    head = ("metric", "value", "unit", "n_gpus", "steps", "warmup", "ms_per_step", "higher_is_better", "scaling",
+            "vs_baseline", "dtype", "data", "config", "roofline", "configs_summary")
+    print(json.dumps({k: line[k] for k in head}), flush=True)
     return 0
 
 
