@@ -21,6 +21,7 @@ from typing import List, Optional
 import torch
 
 from .. import _cabi
+from ._run import current_stream
 
 
 def run(key: torch.Tensor, value: torch.Tensor, key_cache: torch.Tensor, value_cache: torch.Tensor,
@@ -66,7 +67,7 @@ def run(key: torch.Tensor, value: torch.Tensor, key_cache: torch.Tensor, value_c
         if not fp8:
             raise _cabi.PagedAttentionError(_cabi.FA_ERR_UNSUPPORTED_DTYPE, "k_scales / v_scales belong to FP8 pools")
         _cabi.set_kv_scales(op, k_scales, v_scales, sh.num_kv_heads, sh.num_pool_blocks, key.device)
-    op.stream = torch.cuda.current_stream(key.device).cuda_stream
+    op.stream = current_stream(key.device)
     op.elapsed_us = ctypes.cast(elapsed, ctypes.POINTER(ctypes.c_float)) if timed else None
     with torch.cuda.device(key.device):
         _cabi.check(L.fa_kv_cache_write(key.data_ptr(), value.data_ptr(), key_cache.data_ptr(),

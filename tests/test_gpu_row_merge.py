@@ -296,3 +296,17 @@ def test_scales_of_byte_caches_in_cut_rows(oracle, per_block, fp8, d, lens, quer
     out = _run(w, dev, query=query, k_scales=ks.to(dev), v_scales=vs.to(dev), **kw)
     torch.cuda.synchronize()
     _check(oracle, w, out, query=query, k_scales=ks, v_scales=vs, **kw)
+
+
+def test_calls_go_to_the_current_stream():
+    from flash_attention_factory_amd.lib import _run as body
+    dev = torch.device("cuda:0")
+    w = _workload([6000, 40], 1, 2, 128)
+    wd = w.to(dev)
+    for stream in (torch.cuda.current_stream(), torch.cuda.Stream(), torch.cuda.Stream()):
+        with torch.cuda.stream(stream):
+            assert body.current_stream(dev) == stream.cuda_stream == torch.cuda.current_stream().cuda_stream
+            out = _run(wd, dev)
+            again = torch.empty_like(out).copy_(out)  # ordered behind the call on its stream only
+        stream.synchronize()
+        assert torch.equal(out, again) and torch.isfinite(again.float()).all()
