@@ -273,9 +273,9 @@ def load() -> ctypes.CDLL:
     if L.fa_paged_attention_abi_version() != ABI_REVISION:
         raise RuntimeError(f"{LIBRARY} has ABI revision {L.fa_paged_attention_abi_version()}, this binding is "
                            f"written for {ABI_REVISION}: rebuild the library")
-    _lib = L
     for then in _when_loaded:
         then(L)
+    _lib = L
     return L
 
 

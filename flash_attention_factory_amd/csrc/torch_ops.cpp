@@ -297,10 +297,11 @@ void cache_write(const c10::OperatorHandle &op, torch::jit::Stack *stack) {
 
 }  // namespace
 
-// table: addresses of the entry points in the order of Entries.
-extern "C" __attribute__((visibility("default"))) void fa_torch_ops_bind(void *const *table, size_t count) {
-  TORCH_CHECK(count * sizeof(void *) == sizeof(Entries), "fa_torch_ops_bind: ", count, " entry points");
+// table: addresses of the entry points in the order of Entries; 0: not as many as this library was built for.
+extern "C" __attribute__((visibility("default"))) int fa_torch_ops_bind(void *const *table, size_t count) {
+  if (count * sizeof(void *) != sizeof(Entries)) return 0;
   memcpy(&entries, table, sizeof(Entries));
+  return 1;
 }
 
 extern "C" __attribute__((visibility("default"))) void fa_torch_ops_capacity_warned() { capacity_warned.store(true); }

@@ -163,12 +163,16 @@ def _bind(L: ctypes.CDLL) -> None:
                L.fa_paged_attention_fp8_reduce, L.fa_kv_cache_write, L.fa_paged_attention_loop_workspace_bytes)
     table = (ctypes.c_void_p * len(entries))(*(ctypes.cast(e, ctypes.c_void_p).value for e in entries))
     global _native
-    _native = ctypes.CDLL(_build.TORCH_OPS_LIBRARY)
-    _native.fa_torch_ops_bind.argtypes, _native.fa_torch_ops_bind.restype = [ctypes.c_void_p, ctypes.c_size_t], None
-    _native.fa_torch_ops_capacity_warned.argtypes, _native.fa_torch_ops_capacity_warned.restype = [], None
-    _native.fa_torch_ops_bind(table, len(entries))
+    native = ctypes.CDLL(_build.TORCH_OPS_LIBRARY)
+    exported = all(hasattr(native, name) for name in ("fa_torch_ops_bind", "fa_torch_ops_capacity_warned"))
+    if exported:
+        native.fa_torch_ops_bind.argtypes, native.fa_torch_ops_bind.restype = [ctypes.c_void_p, ctypes.c_size_t], ctypes.c_int
+        native.fa_torch_ops_capacity_warned.argtypes, native.fa_torch_ops_capacity_warned.restype = [], None
+    if not exported or not native.fa_torch_ops_bind(table, len(entries)):
+        raise RuntimeError(f"{_build.TORCH_OPS_LIBRARY} was built from other sources than this module: rebuild the library")
+    _native = native
     if _warned_capacity:
-        _native.fa_torch_ops_capacity_warned()
+        native.fa_torch_ops_capacity_warned()
 
 
 def _load_native():

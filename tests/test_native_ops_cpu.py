@@ -57,3 +57,19 @@ def test_schemas_without_the_library(tmp_path):
     assert res.returncode == 0, res.stderr
     here = [f"{op._schema} {sorted(map(str, op.tags))}" for op in (getattr(torch.ops.fa_amd, n).default for n in torch_ops._NAMES)]
     assert res.stdout.splitlines() == here
+
+
+def test_operators_of_other_sources_say_so(tmp_path):
+    """A library that registers operators but does not take the entry points: no call, on whatever path, goes on
+    without them."""
+    source, library = tmp_path / "other.c", tmp_path / "other.so"
+    source.write_text("int nothing(void) { return 0; }")
+    subprocess.run(["gcc", "-shared", "-fPIC", str(source), "-o", str(library)], check=True)
+    code = ("from flash_attention_factory_amd import _build, _cabi; _build.TORCH_OPS_LIBRARY = %r\n"
+            "import flash_attention_factory_amd.torch_ops as ops\n" % str(library))
+    # (the stub registers nothing, so the schemas are missing; what matters is that loading the C ABI raises)
+    code = code.replace("import flash", "import torch; [torch.library.define('fa_amd::' + n, '(Tensor x) -> ()') for n in "
+                        "('paged_attention_loop', 'paged_attention_fp8_loop', 'paged_attention_reduce', "
+                        "'paged_attention_fp8_reduce', 'kv_cache_write')]\nimport flash", 1)
+    res = _in_a_process(code + "_cabi.load()")
+    assert res.returncode != 0 and "built from other sources" in res.stderr, res.stderr
