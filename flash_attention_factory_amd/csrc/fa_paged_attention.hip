@@ -232,7 +232,8 @@ FA_EXPORT int32_t fa_paged_attention_reduce_plan(const fa_paged_attention_shape 
 
 FA_EXPORT int32_t fa_paged_attention_kernel_status(void *stream, int32_t clear) {
   fa::error_buffer()[0] = 0;
-  return fa::read_kernel_status(reinterpret_cast<hipStream_t>(stream), clear != 0, 0);
+  FA_HIP_CHECK(hipStreamSynchronize(reinterpret_cast<hipStream_t>(stream)));
+  return fa::read_kernel_status(clear != 0, 0);
 }
 
 #ifdef FA_TIMELINE

@@ -56,26 +56,41 @@ inline fa_status fail(fa_status code, const char *fmt, ...) {
 
 // The status word of the persistent kernels: a wavefront that exhausts its spin limit while it
 // waits for the other wavefronts of its work-group stores kStatusSpinLimit here and goes on (so
-// the grid drains) with a result that is wrong.  One word per GPU, in device memory; as with any
-// __device__ variable the name is only a handle on the host, the address on the current device
-// comes from hipGetSymbolAddress, once per device.
-static __device__ int32_t kernel_status_word;
-
-inline fa_status kernel_status_of_current_device(int32_t **word) {
-  constexpr int kMaxDevices = 64;
+// the grid drains) with a result that is wrong.  One word per GPU, in pinned host memory: it is written
+// hardly ever and read after every blocking call, whose host side then looks at its own memory where it had
+// to copy a word from the device and wait for the copy (the reference's measuring loop, 35 us of kernel: 82 -> 66 us
+// a call).  The words live as long as the process.  Allocated at the first call; a stream that is being captured
+// does not mind (hipThreadExchangeStreamCaptureMode).
+inline fa_status kernel_status_of_current_device(int32_t **word, int32_t **device_word = nullptr) {
+  constexpr int kMaxDevices = 64, kStride = 64 / sizeof(int32_t);  // a cache line each
   static std::mutex mutex;
-  static int32_t *address[kMaxDevices];  // nullptr until the device's first launch
+  static int32_t *block = nullptr;
+  static int32_t *address[kMaxDevices];  // as the device sees it; nullptr until the device's first launch
   int dev = 0;
   FA_HIP_CHECK(hipGetDevice(&dev));
   if (dev < 0 || dev >= kMaxDevices)
     return fail(FA_ERR_RUNTIME, "device %d is beyond the %d devices this library serves", dev, kMaxDevices);
   std::lock_guard<std::mutex> guard(mutex);
   if (address[dev] == nullptr) {
+    hipStreamCaptureMode mode = hipStreamCaptureModeRelaxed;
+    FA_HIP_CHECK(hipThreadExchangeStreamCaptureMode(&mode));
+    hipError_t e = hipSuccess;
+    if (block == nullptr) {
+      void *b = nullptr;
+      e = hipHostMalloc(&b, kMaxDevices * kStride * sizeof(int32_t), hipHostMallocPortable | hipHostMallocMapped | hipHostMallocCoherent);
+      if (e == hipSuccess) {
+        memset(b, 0, kMaxDevices * kStride * sizeof(int32_t));
+        block = static_cast<int32_t *>(b);
+      }
+    }
     void *a = nullptr;
-    FA_HIP_CHECK(hipGetSymbolAddress(&a, HIP_SYMBOL(kernel_status_word)));
+    if (e == hipSuccess) e = hipHostGetDevicePointer(&a, block + dev * kStride, 0);
+    (void)hipThreadExchangeStreamCaptureMode(&mode);
+    FA_HIP_CHECK(e);
     address[dev] = static_cast<int32_t *>(a);
   }
-  *word = address[dev];
+  if (word) *word = block + dev * kStride;
+  if (device_word) *device_word = address[dev];
   return FA_OK;
 }
 
@@ -174,7 +189,7 @@ struct Resolved {
   bool keep_split;   // a reduce entry runs its two kernels however short the rows
   int32_t segment_partitions;  // > 0: partitions per partial of the segment form, fixed by the caller; -1: even shares
   bool pair_heads;   // two adjacent kv heads with 64-byte token rows run as one (WaveAttn::kPairable)
-  int32_t *status;   // status word of the current device (nullptr with validate_only)
+  int32_t *status;   // status word of the current device, as the device sees it (nullptr with validate_only)
   int32_t spin_limit;
   hipStream_t stream;
   float *elapsed_us;
@@ -309,29 +324,19 @@ inline fa_status validate_and_resolve(const void *out, const void *query, const 
   r->workspace_bytes = 0;
   r->status = nullptr;
   r->spin_limit = spin_limit_of(o);
-  if (!r->validate_only) return kernel_status_of_current_device(&r->status);
+  if (!r->validate_only) return kernel_status_of_current_device(nullptr, &r->status);
   return FA_OK;
 }
 
-// Did a kernel of the current GPU give up a wait since the status word was last cleared?  Waits for
-// `stream`, reads the word, clears it on request, and turns a set word into FA_ERR_RUNTIME.
-inline fa_status read_kernel_status(hipStream_t stream, bool clear, int32_t spin_limit) {
+// Did a kernel of the current GPU that has ended give up a wait since the status word was last cleared?  Reads the
+// word, clears it on request, and turns a set word into FA_ERR_RUNTIME.
+inline fa_status read_kernel_status(bool clear, int32_t spin_limit) {
   int32_t *word = nullptr;
   const fa_status st = kernel_status_of_current_device(&word);
   if (st != FA_OK) return st;
-  // read through one pinned word per thread (a copy into pageable memory costs ten times as much);
-  // allocated on the first look, like the timing events
-  static thread_local int32_t *pinned = nullptr;
-  if (pinned == nullptr) FA_HIP_CHECK(hipHostMalloc(reinterpret_cast<void **>(&pinned), sizeof(int32_t), hipHostMallocDefault));
-  FA_HIP_CHECK(hipMemcpyAsync(pinned, word, sizeof(int32_t), hipMemcpyDeviceToHost, stream));
-  FA_HIP_CHECK(hipStreamSynchronize(stream));
-  const int32_t seen = *pinned;
+  const int32_t seen = clear && __atomic_load_n(word, __ATOMIC_ACQUIRE) != 0 ? __atomic_exchange_n(word, 0, __ATOMIC_ACQ_REL)
+                                                                            : __atomic_load_n(word, __ATOMIC_ACQUIRE);
   if (seen == 0) return FA_OK;
-  if (clear) {
-    const int32_t zero = 0;
-    FA_HIP_CHECK(hipMemcpyAsync(word, &zero, sizeof(zero), hipMemcpyHostToDevice, stream));
-    FA_HIP_CHECK(hipStreamSynchronize(stream));
-  }
   if (spin_limit > 0)
     return fail(FA_ERR_RUNTIME, "a wavefront gave up waiting for the other wavefronts of its work-group (spin limit %d, "
                                 "status %d): the output of this or an earlier call on this GPU is not valid",
@@ -340,12 +345,12 @@ inline fa_status read_kernel_status(hipStream_t stream, bool clear, int32_t spin
                               "output of this or an earlier call on this GPU is not valid", seen);
 }
 
-// After a timed call (which has synchronised anyway): report and clear the status word.
+// After a timed call (which has waited for its last kernel): report and clear the status word.
 // Asynchronous calls do not look: the word stays set until the next timed call on the device, or
 // fa_paged_attention_kernel_status, reports it.
 inline fa_status report_kernel_status(const Resolved &r) {
   if (!r.elapsed_us || !r.status) return FA_OK;
-  return read_kernel_status(r.stream, true, r.spin_limit);
+  return read_kernel_status(true, r.spin_limit);
 }
 
 inline PagedAttnParams make_params(void *out, float *exp_sums, float *max_logits, const void *query,

@@ -258,7 +258,8 @@ inline fa_status launch_paged_attn_v2_batch(void *out, const void *query, const 
                             Pipeline<KV8>::tiles_per_chunk>,
           grid, dim3(NW * 64), 0, p));
     }
-    if (r.elapsed_us) FA_HIP_CHECK(timer.accumulate(0, &attention_us));
+    // (the last launch's time is asked for behind the reduce launch, so that the two kernels run on end)
+    if (r.elapsed_us && q0 + per_launch < r.query_len) FA_HIP_CHECK(timer.accumulate(0, &attention_us));
   }
 
   // kernel 2: one wavefront per (head, sequence)
@@ -286,8 +287,9 @@ inline fa_status launch_paged_attn_v2_batch(void *out, const void *query, const 
     else FA_HIP_CHECK(timer.launch(paged_attn_reduce_kernel<OUT_D, QT, 4, false>, rgrid, dim3(256), 1, rp));
   }
   if (r.elapsed_us) {
-    us_out[0] += attention_us;
     FA_HIP_CHECK(timer.accumulate(1, &us_out[1]));
+    FA_HIP_CHECK(timer.accumulate(0, &attention_us));
+    us_out[0] += attention_us;
   }
   return FA_OK;
 }

@@ -145,7 +145,7 @@ __device__ __forceinline__ void walk_loop_items(const PagedAttnParams &p, LoopIt
     }
     // Gave up: what follows merges states that are not all there, so the result is wrong; say so in
     // the status word (one lane, a plain vector store) and carry on, so that the grid still drains.
-    if (!arrived && lane == 0) __hip_atomic_store(p.status, kStatusSpinLimit, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    if (!arrived && lane == 0) __hip_atomic_store(p.status, kStatusSpinLimit, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
     __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup");
     const int w0 = team * NT;  // the team's wavefronts: w0 .. w0 + NT - 1
     float M = -INFINITY;

@@ -176,7 +176,7 @@ paged_attn_loop_two_tile_kernel(const PagedAttnParams p) {
       }
       __builtin_amdgcn_s_sleep(1);
     }
-    if (!arrived && lane == 0) __hip_atomic_store(p.status, kStatusSpinLimit, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    if (!arrived && lane == 0) __hip_atomic_store(p.status, kStatusSpinLimit, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
     __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup");
     bool whole = false;
     if constexpr (PART) whole = p.final_out != nullptr && it.part0 == 0 && it.tok_end >= it.ctx;

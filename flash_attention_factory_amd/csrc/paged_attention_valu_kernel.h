@@ -337,7 +337,7 @@ paged_attn_valu_persistent_kernel(const PagedAttnParams p) {
       __builtin_amdgcn_s_sleep(1);
     }
     // gave up: the result is wrong; say so in the status word and carry on, so that the grid drains
-    if (!arrived && lane == 0) __hip_atomic_store(p.status, kStatusSpinLimit, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    if (!arrived && lane == 0) __hip_atomic_store(p.status, kStatusSpinLimit, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
     __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup");
     if (lane < SL) {
       const int d = wave * SL + lane;

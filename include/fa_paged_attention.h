@@ -298,9 +298,9 @@ int32_t fa_paged_attention_fp8_reduce(void *out, const void *query, const void *
                                       const fa_paged_attention_options *options);
 
 /* Everything the library sets up once per GPU, done now on the current device instead of inside the
- * first call there: the device addresses of its two static device arrays (the status word of
- * fa_paged_attention_kernel_status and the scratch of fa_paged_attention_reduce_static_scratch, both
- * through hipGetSymbolAddress, which may load the code object) and the device's compute-unit count.
+ * first call there: the status word of fa_paged_attention_kernel_status (pinned host memory), the device
+ * address of the scratch of fa_paged_attention_reduce_static_scratch (through hipGetSymbolAddress, which
+ * may load the code object) and the device's compute-unit count.
  * A caller that records calls into a HIP graph calls this first, outside the capture, and makes one
  * eager call of each shape it will record (the first launch of a kernel instance asks the occupancy
  * calculator how many of its work-groups stay resident).  No counterpart upstream. */
