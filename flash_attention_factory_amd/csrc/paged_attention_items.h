@@ -175,6 +175,8 @@ struct SegmentItems {
   // batch, the number of work-groups and the compute units they share (partitions_per_segment).
   // heads_per_item: adjacent kv heads that one work-group takes together (its wavefronts in teams);
   // item_row_bytes: bytes of one token's K row (as of its V row) of an item
+  // TWO_TILES: the kernel holds two column tiles
+  template <bool TWO_TILES = false>
   __device__ __forceinline__ void build(const PagedAttnParams &p, int lane_, int groups, int heads_per_item,
                                         int item_row_bytes) {
     static_assert(!ROW_MERGE);
@@ -188,10 +190,14 @@ struct SegmentItems {
       build_even_shares(groups, p.compute_units);
       return;
     }
-    m = p.segment_force > 0 ? min(p.segment_force, kSegmentMaxPartitions)
-                            : partitions_per_segment<NQ>(ctxv, parts, total_parts, S, p.partition_size, Hk, groups,
-                                                         p.compute_units, p.kv_rows_apart != 0,
-                                                         2 * p.partition_size * item_row_bytes);
+    m = p.segment_force > 0 ? min(p.segment_force, kSegmentMaxPartitions) : 0;
+    if constexpr (TWO_TILES) {
+      if (m == 0)
+        m = two_tile_partitions_per_segment<NQ>(ctxv, parts, total_parts, S, p.partition_size, Hk, min(groups, p.compute_units));
+    }
+    if (m == 0)
+      m = partitions_per_segment<NQ>(ctxv, parts, total_parts, S, p.partition_size, Hk, groups, p.compute_units,
+                                     p.kv_rows_apart != 0, 2 * p.partition_size * item_row_bytes);
     cut_rows();
   }
   // ROW_MERGE: rows as cut_pays saw them

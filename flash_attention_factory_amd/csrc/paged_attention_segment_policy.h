@@ -249,6 +249,39 @@ __device__ __forceinline__ int partitions_per_segment(const int (&ctxv)[NQ], con
   return before > 0 ? before : m;
 }
 
+// The same for the kernels of two column tiles, one work-group per compute unit (paged_attention_loop_two_tile_kernel.h):
+// what a partial of 32 columns costs (16 KiB through tmp_out with head size 128, a merge without loads in flight)
+// makes cutting dear.  0: no opinion, partitions_per_segment decides.  Every length was forced in turn on 44 batches (us, with
+// the length that partitions_per_segment takes -> with this one):
+//   rows stay whole where the longest is no more than 4/3 of a unit's mean load: 48 rows of 257-6000 keys, 8 kv heads, byte
+//     cache 78.0 -> 73.0, head size 64 65.2 -> 59.5, 16-bit cache 115.7 -> 115.8; 100 of 400-4000, 4 kv heads 64.3 -> 60.7, 91.4 ->
+//     87.4; 24 of 1000-5000, 16 kv heads 75.5 -> 72.9, 109.3 -> 107.6
+//   a row per unit at most, longer ones among them: the shortest segment of which there are no more than units, if that is
+//     up to 4/3 of the load as well (3 rows of 1000-5000, 32 kv heads, head size 64 33.3 -> 28.0; 64 of 200-8000, 2 kv heads, head
+//     size 64 about 38 -> 34.5)
+template <int NQ>
+__device__ __forceinline__ int two_tile_partitions_per_segment(const int (&ctxv)[NQ], const int (&parts)[NQ], int total_partitions,
+                                                               int S, int partition_size, int num_kv_heads, int units) {
+  int longest = 0, live = 0;
+#pragma unroll
+  for (int j = 0; j < NQ; ++j) {
+    longest = max(longest, parts[j]);
+    if (j * 64 < S) live += __builtin_popcountll(__ballot(parts[j] > 0));
+  }
+  longest = __builtin_amdgcn_readfirstlane(__reduce_max_sync(~0ull, longest));
+  const long long items = (long long)total_partitions * num_kv_heads;
+  if (longest <= kSegmentMaxPartitions && 3LL * longest * units <= 4 * items) return max(longest, 1);
+  if ((long long)live * num_kv_heads > units) return 0;
+  const int mean = (int)((items + units - 1) / units);
+#pragma nounroll
+  for (int m = max(mean, 1); m <= kSegmentMaxPartitions && (m == mean || 3LL * m * units <= 4 * items); ++m) {
+    int whole, all;
+    count_segments<NQ>(ctxv, parts, S, partition_size, m, whole, all);
+    if ((long long)all * num_kv_heads <= units) return m;
+  }
+  return 0;
+}
+
 // Whether a launch that merges the pieces of a row itself cuts its rows at all.  longest, total: partitions of
 // the longest row, and of all sequences; live: sequences that have any; units: compute units of the GPU.  Uncut,
 // the launch lasts as long as its longest row takes one work-group, or as long as the memory takes for all rows;
