@@ -278,10 +278,16 @@ inline fa_status launch_paged_attn_v2_batch(void *out, const void *query, const 
   rp.query_len = r.query_len;
   rp.segment_groups = segment_groups;
   const dim3 rgrid((unsigned)((int64_t)shape.num_heads * shape.num_seqs * r.query_len));
-  const bool one_wave = (int64_t)shape.num_heads * shape.num_seqs * r.query_len >= kReduceSingleWaveMinPairs;
+  const int64_t pairs = (int64_t)shape.num_heads * shape.num_seqs * r.query_len;
+  const bool one_wave = pairs >= kReduceSingleWaveMinPairs;
   if (segment_groups > 0) {
-    if (one_wave) FA_HIP_CHECK(timer.launch(paged_attn_reduce_kernel<OUT_D, QT, 1, true>, rgrid, dim3(64), 1, rp));
-    else FA_HIP_CHECK(timer.launch(paged_attn_reduce_kernel<OUT_D, QT, 4, true>, rgrid, dim3(256), 1, rp));
+    if (pairs <= kReduceAheadMaxPairs && shape.max_num_partitions <= kReduceAheadMaxPartitions)
+      FA_HIP_CHECK(timer.launch(paged_attn_reduce_kernel<OUT_D, QT, kReduceAheadWaves, true>, rgrid, dim3(kReduceAheadWaves * 64), 1, rp));
+    else if (one_wave)
+      FA_HIP_CHECK(timer.launch(paged_attn_reduce_kernel<OUT_D, QT, 1, true>, dim3((unsigned)((pairs + kReducePairs - 1) / kReducePairs)),
+                                dim3(kReducePairs * 64), 1, rp));
+    else
+      FA_HIP_CHECK(timer.launch(paged_attn_reduce_kernel<OUT_D, QT, 4, true>, rgrid, dim3(256), 1, rp));
   } else {
     if (one_wave) FA_HIP_CHECK(timer.launch(paged_attn_reduce_kernel<OUT_D, QT, 1, false>, rgrid, dim3(64), 1, rp));
     else FA_HIP_CHECK(timer.launch(paged_attn_reduce_kernel<OUT_D, QT, 4, false>, rgrid, dim3(256), 1, rp));

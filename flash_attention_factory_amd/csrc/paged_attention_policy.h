@@ -162,5 +162,23 @@ struct PersistentLoop {
 #define FA_REDUCE_1W_MIN_PAIRS 4096
 #endif
 constexpr int kReduceSingleWaveMinPairs = FA_REDUCE_1W_MIN_PAIRS;
+// After the segment kernel also:
+//  * sixteen for up to kReduceAheadMaxPairs pairs of up to kReduceAheadMaxPartitions slots: the launch lasts as long as its trips
+//    to memory follow one another, and sixteen wavefronts ask for a pair's first 64 rows of tmp_out together with the
+//    scalars that say which of them count (us a call, four wavefronts -> sixteen: 32 pairs of 59 slots 29.4 -> 25.6, 64 of 32
+//    25.4 -> 24.0, 128 of 16 24.8 -> 24.1; 256 of 8 24.2 both, 256 of 32 67.0 -> 67.2, 512 of 16 68.0 -> 69.1, and
+//    32 of 235, most of them beyond the first 64, 25.0 -> 26.0)
+//  * where one wavefront takes a pair, kReducePairs of them in a work-group: thousands of work-groups of one wavefront, most of
+//    which find nothing to do, are launched more slowly than they run (12288 pairs 75.2 -> 74.2; 4, 8 and 16 alike)
+#ifndef FA_REDUCE_AHEAD_MAX_PAIRS
+#define FA_REDUCE_AHEAD_MAX_PAIRS 128
+#endif
+constexpr int kReduceAheadMaxPairs = FA_REDUCE_AHEAD_MAX_PAIRS;
+constexpr int kReduceAheadMaxPartitions = 128;
+constexpr int kReduceAheadWaves = 16;
+#ifndef FA_REDUCE_PAIRS
+#define FA_REDUCE_PAIRS 8
+#endif
+constexpr int kReducePairs = FA_REDUCE_PAIRS;
 
 }  // namespace fa

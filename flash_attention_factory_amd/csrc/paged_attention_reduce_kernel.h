@@ -9,7 +9,7 @@
 // of the first, the others hold a mark (paged_attention_segment_policy.h); and a row of a single
 // partial is left alone: the attention kernel has stored it into `out` already.
 //
-// One work-group of one or four wavefronts per (sequence, head).  The kernel is a chain
+// One work-group of four or sixteen wavefronts per (sequence, head), or one wavefront of a work-group.  The kernel is a chain
 // of dependent memory round trips, so it is built to have as few of them as possible:
 // wavefront w owns partitions w, w+NW, w+2NW, ... and requests up to 16 (4) of their tmp_out
 // rows (one coalesced 512-byte row per load) together with the partition scalars, before
@@ -49,6 +49,18 @@ struct ReduceParams {
 // register set then lets twice as many work-groups stay resident.
 template <bool SEGMENTS>
 constexpr int reduce_rows_in_flight() { return SEGMENTS ? FA_REDUCE_SEGMENT_ROWS : 16; }
+
+// A lane's EPL elements of a row of tmp_out (rows are a multiple of 8 bytes from an array aligned to 16).
+template <int EPL>
+__device__ __forceinline__ void load_row(float (&v)[EPL], const float *at) {
+  if constexpr (EPL == 2) {
+    const u32x2 w = *reinterpret_cast<const u32x2 *>(at);
+    v[0] = __uint_as_float(w[0]);
+    v[1] = __uint_as_float(w[1]);
+  } else {
+    v[0] = *at;
+  }
+}
 
 // kReduceWaves wavefronts per (sequence, head): 4 when there are few (sequence, head)
 // pairs -- the launch is then short of parallelism and each pair's rows should be in
@@ -159,11 +171,19 @@ __device__ __forceinline__ void reduce_marked_partials(const ReduceParams &p) {
   constexpr int EPL = D / 64;  // output elements per lane (2 or 1)
   constexpr int R = reduce_rows_in_flight<SEGMENTS>();
   const int lane = threadIdx.x & 63;
-  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-  // one work-group per (row, head), heads fastest; a row of out and of the scratch arrays is a
-  // sequence, or a (sequence, query token) pair
-  const int seq = blockIdx.x / p.num_heads;
-  const int head = blockIdx.x - seq * p.num_heads;
+  int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  // one work-group per (row, head), heads fastest, or one wavefront of a work-group of kReducePairs; a row of out and
+  // of the scratch arrays is a sequence, or a (sequence, query token) pair
+  uint32_t nth_pair = blockIdx.x;
+  if constexpr (kReduceWaves == 1) {
+    nth_pair = nth_pair * kReducePairs + wave;
+    wave = 0;
+  }
+  const int seq = nth_pair / (uint32_t)p.num_heads;
+  if constexpr (kReduceWaves == 1) {
+    if (seq >= p.num_seqs * p.query_len) return;
+  }
+  const int head = nth_pair - seq * p.num_heads;
   const int64_t base = ((int64_t)seq * p.num_heads + head) * p.max_num_partitions;
   const float *ml = p.max_logits + base;
   const float *es = p.exp_sums + base;
@@ -172,8 +192,17 @@ __device__ __forceinline__ void reduce_marked_partials(const ReduceParams &p) {
   // the row turns out to have that many partitions, so that one wait covers both (slots past the
   // live ones are read and dropped: they lie inside the row).
   const int first_slots = min(p.max_num_partitions, 64);
-  const float ml_first = lane < first_slots ? ml[lane] : -INFINITY;
-  const float es_first = lane < first_slots ? es[lane] : 0.f;
+  // kAhead: so are the rows of tmp_out of those slots, whether or not they hold a partial
+  constexpr bool kAhead = kReduceWaves == kReduceAheadWaves;
+  constexpr int RA = kAhead ? 64 / kReduceWaves : 1;
+  float ahead[RA][EPL];
+  if constexpr (kAhead) {
+#pragma unroll
+    for (int u = 0; u < RA; ++u) load_row<EPL>(ahead[u], tmp + (int64_t)min(wave + kReduceWaves * u, first_slots - 1) * D);
+  }
+  const int my_slot = min(lane, first_slots - 1);  // (no branch around a load; a lane past the last slot drops what it reads)
+  const float ml_first = ml[my_slot];
+  const float es_first = es[my_slot];
   const int ctx = min(p.context_lens[p.query_len > 1 ? seq / p.query_len : seq], p.max_context);
   if (ctx <= 0) return;
   int np = (ctx + p.partition_size - 1) / p.partition_size;
@@ -218,6 +247,20 @@ __device__ __forceinline__ void reduce_marked_partials(const ReduceParams &p) {
     const float w_lane = there ? e_q * __expf(m_q - M) : 0.f;
     W += w_lane;
     unsigned long long todo = __ballot(there);
+    if constexpr (kAhead) {
+      if (g0 == 0) {
+#pragma unroll
+        for (int u = 0; u < RA; ++u) {
+          const int q = wave + kReduceWaves * u;
+          if (todo >> q & 1) {  // wave-uniform; a row without a partial may hold anything
+            const float w = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(w_lane), q));
+#pragma unroll
+            for (int e = 0; e < EPL; ++e) acc[e] += w * ahead[u][e];
+          }
+        }
+        continue;
+      }
+    }
     while (todo) {  // wave-uniform: R rows of tmp_out per wavefront in flight at a time
       int slot[R];
       float v[R][EPL];
@@ -229,12 +272,12 @@ __device__ __forceinline__ void reduce_marked_partials(const ReduceParams &p) {
           todo &= todo - 1;
           if ((nth++ % kReduceWaves) == wave) slot[u] = q;
         }
-#pragma unroll
-        for (int e = 0; e < EPL; ++e) v[u][e] = slot[u] >= 0 ? tmp[(int64_t)(g0 + slot[u]) * D + e] : 0.f;
+        if (slot[u] >= 0) load_row<EPL>(v[u], tmp + (int64_t)(g0 + slot[u]) * D);  // wave-uniform
       }
 #pragma unroll
       for (int u = 0; u < R; ++u) {
-        const float w = slot[u] >= 0 ? __int_as_float(__builtin_amdgcn_readlane(__float_as_int(w_lane), __builtin_amdgcn_readfirstlane(slot[u]))) : 0.f;
+        if (slot[u] < 0) continue;
+        const float w = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(w_lane), __builtin_amdgcn_readfirstlane(slot[u])));
 #pragma unroll
         for (int e = 0; e < EPL; ++e) acc[e] += w * v[u][e];
       }
@@ -271,8 +314,11 @@ __device__ __forceinline__ void reduce_marked_partials(const ReduceParams &p) {
   }
 }
 
+template <int kReduceWaves, bool SEGMENTS>
+constexpr int reduce_threads() { return 64 * (SEGMENTS && kReduceWaves == 1 ? kReducePairs : kReduceWaves); }
+
 template <int D, typename QT, int kReduceWaves, bool SEGMENTS = false>
-__global__ void __launch_bounds__(kReduceWaves * 64) paged_attn_reduce_kernel(const ReduceParams p) {
+__global__ void __launch_bounds__((reduce_threads<kReduceWaves, SEGMENTS>())) paged_attn_reduce_kernel(const ReduceParams p) {
   if constexpr (SEGMENTS) reduce_marked_partials<D, QT, kReduceWaves>(p);
   else reduce_every_partition<D, QT, kReduceWaves>(p);
 }
