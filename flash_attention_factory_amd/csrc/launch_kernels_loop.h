@@ -43,7 +43,7 @@ namespace fa {
 // A launch of few rows leaves most compute units idle, or waits for its longest row.  Given workspace, it cuts its
 // rows (paged_attention_row_merge.h) where that pays.  The host knows the number of rows and a bound on their length;
 // whether the rows at hand are worth it the device decides (cut_pays).  Back to back, us, whole -> cut:
-//   8 rows of 30011 keys 402 -> 32 (the split path's two kernels: 37), 24 rows of 900-4096 keys 49 -> 18, 110 rows
+//   8 rows of 30011 keys 402 -> 29 (the split path's two kernels: 26), 24 rows of 900-4096 keys 49 -> 15, 110 rows
 //   of 622-5556 keys 53 -> 19, 64 rows of 8192-32768 keys 432 -> 113 (floor 103), 320 rows of 2698-5095 keys 146 -> 105
 // Beyond kRowMergeMaxItems rows units have two rows each and cutting gives little: 416 to 720 rows measured between
 // 0.91 and 1.02 of the whole rows' speed.  Rows that stay whole take as long as in the persistent loop kernel (0.4 to
@@ -52,14 +52,18 @@ namespace fa {
 #ifndef FA_ROW_MERGE_MAX_ITEMS
 #define FA_ROW_MERGE_MAX_ITEMS 384
 #endif
+constexpr int kRowMergeMaxItems = FA_ROW_MERGE_MAX_ITEMS;
+// Pieces are a whole number of partitions, which are this many bytes of K and V; rows of up to merge_whole_partitions of
+// them stay whole.  Half as long with head size 64, whose pieces have half as much to hand over (us, 128 KiB -> 64 KiB:
+// 24 rows of 900-4096 keys, byte cache 12.9 -> 11.4, 16-bit cache 13.0 -> 11.9; 320 rows of 2698-5095 keys, 16-bit cache 76.5 ->
+// 65.0; with head size 128 15.0 -> 15.6, and 240 log-normal rows of byte caches 19.5 -> 23.4).
 #ifndef FA_ROW_MERGE_PIECE_BYTES
 #define FA_ROW_MERGE_PIECE_BYTES (128 << 10)
 #endif
-constexpr int kRowMergeMaxItems = FA_ROW_MERGE_MAX_ITEMS;
-// Pieces are a whole number of partitions of this many bytes of K and V, two at least; rows of up to
-// kMergeWholePartitions of them stay whole.
-constexpr int kRowMergePartitionBytes = FA_ROW_MERGE_PIECE_BYTES;
-static_assert((kRowMergePartitionBytes & (kRowMergePartitionBytes - 1)) == 0, "MergeRows::cut shifts");
+constexpr int row_merge_partition_bytes(int head_size) {
+  return head_size == 64 ? FA_ROW_MERGE_PIECE_BYTES / 2 : FA_ROW_MERGE_PIECE_BYTES;
+}
+static_assert((FA_ROW_MERGE_PIECE_BYTES & (FA_ROW_MERGE_PIECE_BYTES - 1)) == 0, "MergeRows::cut shifts");
 static_assert(kMergeMaxSeqs == kLoopPersistentMaxSeqs, "a launch takes as many rows whole as in pieces");
 
 // Wavefronts per work-group; wide where the launch without cuts would be (FA_PLOOP_WIDE).
@@ -79,7 +83,9 @@ inline int64_t visible_row_bound(const fa_paged_attention_shape &shape, const Re
   return bound;
 }
 
-inline int row_merge_partition(int row_bytes) { return kRowMergePartitionBytes / (2 * row_bytes); }
+inline int row_merge_partition(int head_size, int elem_bytes) {
+  return row_merge_partition_bytes(head_size) / (2 * head_size * elem_bytes);
+}
 
 inline RowMergeSpace row_merge_space(const fa_paged_attention_shape &shape, const Resolved &r, int32_t max_context_len) {
   RowMergeSpace space;
@@ -91,7 +97,7 @@ inline RowMergeSpace row_merge_space(const fa_paged_attention_shape &shape, cons
     return space;
   if (r.query_len > kMaxGroup / group) return space;  // (two column tiles per wavefront)
   if (items > kRowMergeMaxItems || visible_row_bound(shape, r, max_context_len) <=
-                                       kMergeWholePartitions * row_merge_partition(head_size * r.kv_elem_bytes))
+                                       merge_whole_partitions(head_size) * row_merge_partition(head_size, r.kv_elem_bytes))
     return space;
   // one slice per wavefront, of four wavefronts or of eight (see the launch)
   const int slices = head_size == 128 ? kMergeWaves<true> : kMergeWaves<false>;
@@ -169,7 +175,7 @@ inline fa_status launch_paged_attn_loop_rows(void *out, const void *query, const
       FA_HIP_CHECK(resident_groups(kernel, waves * 64, &resident));
       p.compute_units = cus;
       p.segment_force = 0;
-      p.partition_size = row_merge_partition(HEAD_SIZE * (KV8 ? 1 : 2));
+      p.partition_size = row_merge_partition(HEAD_SIZE, KV8 ? 1 : 2);
       p.merge_flags = static_cast<uint64_t *>(r.workspace);
       p.merge_pieces = reinterpret_cast<float *>(p.merge_flags + merge.flags);
       p.merge_nonce = next_merge_nonce();

@@ -28,7 +28,7 @@ struct WorkItem { int seq, kvh, ctx, c_lo, c_end, tok_end, part0, parts; };
 // length; numbers, among all pieces of the launch, of this piece, of the row's first whole piece (the next ones
 // follow piece_step apart) and of the shorter piece that ends the row.  (Not part of WorkItem: the other kernels'
 // copies of the fields ended up in LDS and cost the segment kernel 7 us a launch.)
-struct MergeItem : WorkItem { int pieces, whole, piece, first_piece, piece_step, last_piece; };
+struct MergeItem : WorkItem { int pieces, whole, piece, first_piece, piece_step, last_piece, first_flag; };
 
 __device__ __forceinline__ int snake_position(int nth, int groups, int group) {
   return nth * groups + ((nth & 1) ? groups - 1 - group : group);
@@ -129,15 +129,17 @@ struct MergeRows {
   int keys[2];   // keys from there on
   int parts[2];  // partitions of them
   int total;     // of all sequences
+  int longest;   // of one
 
   // Whether the launch cuts its rows.  len0, len1: lengths as LoopItems has them (negative: no sequence).  Every
   // wavefront goes through this before its first load of keys, at the speed at which instructions arrive from memory:
   // partitions are a power of two long (row_merge_partition) and everything fits 32 bits (rows below 2^23 keys and
   // 2^15 partitions, at most 2^9 of them).
-  __device__ __forceinline__ bool cut(const PagedAttnParams &p, int len0, int len1) {
+  __device__ __forceinline__ bool cut(const PagedAttnParams &p, int len0, int len1, int stay_whole) {
     const int log2 = 31 - __builtin_clz(p.partition_size);
     const int len[2] = {max(len0, 0), max(len1, 0)};
-    int longest = 0, live = 0, sum = 0;
+    int live = 0, sum = 0;
+    longest = 0;
 #pragma unroll
     for (int j = 0; j < 2; ++j) {
       base[j] = 0;
@@ -151,7 +153,7 @@ struct MergeRows {
     }
     total = wave_total(sum);
     longest = __builtin_amdgcn_readfirstlane(__reduce_max_sync(~0ull, longest));
-    return cut_pays(longest, total, live, p.num_kv_heads, p.compute_units);
+    return cut_pays(longest, total, live, p.num_kv_heads, p.compute_units, stay_whole);
   }
 };
 
@@ -212,7 +214,11 @@ struct SegmentItems {
     }
     m = partitions_per_segment<NQ>(ctxv, parts, rows.total, S, p.partition_size, Hk, groups, p.compute_units,
                                    p.kv_rows_apart != 0, 2 * p.partition_size * item_row_bytes);
-    m = max(m, 2);  // (a piece costs its merge whatever its length)
+    // one partition a piece where every piece gets a unit of its own, else two; where so many pieces of a row meet that their merge
+    // takes many trips to memory, 256 KiB at least (kMergeShortPieces)
+    const int meeting = rows.longest * p.group * p.query_count;
+    if (rows.total * Hk > p.compute_units || meeting > kMergeShortPieces) m = max(m, 2);
+    if (meeting > 4 * kMergeShortPieces) m = max(m, (128 << 10) / (p.partition_size * item_row_bytes));
     const int max_ctx = p.max_blocks_per_seq << p.block_shift;
     while (true) {  // ends: one whole piece per row at most once m spans the longest
       int whole, all;
@@ -410,6 +416,7 @@ struct SegmentItems {
       it.piece_step = Hk;
       it.last_piece = (full_total + s) * Hk + it.kvh;
       it.piece = full ? it.first_piece + seg * Hk : it.last_piece;
+      it.first_flag = (inc_s - full_s + s) * Hk + it.kvh * (full_s + 1);
       return true;
     }
     const int seg = full ? q - (inc_s - full_s) : full_s;

@@ -28,11 +28,21 @@ constexpr int kSegmentMaxPartitions = FA_SEGMENT_MAX_PARTS;
 // cut, over all its rows; what is left of a row behind its whole pieces is one more.  The length of a piece grows
 // until that holds.
 constexpr int kMergeWholePieces = 1024;
-// Rows of up to this many partitions stay whole.
+// The most pieces of a single partition that a row is cut into, times the columns of a piece (a merging wavefront has 64 of
+// these in flight).  us, two partitions a piece -> one: 24 rows of 900-4096 keys 18.4 -> 15.0 (with what the flags in order
+// gave), 8 rows of 16 pieces of 4 columns 17.9 -> 13.4, of 32 20.8 -> 14.7, 2 rows of 118 28.7 -> 21.5; one row of 118 pieces of
+// 16 columns 26.5 -> 34.7 (and so again with 64 KiB a partition, hence four times as many are kept to 256 KiB a piece).
+constexpr int kMergeShortPieces = 512;
+// Rows of up to this many partitions stay whole (their partitions are half as long with head size 64: row_merge_partition).
 #ifndef FA_MERGE_WHOLE_PARTITIONS
 #define FA_MERGE_WHOLE_PARTITIONS 5
 #endif
-constexpr int kMergeWholePartitions = FA_MERGE_WHOLE_PARTITIONS;
+#ifndef FA_MERGE_WHOLE_PARTITIONS_64
+#define FA_MERGE_WHOLE_PARTITIONS_64 3
+#endif
+constexpr int merge_whole_partitions(int head_size) {
+  return head_size == 64 ? FA_MERGE_WHOLE_PARTITIONS_64 : FA_MERGE_WHOLE_PARTITIONS;
+}
 // Where work-groups share a compute unit and each should have work throughout (see `halves` below):
 // bytes of K and V that a unit must have per segment it is given.
 #ifndef FA_SEGMENT_BYTES_WORTH_CUTTING
@@ -283,20 +293,22 @@ __device__ __forceinline__ int two_tile_partitions_per_segment(const int (&ctxv)
 }
 
 // Whether a launch that merges the pieces of a row itself cuts its rows at all.  longest, total: partitions of
-// the longest row, and of all sequences; live: sequences that have any; units: compute units of the GPU.  Uncut,
+// the longest row, and of all sequences; live: sequences that have any; units: compute units of the GPU; stay_whole:
+// merge_whole_partitions.  Uncut,
 // the launch lasts as long as its longest row takes one work-group, or as long as the memory takes for all rows;
-// a cut costs some 4 us (the pieces through memory, flags, merge), as much as two partitions (a partition is
-// 128 KiB of K and V: row_merge_partition).  Measured with rows cut always (us, whole -> cut):
-//   rows of up to kMergeWholePartitions lose: 11 to 296 rows 7.7 -> 11.1, 10.6 -> 16.0, 16.8 -> 17.6, 14.0 -> 24.2
+// a cut costs some 2 us (the pieces through memory, flags, merge), as much as a partition (128 KiB of K and V with head
+// size 128: row_merge_partition; 128 rows of 2500 keys 42.4 -> 35.9).  Measured with rows cut always (us, whole -> cut):
+//   rows of up to merge_whole_partitions gain or lose with their number (16 rows of 600 keys 11.2 -> 11.9, 24 of 1300 in byte
+//     caches 12.4 -> 12.6, 40 of 900 16.9 -> 13.0)
 //   up to one row per unit: a work-group alone on its unit streams 1 / 160 of what the memory gives 256 units, so
 //     cutting pays where the longest row exceeds that share of all rows.  Unequal rows: 24 rows 49 -> 18, 110 rows
 //     53 -> 19, 168 rows 39 -> 31; equal ones, whose sum already keeps the memory busy: 176 rows 30 -> 44, 192 rows
 //     114 -> 119, 208 rows 39 -> 43 (and 119 rows 152 -> 96, 8 rows 402 -> 32)
 //   more rows than units: a unit has two rows or one, and unequal rows meet badly.  268 rows 66 -> 46, 288 rows
 //     118 -> 94, 320 rows 147 -> 105; equal rows 384: 76 -> 88
-__device__ __forceinline__ bool cut_pays(int longest, int total, int live, int num_kv_heads, int units) {
-  if (longest <= kMergeWholePartitions) return false;
-  if (live * num_kv_heads <= units) return (longest - 2) * (units * 5 >> 3) > total * num_kv_heads;
+__device__ __forceinline__ bool cut_pays(int longest, int total, int live, int num_kv_heads, int units, int stay_whole) {
+  if (longest <= stay_whole) return false;
+  if (live * num_kv_heads <= units) return (longest - 1) * (units * 5 >> 3) > total * num_kv_heads;
   return 4 * longest * live > 5 * total;
 }
 

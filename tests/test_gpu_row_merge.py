@@ -310,3 +310,22 @@ def test_calls_go_to_the_current_stream():
             again = torch.empty_like(out).copy_(out)  # ordered behind the call on its stream only
         stream.synchronize()
         assert torch.equal(out, again) and torch.isfinite(again.float()).all()
+
+
+@pytest.mark.parametrize("lens, hk, group, fp8", [
+    ([32768, 300], 1, 4, None),        # 128 partitions in the longest row: a partition a piece
+    ([32769, 300], 1, 4, None),        # 129: two
+    ([16384, 16128], 2, 2, None),      # 254 pieces of one partition for 256 units
+    ([16384, 16385], 2, 2, None),      # 258 would be: two partitions a piece
+    ([7000, 0, 513, 4097, 1], 8, 8, E5M2),  # 25 partitions x 8 kv heads, eight wavefronts a work-group
+    ([3000] * 9, 4, 1, None),          # 108 pieces, one head a kv head
+])
+def test_pieces_of_one_partition(oracle, lens, hk, group, fp8):
+    """Both sides of the rule by which a piece is one partition or two, from memory that held another batch's flags."""
+    w = _workload(lens, hk, group, 128, fp8, bf16=True, sinks=True)
+    assert _needs(w) > 0
+    dev = torch.device("cuda:0")
+    out, again = _run(w, dev), _run(w, dev)
+    torch.cuda.synchronize()
+    assert torch.equal(out, again), "the order of arrival shows in the result"
+    _check(oracle, w, out)
