@@ -307,8 +307,23 @@ inline bool loop_persistent_fits(const fa_paged_attention_shape &shape) {
          (int64_t)shape.max_blocks_per_seq * shape.block_size < kLoopPersistentMaxContext;
 }
 
+// Whether a batch of more sequences than the persistent kernel ranks, from a 16-bit cache, is one launch of the grid form
+// all the same: sub-batches pay a launch's fixed cost twice or more, the grid form starts a stream for every row.  Measured on
+// 206 batches of 130 to 512 sequences of up to 2048 keys, 260 to 4800 rows, sub-batches against grid form:
+//   head size 64    1.45 times as fast in the mean of 122, 5 % slower in two (200 sequences of 40-200 keys, 4 kv heads 14.7 -> 10.1 us)
+//   head size 128   up to 5 rows for every unit 1.34 times in the mean of 59, 3 % slower at worst (130 of 200-1000 keys, 2 kv heads 37.0 ->
+//                   23.7 us); more rows 0.96 times in the mean of 25, 0.68 at worst (150 of 12-64 keys, 32 kv heads)
+// Longer rows, and several query tokens that do not fit one column tile, stay with the sub-batches.
+constexpr int kGridBelowTokens = 2048, kGridRowsPerUnit = 5;
+inline bool large_batch_runs_as_grid(const fa_paged_attention_shape &shape, const Resolved &r, int compute_units) {
+  int64_t bound = (int64_t)shape.max_blocks_per_seq * shape.block_size;
+  if (r.max_context_len > 0) bound = std::min<int64_t>(bound, r.max_context_len);
+  if (bound > kGridBelowTokens || r.query_len > kMaxGroup / r.group) return false;
+  return shape.head_size == 64 || (int64_t)shape.num_seqs * shape.num_kv_heads <= (int64_t)kGridRowsPerUnit * compute_units;
+}
+
 // A batch of more sequences than the persistent kernel ranks is cut into equal sub-batches,
-// one persistent launch each, where that beats the grid form (PersistentLoop::sub_batches).
+// one persistent launch each, where that beats the grid form (PersistentLoop::sub_batches, large_batch_runs_as_grid).
 template <int HEAD_SIZE, typename QT, int KVF>
 inline fa_status launch_paged_attn_loop(void *out, const void *query, const void *key_cache,
                                         const void *value_cache, const int32_t *block_tables,
@@ -332,8 +347,13 @@ inline fa_status launch_paged_attn_loop(void *out, const void *query, const void
   }
   if (dot.schedule != r.schedule) return launch_paged_attn_loop<HEAD_SIZE, QT, KVF>(out, query, key_cache, value_cache, block_tables,
                                                                                     context_lens, scale, shape, dot);
-  const bool persistent_pieces = PersistentLoop<(KVF != kKv16)>::sub_batches && r.schedule == FA_SCHEDULE_AUTO &&
-                                 loop_persistent_fits(shape) && shape.num_seqs > kLoopPersistentMaxSeqs;
+  bool persistent_pieces = PersistentLoop<(KVF != kKv16)>::sub_batches && r.schedule == FA_SCHEDULE_AUTO &&
+                           loop_persistent_fits(shape) && shape.num_seqs > kLoopPersistentMaxSeqs;
+  if (persistent_pieces) {
+    int cus = 0;
+    FA_HIP_CHECK(compute_units_of_current_device(&cus));
+    persistent_pieces = !large_batch_runs_as_grid(shape, r, cus);
+  }
   const int most = persistent_pieces ? kLoopPersistentMaxSeqs : kGridMaxSeqs;
   if (shape.num_seqs > most) {
     const int pieces = (shape.num_seqs + most - 1) / most;
