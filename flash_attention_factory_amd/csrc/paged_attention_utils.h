@@ -194,16 +194,24 @@ __device__ __forceinline__ uint32_t fp8_adjacent_pair(uint32_t w, int half) {
   }
 }
 
-// Reductions over the four 16-lane rows of a wavefront (lanes i, i+16, i+32, i+48).
+// Reductions over the four 16-lane rows of a wavefront (lanes i, i+16, i+32, i+48), the result in every lane.  v_permlane16_swap
+// exchanges the odd rows of one register with the even rows of another, v_permlane32_swap the upper half with the lower
+// half: given the same value twice, they leave a pair's two members in the same lane of the two registers.  Vector
+// instructions; the shuffles through LDS that did this before took two LDS latencies, one behind the other, of
+// every chunk of keys, between its scores and its exponentials.
+template <typename F>
+__device__ __forceinline__ float rows_fold(float v, F &&f) {
+  const uint32_t a = __builtin_bit_cast(uint32_t, v);
+  const auto x = __builtin_amdgcn_permlane16_swap(a, a, false, false);
+  const uint32_t b = __builtin_bit_cast(uint32_t, f(__builtin_bit_cast(float, (uint32_t)x[0]), __builtin_bit_cast(float, (uint32_t)x[1])));
+  const auto y = __builtin_amdgcn_permlane32_swap(b, b, false, false);
+  return f(__builtin_bit_cast(float, (uint32_t)y[0]), __builtin_bit_cast(float, (uint32_t)y[1]));
+}
 __device__ __forceinline__ float rows_max(float v) {
-  v = fmaxf(v, __shfl_xor(v, 16));
-  v = fmaxf(v, __shfl_xor(v, 32));
-  return v;
+  return rows_fold(v, [](float x, float y) { return fmaxf(x, y); });
 }
 __device__ __forceinline__ float rows_sum(float v) {
-  v += __shfl_xor(v, 16);
-  v += __shfl_xor(v, 32);
-  return v;
+  return rows_fold(v, [](float x, float y) { return x + y; });
 }
 __device__ __forceinline__ float wave_max(float v) {
 #pragma unroll
