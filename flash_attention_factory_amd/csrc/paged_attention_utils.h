@@ -213,15 +213,24 @@ __device__ __forceinline__ float rows_max(float v) {
 __device__ __forceinline__ float rows_sum(float v) {
   return rows_fold(v, [](float x, float y) { return x + y; });
 }
+// The value of the lane N places on within a row of 16 lanes (in a ring).
+template <int N>
+__device__ __forceinline__ float row_rotated(float v) {
+  return __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, v), 0x120 + N, 0xF, 0xF, true));
+}
 __device__ __forceinline__ float wave_max(float v) {
-#pragma unroll
-  for (int o = 32; o >= 1; o >>= 1) v = fmaxf(v, __shfl_xor(v, o));
-  return v;
+  v = fmaxf(v, row_rotated<8>(v));
+  v = fmaxf(v, row_rotated<4>(v));
+  v = fmaxf(v, row_rotated<2>(v));
+  v = fmaxf(v, row_rotated<1>(v));
+  return rows_max(v);
 }
 __device__ __forceinline__ float wave_sum(float v) {
-#pragma unroll
-  for (int o = 32; o >= 1; o >>= 1) v += __shfl_xor(v, o);
-  return v;
+  v += row_rotated<8>(v);
+  v += row_rotated<4>(v);
+  v += row_rotated<2>(v);
+  v += row_rotated<1>(v);
+  return rows_sum(v);
 }
 
 // Load one int32 of read-only input through the scalar unit.  `p` must be wave-uniform and
