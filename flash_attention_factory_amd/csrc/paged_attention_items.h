@@ -177,8 +177,8 @@ struct SegmentItems {
   // batch, the number of work-groups and the compute units they share (partitions_per_segment).
   // heads_per_item: adjacent kv heads that one work-group takes together (its wavefronts in teams);
   // item_row_bytes: bytes of one token's K row (as of its V row) of an item
-  // TWO_TILES: the kernel holds two column tiles
-  template <bool TWO_TILES = false>
+  // TWO_TILE_HEAD: head size of a kernel that holds two column tiles (0: it does not)
+  template <int TWO_TILE_HEAD = 0>
   __device__ __forceinline__ void build(const PagedAttnParams &p, int lane_, int groups, int heads_per_item,
                                         int item_row_bytes) {
     static_assert(!ROW_MERGE);
@@ -193,9 +193,10 @@ struct SegmentItems {
       return;
     }
     m = p.segment_force > 0 ? min(p.segment_force, kSegmentMaxPartitions) : 0;
-    if constexpr (TWO_TILES) {
+    if constexpr (TWO_TILE_HEAD > 0) {
       if (m == 0)
-        m = two_tile_partitions_per_segment<NQ>(ctxv, parts, total_parts, S, p.partition_size, Hk, min(groups, p.compute_units));
+        m = two_tile_partitions_per_segment<NQ, TWO_TILE_HEAD>(ctxv, parts, total_parts, S, p.partition_size, Hk, groups,
+                                                               min(groups, p.compute_units), 2 * item_row_bytes, heads_per_item > 1);
     }
     if (m == 0)
       m = partitions_per_segment<NQ>(ctxv, parts, total_parts, S, p.partition_size, Hk, groups, p.compute_units,

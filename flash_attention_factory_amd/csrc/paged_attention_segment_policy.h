@@ -259,19 +259,60 @@ __device__ __forceinline__ int partitions_per_segment(const int (&ctxv)[NQ], con
   return before > 0 ? before : m;
 }
 
+// Keys, in steps of 32, that work-group 0 gets if every row stays whole: of the rows, longest first and kv heads fastest, it takes
+// positions 0, 2G - 1, 2G, 4G - 1, 4G, ... (snake_position), the heaviest share where a few rows are much longer than the
+// others.  The length at a position is found from the top, two bits at a time.  (Counting the rows above 16 levels, whatever the
+// number of positions, took 2 to 3 us of a launch.)  rows: of all kv heads, below 2^24; longest: of them, in steps as well
+template <int NQ>
+__device__ __forceinline__ long long whole_rows_of_first_group(const int (&steps)[NQ], int S, int rows, int num_kv_heads, int groups,
+                                                               int longest) {
+  long long load = longest;
+  const float inv = __builtin_amdgcn_rcpf((float)num_kv_heads);
+#pragma nounroll
+  for (int pos = 2 * groups - 1; pos < rows; pos += 2 * groups) {
+    int rem, length = 0;
+    const int rank = quotient_below_2p24(pos, num_kv_heads, inv, rem);
+#pragma nounroll
+    for (int bit = (31 - __builtin_clz(longest | 1)) & ~1; bit >= 0; bit -= 2) {
+      int at_least[3] = {0, 0, 0};
+#pragma unroll
+      for (int j = 0; j < NQ; ++j)
+        if (j * 64 < S) {
+#pragma unroll
+          for (int c = 0; c < 3; ++c) at_least[c] += __builtin_popcountll(__ballot(steps[j] >= (length | ((c + 1) << bit))));
+        }
+      length |= ((at_least[0] > rank) + (at_least[1] > rank) + (at_least[2] > rank)) << bit;
+    }
+    load += pos + 1 < rows ? 2 * length : length;  // (both positions of the pair: a row apart at most)
+  }
+  return load;
+}
+
 // The same for the kernels of two column tiles, one work-group per compute unit (paged_attention_loop_two_tile_kernel.h):
 // what a partial of 32 columns costs (16 KiB through tmp_out with head size 128, a merge without loads in flight)
-// makes cutting dear.  0: no opinion, partitions_per_segment decides.  Every length was forced in turn on 44 batches (us, with
-// the length that partitions_per_segment takes -> with this one):
-//   rows stay whole where the longest is no more than 4/3 of a unit's mean load: 48 rows of 257-6000 keys, 8 kv heads, byte
-//     cache 78.0 -> 73.0, head size 64 65.2 -> 59.5, 16-bit cache 115.7 -> 115.8; 100 of 400-4000, 4 kv heads 64.3 -> 60.7, 91.4 ->
-//     87.4; 24 of 1000-5000, 16 kv heads 75.5 -> 72.9, 109.3 -> 107.6
-//   a row per unit at most, longer ones among them: the shortest segment of which there are no more than units, if that is
-//     up to 4/3 of the load as well (3 rows of 1000-5000, 32 kv heads, head size 64 33.3 -> 28.0; 64 of 200-8000, 2 kv heads, head
-//     size 64 about 38 -> 34.5)
-template <int NQ>
+// makes cutting dear.  0: no opinion, partitions_per_segment decides.  key_bytes: of an item, K and V.  Measured on some 200 batches
+// (us, with the length that partitions_per_segment takes -> with this one):
+//   rows stay whole where the longest is no more than 4/3 of a unit's mean load and the unit that gets it, and others, has no
+//     more than kTwoTileWholeExcess (teams: kTwoTileWholeExcessTeams), or a sixth of it, above the mean: 48 rows of 257-6000 keys, 8 kv heads, byte cache 78.0 -> 72.9, head size
+//     64 65.2 -> 59.5, 16-bit cache 115.7 -> 115.8; 100 of 400-4000, 4 kv heads 64.3 -> 60.7, 91.4 -> 87.4; 24 of 1000-5000,
+//     16 kv heads 75.5 -> 72.9, 109.3 -> 107.6.  Batches with 50 to 480 KiB above the mean were 0.86 to 1.00 times as long (teams of kv
+//     heads with 230 and 262 KiB 1.05 and 1.01), with 500 to 570 KiB 1.02 to 1.06 (0.94 where that is an eighth of the mean), with 0.9
+//     to 4.7 MiB 1.04 to 1.23: log-normal
+//     lengths, whose longest row meets others (157 rows of median 2000 keys, 8 kv heads, byte cache 214 -> 263 if whole)
+//   a row per unit at most, longer ones among them: the shortest segment of which there are no more than units, if that is up to
+//     4/3 of the load as well, or the mean load in partitions, rounded up (3 rows of 1000-5000, 32 kv heads, head size 64 33.3 -> 28.0;
+//     64 of 200-8000, 2 kv heads, head size 64 38.3 -> 35.8; 16 of 745-3191, 8 kv heads, byte cache 31.8 -> 27.4) -- and no more
+//     than kTwoTileSegmentExcess above the mean where that is large: partitions of 256 KiB rounded up (9 rows of 1623 keys,
+//     8 kv heads, 16-bit cache 26.4 -> 28.4), and 4/3 with head size 64, whose partials are half as large (34 of 4748-10618, 4 teams
+//     of kv heads, 16-bit cache 101.7 -> 106.8)
+// The batch's keys are added up only where a bound is in keys: every instruction here lies before the first load of a launch (0.5 us
+// where they always were).
+constexpr int kTwoTileWholeExcess = 480 << 10, kTwoTileWholeExcessTeams = 192 << 10;
+constexpr int kTwoTileSegmentExcess128 = 280 << 10, kTwoTileSegmentExcess64 = 224 << 10;
+template <int NQ, int D>
 __device__ __forceinline__ int two_tile_partitions_per_segment(const int (&ctxv)[NQ], const int (&parts)[NQ], int total_partitions,
-                                                               int S, int partition_size, int num_kv_heads, int units) {
+                                                               int S, int partition_size, int num_kv_heads, int groups, int units,
+                                                               int key_bytes, bool teams) {
   int longest = 0, live = 0;
 #pragma unroll
   for (int j = 0; j < NQ; ++j) {
@@ -279,14 +320,38 @@ __device__ __forceinline__ int two_tile_partitions_per_segment(const int (&ctxv)
     if (j * 64 < S) live += __builtin_popcountll(__ballot(parts[j] > 0));
   }
   longest = __builtin_amdgcn_readfirstlane(__reduce_max_sync(~0ull, longest));
-  const long long items = (long long)total_partitions * num_kv_heads;
-  if (longest <= kSegmentMaxPartitions && 3LL * longest * units <= 4 * items) return max(longest, 1);
-  if ((long long)live * num_kv_heads > units) return 0;
-  const int mean = (int)((items + units - 1) / units);
+  const long long items = (long long)total_partitions * num_kv_heads, rows = (long long)live * num_kv_heads;
+  const bool whole = longest <= kSegmentMaxPartitions && 3LL * longest * units <= 4 * items;
+  if (whole && rows < 2 * groups) return max(longest, 1);  // (work-group 0 gets one row)
+  if (rows > (whole ? (1 << 24) - 1 : units)) return 0;
+  const int mean = max((int)((items + units - 1) / units), 1);
+  const bool within = 3LL * mean * units <= 4 * items;
+  const bool bounded = whole || (D == 128 ? !within && partition_size * key_bytes > 128 << 10 : within);
+  long long load = 0;  // of all units, in steps of 32 keys
+  int steps[NQ];
+  if (bounded) {
+    int sum = 0, longest_row = 0;
+#pragma unroll
+    for (int j = 0; j < NQ; ++j) {
+      steps[j] = (min(ctxv[j], parts[j] * partition_size) + 16) >> 5;
+      longest_row = max(longest_row, steps[j]);
+      sum += steps[j];
+    }
+    load = (long long)wave_total(sum) * num_kv_heads;
+    if (whole) {
+      longest_row = __builtin_amdgcn_readfirstlane(__reduce_max_sync(~0ull, longest_row));
+      const long long bound = teams ? kTwoTileWholeExcessTeams : kTwoTileWholeExcess;
+      if ((long long)longest_row * (32 * key_bytes) <= bound) return longest;  // (never more than that above the mean)
+      const long long excess = whole_rows_of_first_group<NQ>(steps, S, (int)rows, num_kv_heads, groups, longest_row) * units - load;
+      return excess * (32 * key_bytes) <= bound * units || 6 * excess <= load ? longest : 0;
+    }
+  }
+  constexpr long long kExcess = D == 128 ? kTwoTileSegmentExcess128 : kTwoTileSegmentExcess64;
 #pragma nounroll
-  for (int m = max(mean, 1); m <= kSegmentMaxPartitions && (m == mean || 3LL * m * units <= 4 * items); ++m) {
-    int whole, all;
-    count_segments<NQ>(ctxv, parts, S, partition_size, m, whole, all);
+  for (int m = mean; m <= kSegmentMaxPartitions && (m == mean || 3LL * m * units <= 4 * items); ++m) {
+    if (bounded && (((long long)m * partition_size >> 5) * units - load) * (32 * key_bytes) > kExcess * units) return 0;
+    int all, unused;
+    count_segments<NQ>(ctxv, parts, S, partition_size, m, unused, all);
     if ((long long)all * num_kv_heads <= units) return m;
   }
   return 0;

@@ -109,6 +109,63 @@ def partitions_per_segment(lens, *, partition_size: int, max_num_partitions: int
     return before if before > 0 else m
 
 
+def whole_rows_of_first_group(steps, num_kv_heads: int, groups: int) -> int:
+    order = sorted((x for x in steps if x > 0), reverse=True)
+    rows = len(order) * num_kv_heads
+    load = order[0] if order else 0
+    for pos in range(2 * groups - 1, rows, 2 * groups):
+        load += order[pos // num_kv_heads] * (2 if pos + 1 < rows else 1)
+    return load
+
+
+TWO_TILE_WHOLE_EXCESS = {False: 480 << 10, True: 192 << 10}  # teams of kv heads
+TWO_TILE_SEGMENT_EXCESS = {128: 280 << 10, 64: 224 << 10}
+
+
+def two_tile_partitions_per_segment(lens, *, head_size: int, partition_size: int, max_num_partitions: int, max_ctx: int,
+                                    num_kv_heads: int, groups: int, cus: int, rows_apart: bool, partition_bytes: int, teams: bool) -> int:
+    """The rule of the kernels of two column tiles, and partitions_per_segment where it has no opinion."""
+    ctx, parts = live_partitions(lens, partition_size, max_num_partitions, max_ctx)
+    units = min(groups, cus)
+    steps = [(min(c, p * partition_size) + 16) >> 5 for c, p in zip(ctx, parts)]
+    longest, rows = max(parts), sum(p > 0 for p in parts) * num_kv_heads
+    items, load = sum(parts) * num_kv_heads, sum(steps) * num_kv_heads
+    step_bytes = 32 * (partition_bytes // partition_size)
+    whole = longest <= SEGMENT_MAX_PARTITIONS and 3 * longest * units <= 4 * items
+    if whole and rows < 2 * groups:
+        return max(longest, 1)
+    if whole:
+        excess = whole_rows_of_first_group(steps, num_kv_heads, groups) * units - load
+        bound = TWO_TILE_WHOLE_EXCESS[teams]
+        if max(steps) * step_bytes <= bound or excess * step_bytes <= bound * units or 6 * excess <= load:
+            return longest
+    elif rows <= units:
+        mean = m = max(-(-items // units), 1)
+        within = 3 * mean * units <= 4 * items
+        bounded = not within and partition_bytes > 128 << 10 if head_size == 128 else within
+        while m <= SEGMENT_MAX_PARTITIONS and (m == mean or 3 * m * units <= 4 * items):
+            if bounded and ((m * partition_size >> 5) * units - load) * step_bytes > TWO_TILE_SEGMENT_EXCESS[head_size] * units:
+                break
+            if count_segments(ctx, parts, partition_size, m)[1] * num_kv_heads <= units:
+                return m
+            m += 1
+    return partitions_per_segment(lens, partition_size=partition_size, max_num_partitions=max_num_partitions, max_ctx=max_ctx,
+                                  num_kv_heads=num_kv_heads, groups=groups, cus=cus, rows_apart=rows_apart,
+                                  partition_bytes=partition_bytes)
+
+
+def dealt_keys(lens, m: int, *, partition_size: int, max_num_partitions: int, max_ctx: int, num_kv_heads: int, groups: int):
+    """Keys that every work-group reads when the batch is cut into segments of m partitions: whole segments first, then the
+    rows' ends, longest first, dealt to and fro (csrc/paged_attention_items.h: SegmentItems::at, snake_position)."""
+    segs = sorted(segments_of(lens, m, partition_size=partition_size, max_num_partitions=max_num_partitions, max_ctx=max_ctx),
+                  reverse=True)
+    keys = [0] * groups
+    for pos in range(len(segs) * num_kv_heads):
+        nth, g = divmod(pos, groups)
+        keys[groups - 1 - g if nth & 1 else g] += segs[pos // num_kv_heads]
+    return keys
+
+
 SHARE_TOKENS = 32
 SHARE_PIECE_COST = 4
 

@@ -8,6 +8,7 @@ import json
 import math
 import os
 import random
+import statistics
 
 import pytest
 
@@ -130,3 +131,46 @@ def test_properties_over_random_batches():
         # unit's mean load (in partitions, rounded up) unless one partition already is
         per_unit = total / min(groups, cus)
         assert m <= max(1, math.ceil(2 * per_unit)), (m, per_unit, kw)
+
+
+def _two_tile_args(**kw):
+    base = dict(head_size=128, partition_size=512, max_num_partitions=64, max_ctx=32768, num_kv_heads=8, groups=256, cus=256,
+                rows_apart=False, partition_bytes=512 * 256, teams=False)
+    base.update(kw)
+    return base
+
+
+def test_two_tile_rule_constants_are_the_ones_replayed():
+    src = open(os.path.join(os.path.dirname(HERE), "flash_attention_factory_amd", "csrc", "paged_attention_segment_policy.h")).read()
+    for literal in ("kTwoTileWholeExcess = 480 << 10", "kTwoTileWholeExcessTeams = 192 << 10", "kTwoTileSegmentExcess128 = 280 << 10",
+                    "kTwoTileSegmentExcess64 = 224 << 10", "3LL * longest * units <= 4 * items", "rows < 2 * groups",
+                    "6 * excess <= load", "partition_size * key_bytes > 128 << 10"):
+        assert literal in src, literal
+
+
+def test_two_tile_rows_stay_whole_only_where_the_deal_balances():
+    """Log-normal lengths: the work-group with the longest rows gets no more above the mean than the bound, whatever the
+    number of rows a unit has; rows much like each other, and rows of a unit each, stay whole."""
+    normal = statistics.NormalDist()
+    cut = left = 0
+    for heads in (4, 8, 16):
+        for n in range(20, 250, 13):
+            for median in (400, 1000, 2000):
+                lens = [min(16384, int(median * math.exp(0.75 * normal.inv_cdf((k + 0.5) / n)))) for k in range(n)]
+                m = P.two_tile_partitions_per_segment(lens, **_two_tile_args(num_kv_heads=heads))
+                if m * 512 < max(lens) or n * heads < 512:
+                    cut += m * 512 < max(lens)
+                    continue
+                left += 1
+                keys = P.dealt_keys(lens, m, partition_size=512, max_num_partitions=64, max_ctx=32768, num_kv_heads=heads, groups=256)
+                mean = sum(keys) / 256
+                # (lengths count in steps of 32 keys, and the two rows of a pair of positions as the longer one)
+                assert max(keys) - mean <= max((480 << 10) / 256, mean / 6, max(lens) if max(lens) * 256 <= 480 << 10 else 0) + 64 * n * heads / 512 + 600, (heads, n, median)
+    assert cut > 20 and left > 20, (cut, left)
+    for lens, heads in (([int(2000 * math.exp(0.75 * normal.inv_cdf((k + 0.5) / 157))) for k in range(157)], 8),
+                        ([min(16384, int(553 * (16883 / 553) ** (k / 48))) for k in range(49)], 16)):
+        args = _two_tile_args(num_kv_heads=heads)
+        base = {k: v for k, v in args.items() if k not in ("head_size", "teams")}
+        assert P.two_tile_partitions_per_segment(lens, **args) == P.partitions_per_segment(lens, **base) < max(lens) // 512
+    assert P.two_tile_partitions_per_segment([257 + 5743 * k // 47 for k in range(48)], **_two_tile_args()) == 12
+    assert P.two_tile_partitions_per_segment([3000] * 30, **_two_tile_args()) == 6
