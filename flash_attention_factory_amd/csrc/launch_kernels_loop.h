@@ -97,7 +97,7 @@ inline RowMergeSpace row_merge_space(const fa_paged_attention_shape &shape, cons
     return space;
   if (r.query_len > kMaxGroup / group) return space;  // (two column tiles per wavefront)
   if (items > kRowMergeMaxItems || visible_row_bound(shape, r, max_context_len) <=
-                                       merge_whole_partitions(head_size) * row_merge_partition(head_size, r.kv_elem_bytes))
+                                       merge_whole_partitions(head_size, r.kv_elem_bytes) * row_merge_partition(head_size, r.kv_elem_bytes))
     return space;
   // one slice per wavefront, of four wavefronts or of eight (see the launch)
   const int slices = head_size == 128 ? kMergeWaves<true> : kMergeWaves<false>;

@@ -134,26 +134,27 @@ struct MergeRows {
   // Whether the launch cuts its rows.  len0, len1: lengths as LoopItems has them (negative: no sequence).  Every
   // wavefront goes through this before its first load of keys, at the speed at which instructions arrive from memory:
   // partitions are a power of two long (row_merge_partition) and everything fits 32 bits (rows below 2^23 keys and
-  // 2^15 partitions, at most 2^9 of them).
-  __device__ __forceinline__ bool cut(const PagedAttnParams &p, int len0, int len1, int stay_whole) {
+  // 2^15 partitions, at most 2^9 of them).  SEEN: the longest row counts by the keys that are seen, without those that
+  // lie before the window in its first partition
+  template <bool SEEN>
+  __device__ __forceinline__ bool cut(const PagedAttnParams &p, int len0, int len1, int stay_whole, int extra) {
     const int log2 = 31 - __builtin_clz(p.partition_size);
     const int len[2] = {max(len0, 0), max(len1, 0)};
     int live = 0, sum = 0;
     longest = 0;
 #pragma unroll
     for (int j = 0; j < 2; ++j) {
-      base[j] = 0;
-      if (p.mask_flags & kMaskWindow)
-        base[j] = max(0, len[j] - p.query_len + p.query_first - p.window_left) >> log2 << log2;
+      const int first = (p.mask_flags & kMaskWindow) ? max(0, len[j] - p.query_len + p.query_first - p.window_left) : 0;
+      base[j] = first >> log2 << log2;
       keys[j] = len[j] - base[j];
       parts[j] = (keys[j] + p.partition_size - 1) >> log2;
-      longest = max(longest, parts[j]);
+      longest = max(longest, SEEN ? (len[j] - first + p.partition_size - 1) >> log2 : parts[j]);
       sum += parts[j];
       live += __builtin_popcountll(__ballot(parts[j] > 0));
     }
     total = wave_total(sum);
     longest = __builtin_amdgcn_readfirstlane(__reduce_max_sync(~0ull, longest));
-    return cut_pays(longest, total, live, p.num_kv_heads, p.compute_units, stay_whole);
+    return cut_pays(longest, total, live, p.num_kv_heads, p.compute_units, stay_whole, extra);
   }
 };
 

@@ -40,8 +40,9 @@ paged_attn_loop_cut_kernel(const PagedAttnParams p) {
   LoopItems<TPC> rows;
   rows.build(p, lane, wave, row_count, W::CT);
   MergeRows merge;
-  bool cut = __any(max(rows.len0, rows.len1) > merge_whole_partitions(D) * p.partition_size);
-  if (cut) cut = merge.cut(kernel_params(), rows.len0, rows.len1, merge_whole_partitions(D));
+  constexpr int kBytes = KVF == kKv16 ? 2 : 1, kStayWhole = merge_whole_partitions(D, kBytes);
+  bool cut = __any(max(rows.len0, rows.len1) > kStayWhole * p.partition_size);
+  if (cut) cut = merge.cut<D == 64>(kernel_params(), rows.len0, rows.len1, kStayWhole, merge_extra_cost(D, kBytes));
   if (!cut) {
     if ((int)blockIdx.x >= row_count) return;
     // (the extended instances, given p, get a stack frame that they do not use, and with it scratch memory)

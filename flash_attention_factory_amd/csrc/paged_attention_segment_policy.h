@@ -33,16 +33,13 @@ constexpr int kMergeWholePieces = 1024;
 // gave), 8 rows of 16 pieces of 4 columns 17.9 -> 13.4, of 32 20.8 -> 14.7, 2 rows of 118 28.7 -> 21.5; one row of 118 pieces of
 // 16 columns 26.5 -> 34.7 (and so again with 64 KiB a partition, hence four times as many are kept to 256 KiB a piece).
 constexpr int kMergeShortPieces = 512;
-// Rows of up to this many partitions stay whole (their partitions are half as long with head size 64: row_merge_partition).
-#ifndef FA_MERGE_WHOLE_PARTITIONS
-#define FA_MERGE_WHOLE_PARTITIONS 5
-#endif
-#ifndef FA_MERGE_WHOLE_PARTITIONS_64
-#define FA_MERGE_WHOLE_PARTITIONS_64 3
-#endif
-constexpr int merge_whole_partitions(int head_size) {
-  return head_size == 64 ? FA_MERGE_WHOLE_PARTITIONS_64 : FA_MERGE_WHOLE_PARTITIONS;
-}
+// Rows of up to this many partitions stay whole (with head size 64 partitions are half as long: row_merge_partition), fewer where a
+// partition has 512 keys.  Head size 64, us, whole -> cut: 3 rows of 1409-3189 keys, byte cache 16.6 -> 10.5, 20 of 1948-4124 13.9 ->
+// 11.8; 16-bit cache 4 rows of 1918 keys 14.1 -> 9.9, 24 of 620-1236 12.5 -> 10.8; but of up to 1024 keys 16 of 774 8.9 -> 9.7,
+// 32 of 826 9.9 -> 11.4, 208 of 30-992 10.7 -> 12.9, 168 of 270-827 11.1 -> 12.8.
+constexpr int merge_whole_partitions(int head_size, int elem_bytes) { return head_size == 128 ? 5 : elem_bytes == 2 ? 4 : 3; }
+// What a cut costs beyond a partition, in partitions (cut_pays).
+constexpr int merge_extra_cost(int head_size, int elem_bytes) { return head_size == 64 && elem_bytes == 2 ? 1 : 0; }
 // Where work-groups share a compute unit and each should have work throughout (see `halves` below):
 // bytes of K and V that a unit must have per segment it is given.
 #ifndef FA_SEGMENT_BYTES_WORTH_CUTTING
@@ -359,22 +356,25 @@ __device__ __forceinline__ int two_tile_partitions_per_segment(const int (&ctxv)
 
 // Whether a launch that merges the pieces of a row itself cuts its rows at all.  longest, total: partitions of
 // the longest row, and of all sequences; live: sequences that have any; units: compute units of the GPU; stay_whole:
-// merge_whole_partitions.  Uncut,
-// the launch lasts as long as its longest row takes one work-group, or as long as the memory takes for all rows;
-// a cut costs some 2 us (the pieces through memory, flags, merge), as much as a partition (128 KiB of K and V with head
-// size 128: row_merge_partition; 128 rows of 2500 keys 42.4 -> 35.9).  Measured with rows cut always (us, whole -> cut):
+// merge_whole_partitions; extra: merge_extra_cost.  Uncut, the launch lasts as long as its longest row takes one work-group, or as
+// long as the memory takes for all rows; a cut costs some 2 us (the pieces through memory, flags, merge), as much as a partition
+// (128 KiB of K and V with head size 128: row_merge_partition; 128 rows of 2500 keys 42.4 -> 35.9), or `extra` more where
+// most pieces share a unit.  Measured with rows cut always (us, whole -> cut):
 //   rows of up to merge_whole_partitions gain or lose with their number (16 rows of 600 keys 11.2 -> 11.9, 24 of 1300 in byte
 //     caches 12.4 -> 12.6, 40 of 900 16.9 -> 13.0)
 //   up to one row per unit: a work-group alone on its unit streams 1 / 160 of what the memory gives 256 units, so
-//     cutting pays where the longest row exceeds that share of all rows.  Unequal rows: 24 rows 49 -> 18, 110 rows
-//     53 -> 19, 168 rows 39 -> 31; equal ones, whose sum already keeps the memory busy: 176 rows 30 -> 44, 192 rows
-//     114 -> 119, 208 rows 39 -> 43 (and 119 rows 152 -> 96, 8 rows 402 -> 32)
+//     cutting pays where the longest row exceeds that share of all rows.  Unequal rows: 24 rows 49 -> 15, 110 rows
+//     53 -> 19, 168 rows 39 -> 31; equal ones, whose sum already keeps the memory busy: 176 rows 36.7 -> 42.4, 192 rows
+//     70 -> 75, 208 rows 39 -> 43 (and 119 rows 152 -> 96, 8 rows 402 -> 29)
 //   more rows than units: a unit has two rows or one, and unequal rows meet badly.  268 rows 66 -> 46, 288 rows
-//     118 -> 94, 320 rows 147 -> 105; equal rows 384: 76 -> 88
-__device__ __forceinline__ bool cut_pays(int longest, int total, int live, int num_kv_heads, int units, int stay_whole) {
+//     118 -> 94, 320 rows 146 -> 105; equal rows 384: 76 -> 88
+// Head size 64, 16-bit cache (extra 1): 172 rows of 270-1153 keys 13.7 -> 15.5, 134 of 882-1300 14.8 -> 16.5, 320 of 400-1600 24.4 ->
+// 25.8, but 128 of 1497 18.5 -> 17.3, 138 of 200-2170 20.3 -> 14.9, 336 of 340-2555 40.2 -> 31.7
+__device__ __forceinline__ bool cut_pays(int longest, int total, int live, int num_kv_heads, int units, int stay_whole, int extra) {
   if (longest <= stay_whole) return false;
-  if (live * num_kv_heads <= units) return (longest - 1) * (units * 5 >> 3) > total * num_kv_heads;
-  return 4 * longest * live > 5 * total;
+  const int rows = live * num_kv_heads;
+  if (rows <= units) return (longest - 1 - (2 * rows > units ? extra : 0)) * (units * 5 >> 3) > total * num_kv_heads;
+  return (4 * longest - 6 * extra) * live > 5 * total;
 }
 
 // Live partitions of all sequences, as every wavefront of an attention launch computes them:

@@ -72,7 +72,9 @@ E5M2, E4M3 = torch.float8_e5m2, torch.float8_e4m3fn
     ([1536, 1537, 511, 512, 513], 1, 1, 128, None, 64, True),
     # more pieces than lanes; an empty row between
     ([50001, 0, 700], 1, 2, 128, None, 16, True),
-    # 16-bit rows of 128 bytes, byte rows of 128 and of 64 bytes (partitions of 512, 512, 1024 keys)
+    # 16-bit rows of 128 bytes, byte rows of 128 and of 64 bytes (partitions of 256, 512 and 512 keys)
+    ([1025, 1024, 0, 300], 2, 4, 64, None, 16, True),
+    ([1537, 1536, 40], 3, 2, 64, E5M2, 16, False),
     ([5000, 2561, 2560], 4, 3, 64, None, 32, False),
     ([5121, 2559, 9000], 2, 5, 128, E5M2, 16, False),
     ([2700, 6001], 2, 16, 128, E4M3, 16, True),
@@ -317,11 +319,12 @@ def test_calls_go_to_the_current_stream():
     ([32769, 300], 1, 4, None),        # 129: two
     ([16384, 16128], 2, 2, None),      # 254 pieces of one partition for 256 units
     ([16384, 16385], 2, 2, None),      # 258 would be: two partitions a piece
-    ([7000, 0, 513, 4097, 1], 8, 8, E5M2),  # 25 partitions x 8 kv heads, eight wavefronts a work-group
-    ([3000] * 9, 4, 1, None),          # 108 pieces, one head a kv head
+    ([7000, 0, 513, 4097, 1], 8, 8, E5M2),  # 26 partitions x 8 kv heads, eight wavefronts a work-group
+    ([3000] * 9, 4, 1, None),          # 432 partitions, one head a kv head: two partitions a piece
 ])
 def test_pieces_of_one_partition(oracle, lens, hk, group, fp8):
-    """Both sides of the rule by which a piece is one partition or two, from memory that held another batch's flags."""
+    """Results on both sides of the rule by which a piece is one partition or two (test_the_pieces_are_the_rules looks at the
+    pieces), from memory that held another batch's flags."""
     w = _workload(lens, hk, group, 128, fp8, bf16=True, sinks=True)
     assert _needs(w) > 0
     dev = torch.device("cuda:0")
@@ -329,3 +332,95 @@ def test_pieces_of_one_partition(oracle, lens, hk, group, fp8):
     torch.cuda.synchronize()
     assert torch.equal(out, again), "the order of arrival shows in the result"
     _check(oracle, w, out)
+
+
+@pytest.mark.parametrize("lens, hk, group, d, fp8, m, window", [
+    # m: partitions a piece; 0: rows stay whole; None: cut, the length follows from the launch's work-groups.  Rows on both sides of
+    # what stays whole: five partitions of 256 keys, of 512 in byte caches, also of pairs of kv heads of 64 ...
+    ([1280, 300], 2, 4, 128, None, 0, None),
+    ([1281, 300], 2, 4, 128, None, 1, None),
+    ([2560, 300], 3, 4, 128, E5M2, 0, None),
+    ([2561, 300], 3, 4, 128, E5M2, 1, None),
+    ([2560, 300], 2, 4, 64, E5M2, 0, None),
+    ([2561, 300], 2, 4, 64, E5M2, 1, None),
+    # ... four of 256 keys with head size 64, three of 512
+    ([1024, 300], 2, 4, 64, None, 0, None),
+    ([1025, 300], 2, 4, 64, None, 1, None),
+    ([1536, 300], 3, 4, 64, E5M2, 0, None),
+    ([1537, 300], 3, 4, 64, E4M3, 1, None),
+    # behind a window the keys that are seen count
+    ([5000, 300], 2, 4, 64, None, 0, 1023),
+    ([5000, 300], 2, 4, 64, None, 1, 1024),
+    # the longest row against the others: up to half the units, beyond, more rows than units
+    ([1497] * 16, 8, 1, 64, None, None, None),
+    ([1497] * 43, 3, 1, 64, None, 0, None),
+    ([400 + 1200 * k // 39 for k in range(40)], 8, 1, 64, None, 0, None),
+    ([2555] + [700] * 41, 8, 1, 64, None, None, None),
+    # a partition a piece or two: partitions x columns up to 512 and beyond, pieces for 256 units and more
+    ([32768, 300], 1, 4, 128, None, 1, None),
+    ([32769, 300], 1, 4, 128, None, 2, None),
+    ([16384, 16128], 2, 2, 128, None, 1, None),
+    ([16384, 16385], 2, 2, 128, None, 2, None),
+    ([8192, 300], 1, 16, 64, None, 1, None),
+    ([8193, 300], 1, 16, 64, None, 2, None),
+    # partitions x columns beyond 2048: 256 KiB a piece
+    ([32768, 300], 1, 16, 64, None, 2, None),
+    ([32769, 300], 1, 16, 64, None, 4, None),
+    ([65537, 300], 1, 16, 64, E5M2, 4, None),
+    ([65536, 300], 1, 16, 64, E5M2, 2, None),
+])
+def test_the_pieces_are_the_rules(oracle, lens, hk, group, d, fp8, m, window):
+    """The slots of the workspace that a call has written are those of the pieces that the rule gives, in a block table that
+    does not tell how long the rows are."""
+    dev = torch.device("cuda:0")
+    units = torch.cuda.get_device_properties(dev).multi_processor_count
+    if units != 256:
+        pytest.skip("the batches are made for 256 compute units")
+    w = _workload(lens, hk, group, d, fp8)
+    wide = torch.zeros((len(lens), max(512, w.block_tables.shape[1])), dtype=torch.int32)
+    wide[:, :w.block_tables.shape[1]] = w.block_tables
+    w.block_tables = wide
+    S, H, fill = len(lens), hk * group, 0x5A5A5A5A
+    need = _needs(w)
+    assert need > 0
+    wd = w.to(dev)
+    space = torch.full((need // 4,), fill, dtype=torch.int32, device=dev)
+    sh, op = _cabi.Shape(), _cabi.OptionsWorkspace()
+    op.workspace, op.workspace_bytes = space.data_ptr(), need
+    sh.num_seqs, sh.num_heads, sh.head_size, sh.num_kv_heads = S, H, d, hk
+    sh.block_size, sh.max_blocks_per_seq, sh.max_num_partitions = w.block_size, wide.shape[1], 1
+    sh.kv_block_stride, sh.kv_token_stride, sh.kv_head_stride = w.kv_strides()
+    sh.num_pool_blocks, sh.q_dtype = w.key_cache.shape[0], _cabi.FA_DTYPE_F16
+    op.fp8_scale, op.stream = 1.0, torch.cuda.current_stream().cuda_stream
+    op.kv_fp8_format = _cabi.FA_FP8_E4M3 if fp8 is E4M3 else _cabi.FA_FP8_E5M2
+    if window is not None:
+        op.mask_flags, op.window_left = _cabi.FA_MASK_WINDOW, window
+    out = torch.full_like(wd.query, 7.0)
+    fn = _cabi.load().fa_paged_attention_fp8_loop if fp8 else _cabi.load().fa_paged_attention_loop
+    _cabi.check(fn(out.data_ptr(), wd.query.data_ptr(), wd.key_cache.data_ptr(), wd.value_cache.data_ptr(), wd.block_tables.data_ptr(),
+                   wd.context_lens.data_ptr(), w.scale, 0, ctypes.byref(sh), ctypes.byref(op)))
+    torch.cuda.synchronize()
+    _check(oracle, w, out, **({} if window is None else dict(window_left=window)))
+    # where the pieces lie: flags for (1024 + rows) pieces x slices, then the slots
+    pairs = fp8 is not None and d == 64 and hk % 2 == 0 and 2 * group <= 16 and window is None  # (token-major pools)
+    heads, cols, head = (hk // 2, 2 * group, 128) if pairs else (hk, group, d)
+    rows = S * heads
+    most = 8 if head == 128 else 4                                          # slices that the workspace has room for
+    slices = 8 if head == 128 and window is None and 2 * rows <= units else 4  # and the launch uses: its wavefronts
+    slot = slices * ((cols * (head // slices + 2) + 3) & ~3)
+    slots = space[2 * (1024 + rows) * most:].cpu()
+    written = {k for k in range(min(1024 + rows, slots.numel() // slot)) if (slots[k * slot:(k + 1) * slot] != fill).any()}
+    if not m:
+        assert bool(written) == (m is None), len(written)
+        return
+    psize = (64 if head == 64 else 128) * 1024 // (2 * head * (1 if fp8 else 2))
+    want, before = set(), 0
+    base = [0 if window is None else max(0, n - 1 - window) // psize * psize for n in lens]
+    full = [(n - b) // (m * psize) for n, b in zip(lens, base)]
+    for s, n in enumerate(lens):
+        tail = (n - base[s]) % (m * psize) > 0
+        if full[s] + tail > 1:  # (a row of a single piece leaves nothing)
+            want |= {(before + j) * heads + h for j in range(full[s]) for h in range(heads)}
+            want |= {(sum(full) + s) * heads + h for h in range(heads) if tail}
+        before += full[s]
+    assert written == want, (sorted(written), sorted(want))
