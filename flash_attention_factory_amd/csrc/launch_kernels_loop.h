@@ -87,6 +87,14 @@ inline int row_merge_partition(int head_size, int elem_bytes) {
   return row_merge_partition_bytes(head_size) / (2 * head_size * elem_bytes);
 }
 
+// Rows that are cut only because a partition is 64 KiB with head size 64: with 128 KiB they would stay whole and their calls
+// would ask for no workspace.  A library of that kind took such a call with any workspace; so a caller that keeps to its
+// answer is not refused, and its rows stay whole.
+inline bool row_merge_may_do_without(const fa_paged_attention_shape &shape, const Resolved &r) {
+  return shape.head_size == 64 && !r.pair_heads &&
+         visible_row_bound(shape, r, 0) <= merge_whole_partitions(128, r.kv_elem_bytes) * 2 * row_merge_partition(64, r.kv_elem_bytes);
+}
+
 inline RowMergeSpace row_merge_space(const fa_paged_attention_shape &shape, const Resolved &r, int32_t max_context_len) {
   RowMergeSpace space;
   const int64_t heads = r.pair_heads ? shape.num_kv_heads / 2 : shape.num_kv_heads;
@@ -394,10 +402,11 @@ inline fa_status dispatch_paged_attention_loop_any(void *out, const void *query,
   if (workspace) {
     if ((uintptr_t)workspace % 16) return fail(FA_ERR_BAD_SHAPE, "workspace must be 16-byte aligned");
     const RowMergeSpace space = row_merge_space(*shape, r, 0);
-    if (workspace_bytes < space.bytes)
+    const bool enough = workspace_bytes >= space.bytes;
+    if (!enough && !row_merge_may_do_without(*shape, r))
       return fail(FA_ERR_SCRATCH_TOO_SMALL, "workspace of %lld bytes, this call asks for %lld", (long long)workspace_bytes,
                   (long long)space.bytes);
-    if (space.bytes > 0) {  // (else the launches, sub-batches of this call among them, have none)
+    if (space.bytes > 0 && enough) {  // (else the launches, sub-batches of this call among them, have none)
       r.workspace = workspace;
       r.workspace_bytes = workspace_bytes;
     }

@@ -226,7 +226,9 @@ int32_t fa_paged_attention_loop(void *out, const void *query, const void *key_ca
  * The workspace goes with the options: a caller passes &x.options of the struct below, whose
  * options.struct_size is the size of the whole.  workspace: device memory, 16-byte aligned, contents of no matter
  * before and after; calls that may overlap on the GPU (other streams) need one each.  NULL: none.  Less than the
- * call asks for: FA_ERR_SCRATCH_TOO_SMALL.  Entries other than the two single-pass ones do not look at it. */
+ * call asks for: FA_ERR_SCRATCH_TOO_SMALL; but where head size 64 and rows of at most 640 KiB of K and V (by the block
+ * table's width and the window; heads that do not run in pairs) make a call ask, it runs as if there were none, since
+ * libraries of this ABI version have answered 0 there.  Entries other than the two single-pass ones do not look at it. */
 typedef struct fa_paged_attention_options_workspace {
   fa_paged_attention_options options;
   void *workspace;

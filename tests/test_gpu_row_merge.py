@@ -111,6 +111,30 @@ def test_windows_modifiers_and_query_tokens(oracle, window, query_len, group):
     _check(oracle, w, out, query=query, alibi_slopes=alibi, softcap=20.0, window_left=window)
 
 
+@pytest.mark.parametrize("longest, fp8", [(2560, None), (5120, E5M2)])
+def test_too_little_workspace_for_short_rows_of_head_size_64(oracle, longest, fp8):
+    """Taken, left alone, and the rows stay whole."""
+    w = _workload([longest, 900, 0], 3, 4, 64, fp8)
+    dev = torch.device("cuda:0")
+    assert _needs(w) > 256
+    space = torch.full((256,), 0x5A, dtype=torch.uint8, device=dev)
+    wd = w.to(dev)
+    L, sh, op = _cabi.load(), _cabi.Shape(), _cabi.OptionsWorkspace()
+    op.workspace, op.workspace_bytes = space.data_ptr(), 256
+    sh.num_seqs, sh.num_heads, sh.head_size, sh.num_kv_heads = 3, 12, 64, 3
+    sh.block_size, sh.max_blocks_per_seq, sh.max_num_partitions = w.block_size, w.block_tables.shape[1], 1
+    sh.kv_block_stride, sh.kv_token_stride, sh.kv_head_stride = w.kv_strides()
+    sh.num_pool_blocks, sh.q_dtype = w.key_cache.shape[0], _cabi.FA_DTYPE_F16
+    op.fp8_scale, op.stream, op.kv_fp8_format = 1.0, torch.cuda.current_stream().cuda_stream, _cabi.FA_FP8_E5M2
+    out = torch.full_like(wd.query, 7.0)
+    fn = L.fa_paged_attention_fp8_loop if fp8 else L.fa_paged_attention_loop
+    _cabi.check(fn(out.data_ptr(), wd.query.data_ptr(), wd.key_cache.data_ptr(), wd.value_cache.data_ptr(), wd.block_tables.data_ptr(),
+                   wd.context_lens.data_ptr(), w.scale, 0, ctypes.byref(sh), ctypes.byref(op)))
+    torch.cuda.synchronize()
+    assert (space == 0x5A).all()
+    _check(oracle, w, out)
+
+
 @pytest.mark.parametrize("fill", [0x00, 0xFF, 0x7F])
 def test_contents_of_the_workspace_do_not_matter(oracle, fill):
     """Through the C ABI, twice on the same memory, without clearing it in between."""

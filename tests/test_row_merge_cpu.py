@@ -60,6 +60,27 @@ def test_argument_checks(fp8):
     assert call(p, need) == _cabi.FA_ERR_BAD_SHAPE and b"options.struct_size" in L.fa_last_error()
 
 
+@pytest.mark.parametrize("fp8, blocks, refused", [
+    # 16-bit rows of head size 64 ask from 1025 keys on, byte caches from 1537; up to 2560 and 5120 they do without
+    (0, 64, False), (0, 65, False), (0, 160, False), (0, 161, True),
+    (1, 96, False), (1, 97, False), (1, 320, False), (1, 321, True),
+])
+def test_short_rows_of_head_size_64_take_any_workspace(fp8, blocks, refused):
+    L = _cabi.load()
+    sh, _ = _call(d=64, blocks=blocks)
+    full = _cabi.OptionsWorkspace()
+    need = L.fa_paged_attention_loop_workspace_bytes(ctypes.byref(sh), ctypes.byref(_cabi.Options()), fp8)
+    assert (need > 0) == (blocks not in (64, 96))
+    full.validate_only = 1
+    room = (ctypes.c_char * 64)()
+    p = (ctypes.addressof(room) + 15) // 16 * 16
+    entry = L.fa_paged_attention_fp8_loop if fp8 else L.fa_paged_attention_loop
+    for size in (0, 16, max(need - 1, 0)):
+        full.workspace, full.workspace_bytes = p, size
+        want = _cabi.FA_ERR_SCRATCH_TOO_SMALL if refused else _cabi.FA_OK
+        assert entry(p, p, p, p, p, p, 1.0, 0, ctypes.byref(sh), ctypes.byref(full)) == want, size
+
+
 def test_calls_that_need_not_ask():
     """What lib.*.run rules out without asking, the library answers with 0."""
     asked = 0
