@@ -316,18 +316,17 @@ inline bool loop_persistent_fits(const fa_paged_attention_shape &shape) {
 }
 
 // Whether a batch of more sequences than the persistent kernel ranks, from a 16-bit cache, is one launch of the grid form
-// all the same: sub-batches pay a launch's fixed cost twice or more, the grid form starts a stream for every row.  Measured on
-// 206 batches of 130 to 512 sequences of up to 2048 keys, 260 to 4800 rows, sub-batches against grid form:
-//   head size 64    1.45 times as fast in the mean of 122, 5 % slower in two (200 sequences of 40-200 keys, 4 kv heads 14.7 -> 10.1 us)
-//   head size 128   up to 5 rows for every unit 1.34 times in the mean of 59, 3 % slower at worst (130 of 200-1000 keys, 2 kv heads 37.0 ->
-//                   23.7 us); more rows 0.96 times in the mean of 25, 0.68 at worst (150 of 12-64 keys, 32 kv heads)
-// Longer rows, and several query tokens that do not fit one column tile, stay with the sub-batches.
-constexpr int kGridBelowTokens = 2048, kGridRowsPerUnit = 5;
+// all the same (short_rows_run_as_grid).  Longer rows, and several query tokens that do not fit one column tile, stay with the
+// sub-batches; so do short rows in tables of more than 2048 keys, which the host cannot tell from long ones unless the call says
+// max_context_len.
+constexpr int kGridBelowTokens = 2048;
 inline bool large_batch_runs_as_grid(const fa_paged_attention_shape &shape, const Resolved &r, int compute_units) {
   int64_t bound = (int64_t)shape.max_blocks_per_seq * shape.block_size;
   if (r.max_context_len > 0) bound = std::min<int64_t>(bound, r.max_context_len);
   if (bound > kGridBelowTokens || r.query_len > kMaxGroup / r.group) return false;
-  return shape.head_size == 64 || (int64_t)shape.num_seqs * shape.num_kv_heads <= (int64_t)kGridRowsPerUnit * compute_units;
+  const bool ext = r.mask_flags != 0 || r.query_len > 1 || r.kv_scale_mode != 0;
+  return short_rows_run_as_grid(shape.head_size, shape.num_seqs, kLoopPersistentMaxSeqs, shape.num_kv_heads, compute_units, ext,
+                                shape.kv_token_stride != shape.head_size);
 }
 
 // A batch of more sequences than the persistent kernel ranks is cut into equal sub-batches,

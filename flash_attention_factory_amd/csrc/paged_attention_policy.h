@@ -156,6 +156,28 @@ struct PersistentLoop {
   static constexpr bool sub_batches = !kKV8;
 };
 
+// Short rows (up to 2048 keys) of 16-bit caches in a batch of more sequences than one persistent launch takes (most_seqs): one
+// launch of the grid form, or equal sub-batches, persistent?  Sub-batches pay a launch's fixed cost twice or more, the grid form
+// starts a stream for every row, so the rows that a sub-batch has for each compute unit decide.  extended: modifiers or several query
+// tokens; rows_apart: a token's K rows of adjacent kv heads lie side by side, which persistent work-groups use (two heads each) and the
+// grid form does not.  Measured on 490 batches of 129 to 691 sequences, 134 to 35200 rows (us, sub-batches -> grid form):
+//   head size 64    up to 11 rows a unit in a sub-batch 0.71 times as long in the mean of 186, 0.97 at worst (200 sequences of 40-200
+//                   keys, 4 kv heads 14.7 -> 10.1); beyond that, rows apart, 1.27 times in the mean of 40, 1.61 at worst (307 of 24-57
+//                   keys, 3 query tokens, 32 kv heads 51.5 -> 70.5), else extended 0.83 to 1.25; neither 0.84 in the mean of 19, 0.95 at
+//                   worst (325 of 12-86 keys, 32 kv heads 56.3 -> 40.5)
+//   head size 128   up to 5 rows a unit in all 0.69 times in the mean of 136, 0.95 at worst (130 of 200-1000 keys, 2 kv heads 37.0 ->
+//                   23.7); more rows 1.04 times in the mean of 25, 1.47 at worst; but extended calls of two sub-batches that keep
+//                   every row resident at once (two a unit) and leave few places empty 0.97 times in the mean of 29, 0.78 to 1.13
+//                   (215 of 16-39 keys, 2 query tokens, 4 kv heads 16.6 -> 18.4)
+constexpr bool short_rows_run_as_grid(int head_size, int num_seqs, int most_seqs, int num_kv_heads, int units, bool extended,
+                                      bool rows_apart) {
+  const int pieces = (num_seqs + most_seqs - 1) / most_seqs;
+  const long long rows = (long long)((num_seqs + pieces - 1) / pieces) * num_kv_heads;  // of a sub-batch
+  if (head_size == 64) return rows <= 11LL * units || !(extended || rows_apart);
+  if ((long long)num_seqs * num_kv_heads > 5LL * units) return false;
+  return !(extended && pieces == 2 && 2 * rows > 3LL * units && rows <= 2LL * units);
+}
+
 // ---- reduce kernel ---------------------------------------------------------------------
 // One wavefront per (sequence, head) from this many pairs on, four below.
 #ifndef FA_REDUCE_1W_MIN_PAIRS

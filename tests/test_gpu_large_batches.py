@@ -16,6 +16,11 @@ pytestmark = pytest.mark.gpu
     (160, 8, 8, 128, 100, W.HEAD_MAJOR),      # 1280 rows: five for each of 256 units
     (161, 8, 8, 128, 100, W.HEAD_MAJOR),      # more: sub-batches (bf16: groups of one head in fp16 have a kernel of their own)
     (300, 4, 1, 128, 513, W.TOKEN_MAJOR),
+    (176, 64, 32, 64, 40, W.TOKEN_MAJOR),     # 88 x 32 rows in each of two sub-batches: eleven for each unit
+    (177, 64, 32, 64, 40, W.TOKEN_MAJOR),     # more: sub-batches
+    (177, 64, 32, 64, 40, W.HEAD_MAJOR),      # sub-batches if modified
+    (192, 8, 4, 128, 60, W.HEAD_MAJOR),       # 96 x 4: one and a half
+    (193, 8, 4, 128, 60, W.HEAD_MAJOR),       # sub-batches if modified
 ])
 @pytest.mark.parametrize("mods", [{}, dict(softcap=20.0, apply_softcap=True, window_left=90)], ids=["plain", "modified"])
 def test_against_the_oracle(oracle, S, H, Hk, D, keys, layout, mods):
