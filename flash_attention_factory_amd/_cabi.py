@@ -186,10 +186,10 @@ def set_kv_scales(op: "Options", k_scales, v_scales, num_kv_heads: int, num_pool
 
 # Single-pass calls of more sequences, of more (sequence, kv head) rows, or whose block tables hold no more bytes of K
 # and V per row than this ask for no workspace (fa_paged_attention_loop_workspace_bytes): a call that can tell by that
-# spares itself the question.  (384 rows, pairs of kv heads are one; three partitions of 64 KiB with head size 64, more with 128.)
+# spares itself the question.  (384 rows, pairs of kv heads are one; by head size three partitions of 64 KiB or five of 128 KiB.)
 LOOP_WORKSPACE_MAX_SEQS = 128
 LOOP_WORKSPACE_MAX_ROWS = 2 * 384
-LOOP_WORKSPACE_MIN_HEAD_BYTES = 3 * (64 << 10)
+LOOP_WORKSPACE_MIN_HEAD_BYTES = {64: 3 * (64 << 10), 128: 5 * (128 << 10)}
 
 
 def require_same_device(anchor_name: str, anchor, named_tensors) -> None:

@@ -177,7 +177,7 @@ def run_impl(entry: str, split: bool, fp8: bool, max_logits, exp_sums, tem_outpu
                                             "max_logits/exp_sums must be contiguous fp32")
         args += [exp_sums.data_ptr(), max_logits.data_ptr(), tmp.data_ptr()]
     if not split and S <= _cabi.LOOP_WORKSPACE_MAX_SEQS and S * sh.num_kv_heads <= _cabi.LOOP_WORKSPACE_MAX_ROWS \
-            and sh.max_blocks_per_seq * block_size * 2 * D * key_cache.element_size() > _cabi.LOOP_WORKSPACE_MIN_HEAD_BYTES:
+            and sh.max_blocks_per_seq * block_size * 2 * D * key_cache.element_size() > _cabi.LOOP_WORKSPACE_MIN_HEAD_BYTES.get(D, 0):
         # few rows: memory in which they can be shared among more work-groups (from PyTorch's stream-ordered
         # allocator, so that calls that overlap on other streams, and graphs, have memory of their own)
         need = L.fa_paged_attention_loop_workspace_bytes(ctypes.byref(sh), ctypes.byref(op), int(fp8))

@@ -82,18 +82,20 @@ def test_short_rows_of_head_size_64_take_any_workspace(fp8, blocks, refused):
 
 
 def test_calls_that_need_not_ask():
-    """What lib.*.run rules out without asking, the library answers with 0."""
-    asked = 0
+    """What lib.*.run rules out without asking, the library answers with 0; the shortest tables for which it asks get some."""
+    asked, least = 0, {64: 1 << 40, 128: 1 << 40}
     for fp8, element in ((0, 2), (1, 1)):
         for d in (64, 128):
             for kv_heads in (1, 2, 3, 8, 32):
                 for seqs in (1, 12, 24, 25, 48, 49, 96, 97, 128, 129, 384, 385):
-                    for blocks in (20, 40, 41, 79, 80, 81, 160, 161, 320, 321, 4096):
+                    for blocks in (20, 40, 41, 64, 65, 79, 80, 81, 96, 97, 160, 161, 320, 321, 4096):
                         sh, op = _call(seqs=seqs, kv_heads=kv_heads, group=1, d=d, blocks=blocks)
                         sh.kv_token_stride, sh.kv_head_stride = kv_heads * d, d   # kv heads side by side, as pairs need
                         need = _cabi.load().fa_paged_attention_loop_workspace_bytes(ctypes.byref(sh), ctypes.byref(op), fp8)
                         ruled_out = (seqs > _cabi.LOOP_WORKSPACE_MAX_SEQS or seqs * kv_heads > _cabi.LOOP_WORKSPACE_MAX_ROWS or
-                                     blocks * 16 * 2 * d * element <= _cabi.LOOP_WORKSPACE_MIN_HEAD_BYTES)
+                                     blocks * 16 * 2 * d * element <= _cabi.LOOP_WORKSPACE_MIN_HEAD_BYTES[d])
                         assert not (ruled_out and need), (fp8, d, kv_heads, seqs, blocks)
                         asked += need > 0
-    assert asked > 100
+                        if need:
+                            least[d] = min(least[d], (blocks - 1) * 16 * 2 * d * element)
+    assert asked > 100 and least == _cabi.LOOP_WORKSPACE_MIN_HEAD_BYTES
