@@ -58,7 +58,7 @@ inline fa_status fail(fa_status code, const char *fmt, ...) {
 // waits for the other wavefronts of its work-group stores kStatusSpinLimit here and goes on (so
 // the grid drains) with a result that is wrong.  One word per GPU, in pinned host memory: it is written
 // hardly ever and read after every blocking call, whose host side then looks at its own memory where it had
-// to copy a word from the device and wait for the copy (the reference's measuring loop, 35 us of kernel: 82 -> 66 us
+// to copy a word from the device and wait for the copy (the reference's measuring loop, 35 us of kernel: 83 -> 70 us
 // a call).  The words live as long as the process.  Allocated at the first call; a stream that is being captured
 // does not mind (hipThreadExchangeStreamCaptureMode).
 inline fa_status kernel_status_of_current_device(int32_t **word, int32_t **device_word = nullptr) {

@@ -262,7 +262,7 @@ inline fa_status launch_paged_attn_v2_batch(void *out, const void *query, const 
     if (r.elapsed_us && q0 + per_launch < r.query_len) FA_HIP_CHECK(timer.accumulate(0, &attention_us));
   }
 
-  // kernel 2: one wavefront per (head, sequence)
+  // kernel 2: sixteen, four or one wavefront per (sequence, query token, head) -- kReduceSingleWaveMinPairs has the rule
   ReduceParams rp;
   rp.out = out;
   rp.exp_sums = exp_sums;

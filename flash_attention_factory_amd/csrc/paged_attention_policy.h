@@ -179,7 +179,7 @@ constexpr bool short_rows_run_as_grid(int head_size, int num_seqs, int most_seqs
 }
 
 // ---- reduce kernel ---------------------------------------------------------------------
-// One wavefront per (sequence, head) from this many pairs on, four below.
+// One wavefront per (sequence, query token, head) from this many pairs on, four below.
 #ifndef FA_REDUCE_1W_MIN_PAIRS
 #define FA_REDUCE_1W_MIN_PAIRS 4096
 #endif

@@ -62,11 +62,12 @@ __device__ __forceinline__ void load_row(float (&v)[EPL], const float *at) {
   }
 }
 
-// kReduceWaves wavefronts per (sequence, head): 4 when there are few (sequence, head)
-// pairs -- the launch is then short of parallelism and each pair's rows should be in
-// flight at once -- 1 when there are thousands and every wavefront slot of the GPU is
-// filled anyway (no LDS, no barrier, more groups resident).
-// Every live slot holds a partial (the grid form of the attention kernels).
+// Wavefronts per (sequence, head), kReduceWaves, in both bodies below (the rule with its figures: kReduceSingleWaveMinPairs):
+//   4    few pairs: the launch is short of parallelism and each pair's rows should be in flight at once
+//   1    thousands: every wavefront slot of the GPU is filled anyway (no LDS, no barrier, more groups resident); after the
+//        segment kernels kReducePairs pairs share a work-group
+//   16   after the segment kernels, up to kReduceAheadMaxPairs pairs: rows are asked for before it is known which count
+// This body: every live slot holds a partial (the grid form of the attention kernels).
 template <int D, typename QT, int kReduceWaves>
 __device__ __forceinline__ void reduce_every_partition(const ReduceParams &p) {
   constexpr bool SEGMENTS = false;

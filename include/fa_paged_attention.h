@@ -208,8 +208,10 @@ typedef struct fa_paged_attention_options {
 } fa_paged_attention_options;
 #define FA_PAGED_ATTENTION_OPTIONS_INIT {(uint32_t)sizeof(fa_paged_attention_options)}
 
-/* Single-pass kernel: no scratch.  One launch for a decode batch of up to 128 sequences; larger
- * batches and query blocks of more than 32 (token, head) columns per kv head take several. */
+/* Single-pass kernel: no scratch.  One launch for a decode batch of up to 128 sequences.  A larger
+ * one is one launch too (byte caches; 16-bit caches with one query head per kv head or with rows that the block
+ * tables' width or max_context_len bounds to 2048 keys) or a launch for each of its equal parts of at most 128.  Query
+ * blocks of more (token, head) columns per kv head than a launch holds (32, or 16 in the grid form) take several. */
 int32_t fa_paged_attention_loop(void *out, const void *query, const void *key_cache,
                                 const void *value_cache, const int32_t *block_tables,
                                 const int32_t *context_lens, float scale, int32_t max_context_len,

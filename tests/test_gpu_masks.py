@@ -115,7 +115,8 @@ def _call_multi(w, query4, kernel, **mods):
         head.append(w.fp8_scale)
     alibi, softcap = mods.pop("alibi_slopes", None), mods.pop("softcap", 0.0)
     extra = dict(partition_size=w.partition_size) if "reduce" in kernel else {}
-    times = mod.run(*head, w.block_size, int(w.context_lens.max()), alibi, w.sinks, softcap, **extra, **mods)
+    longest = mods.pop("max_context_len", int(w.context_lens.max()))
+    times = mod.run(*head, w.block_size, longest, alibi, w.sinks, softcap, **extra, **mods)
     if "reduce" in kernel and times[1] == 0.0:
         # rows so short that the split entry ran the single-pass kernel; this test is after the split kernels
         mod.run(*head, w.block_size, int(w.context_lens.max()), alibi, w.sinks, softcap, schedule=3, **extra, **mods)
@@ -207,9 +208,9 @@ def test_query_tokens_head_major_e4m3(oracle):
 
 def test_extended_instances_in_every_scheduling_form(oracle):
     """Modifiers + two query tokens on a batch that the persistent kernels take whole (120
-    sequences, several items per work-group, empty sequences in between), on one they take as
-    sub-batches (300 sequences) and on one left to the grid form (a table of 2^24 tokens per
-    sequence)."""
+    sequences, several items per work-group, empty sequences in between), on one that the split kernels take
+    as sub-batches and the loop entry in the grid form (300 sequences; told of rows of up to 2049 keys, in
+    sub-batches as well) and on one left to the grid form (a table of 2^24 tokens per sequence)."""
     for S, seed, wide in ((120, 31, False), (300, 32, False), (9, 33, True)):
         gen = torch.Generator().manual_seed(seed)
         lens = torch.randint(1, 1500, (S,), generator=gen)
@@ -237,6 +238,11 @@ def test_extended_instances_in_every_scheduling_form(oracle):
             got = _call_multi(wd, query4.to(_dev()), kernel, **dict(mods)).float().cpu()
             assert (got[~live] == 0).all(), (S, kernel)          # empty sequences: rows untouched
             assert_close_to_reference(got[live], ref[live], f"S={S} {kernel}")
+        if S > 128:
+            wd.block_tables = torch.cat([wd.block_tables, torch.zeros((S, 2064 // w.block_size), dtype=torch.int32, device=_dev())], 1)
+            got = _call_multi(wd, query4.to(_dev()), "loop", max_context_len=2049, **dict(mods)).float().cpu()
+            assert (got[~live] == 0).all()
+            assert_close_to_reference(got[live], ref[live], f"S={S} loop in sub-batches")
 
 
 @pytest.mark.parametrize("QL,nheads,nheads_k", [(4, 16, 2), (7, 8, 2), (33, 2, 2), (3, 16, 1)])

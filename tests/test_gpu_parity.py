@@ -39,6 +39,12 @@ def _run(w_cpu, kernel, max_context_len=None, schedule=0, spin_limit=0, timed=Tr
     return bufs, times
 
 
+def _wide(block_tables, columns):
+    table = torch.zeros((block_tables.shape[0], columns), dtype=torch.int32)
+    table[:, :block_tables.shape[1]] = block_tables
+    return table
+
+
 def _check(out, w_cpu, oracle, label, literal_rule=False):
     ref16, ref32 = call_oracle(oracle.attention_ref, w_cpu, want_f32=True)
     got = out.float().cpu()
@@ -284,7 +290,8 @@ def test_edge_cases(oracle):
 
 def test_large_batch_runs_as_sub_batches(oracle):
     """More sequences than the persistent kernels list (256 split, 128 loop): the launchers cut
-    the batch into equal sub-batches, one persistent launch each."""
+    the batch into equal sub-batches, one persistent launch each.  The loop launcher gives short rows of
+    16-bit caches to the grid form in one launch; in a table of more than 2048 keys it cannot tell."""
     gen = torch.Generator().manual_seed(5)
     lens = torch.randint(1, 700, (300,), generator=gen).tolist()
     w = W.make_config(0, num_seqs=300, pool_blocks=300 * 44, lens=lens)
@@ -292,6 +299,9 @@ def test_large_batch_runs_as_sub_batches(oracle):
     for kernel in ("reduce", "loop"):
         bufs, _ = _run(w, kernel)
         _check(bufs.out, w, oracle, f"300 sequences/{kernel}")
+    w.block_tables = _wide(w.block_tables, 2064 // w.block_size)
+    bufs, _ = _run(w, "loop")
+    _check(bufs.out, w, oracle, "300 sequences in a wide table/loop")
 
 
 def test_persistent_split_many_items_per_wavefront(oracle):
@@ -602,7 +612,8 @@ def test_full_size_configs(oracle, index, layout):
 def test_persistent_kernels_small_batches(oracle):
     """Fewer items than resident work-groups, a single sequence, a batch where most
     wavefronts of a loop work-group have no chunk, and 128 sequences (the limit of the
-    persistent loop kernel) next to 129 (two sub-batches of 65 and 64)."""
+    persistent loop kernel) next to 129 (one launch of the grid form; in a table of more than
+    2048 keys two sub-batches of 65 and 64)."""
     cases = [
         W.make_config(1, num_seqs=1, pool_blocks=200, lens=[1999]),
         W.make_config(0, num_seqs=3, pool_blocks=64, lens=[5, 40, 33]),
@@ -614,6 +625,9 @@ def test_persistent_kernels_small_batches(oracle):
         for kernel in (("fp8_loop", "fp8_reduce") if w.is_fp8 else ("loop", "reduce")):
             bufs, _ = _run(w, kernel)
             _check(bufs.out, w, oracle, f"{w.name} S={w.num_seqs}/{kernel}")
+    w.block_tables = _wide(w.block_tables, 2064 // w.block_size)
+    bufs, _ = _run(w, "loop")
+    _check(bufs.out, w, oracle, f"{w.name} S={w.num_seqs}/loop in a wide table")
 
 
 def test_table_wider_than_the_persistent_loop_key(oracle):
