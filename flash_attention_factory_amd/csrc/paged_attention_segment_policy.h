@@ -303,13 +303,15 @@ __device__ __forceinline__ long long whole_rows_of_first_group(const int (&steps
 //     8 kv heads, 16-bit cache 26.4 -> 28.4), and 4/3 with head size 64, whose partials are half as large (34 of 4748-10618, 4 teams
 //     of kv heads, 16-bit cache 101.7 -> 106.8)
 // The batch's keys are added up only where a bound is in keys: every instruction here lies before the first load of a launch (0.5 us
-// where they always were).
+// where they always were).  A batch with a unit for every partition leaves at once, with what the rest would give.
 constexpr int kTwoTileWholeExcess = 480 << 10, kTwoTileWholeExcessTeams = 192 << 10;
 constexpr int kTwoTileSegmentExcess128 = 280 << 10, kTwoTileSegmentExcess64 = 224 << 10;
 template <int NQ, int D>
 __device__ __forceinline__ int two_tile_partitions_per_segment(const int (&ctxv)[NQ], const int (&parts)[NQ], int total_partitions,
                                                                int S, int partition_size, int num_kv_heads, int groups, int units,
                                                                int key_bytes, bool teams) {
+  const long long items = (long long)total_partitions * num_kv_heads;
+  if (items <= units) return 1;
   int longest = 0, live = 0;
 #pragma unroll
   for (int j = 0; j < NQ; ++j) {
@@ -317,7 +319,7 @@ __device__ __forceinline__ int two_tile_partitions_per_segment(const int (&ctxv)
     if (j * 64 < S) live += __builtin_popcountll(__ballot(parts[j] > 0));
   }
   longest = __builtin_amdgcn_readfirstlane(__reduce_max_sync(~0ull, longest));
-  const long long items = (long long)total_partitions * num_kv_heads, rows = (long long)live * num_kv_heads;
+  const long long rows = (long long)live * num_kv_heads;
   const bool whole = longest <= kSegmentMaxPartitions && 3LL * longest * units <= 4 * items;
   if (whole && rows < 2 * groups) return max(longest, 1);  // (work-group 0 gets one row)
   if (rows > (whole ? (1 << 24) - 1 : units)) return 0;

@@ -123,14 +123,18 @@ TWO_TILE_SEGMENT_EXCESS = {128: 280 << 10, 64: 224 << 10}
 
 
 def two_tile_partitions_per_segment(lens, *, head_size: int, partition_size: int, max_num_partitions: int, max_ctx: int,
-                                    num_kv_heads: int, groups: int, cus: int, rows_apart: bool, partition_bytes: int, teams: bool) -> int:
-    """The rule of the kernels of two column tiles, and partitions_per_segment where it has no opinion."""
+                                    num_kv_heads: int, groups: int, cus: int, rows_apart: bool, partition_bytes: int, teams: bool,
+                                    leave_early: bool = True) -> int:
+    """The rule of the kernels of two column tiles, and partitions_per_segment where it has no opinion.  (leave_early: with
+    a unit for every partition the kernels leave before the rest, which would give the same.)"""
     ctx, parts = live_partitions(lens, partition_size, max_num_partitions, max_ctx)
     units = min(groups, cus)
     steps = [(min(c, p * partition_size) + 16) >> 5 for c, p in zip(ctx, parts)]
     longest, rows = max(parts), sum(p > 0 for p in parts) * num_kv_heads
     items, load = sum(parts) * num_kv_heads, sum(steps) * num_kv_heads
     step_bytes = 32 * (partition_bytes // partition_size)
+    if leave_early and items <= units:
+        return 1
     whole = longest <= SEGMENT_MAX_PARTITIONS and 3 * longest * units <= 4 * items
     if whole and rows < 2 * groups:
         return max(longest, 1)

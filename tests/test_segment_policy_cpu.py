@@ -144,8 +144,27 @@ def test_two_tile_rule_constants_are_the_ones_replayed():
     src = open(os.path.join(os.path.dirname(HERE), "flash_attention_factory_amd", "csrc", "paged_attention_segment_policy.h")).read()
     for literal in ("kTwoTileWholeExcess = 480 << 10", "kTwoTileWholeExcessTeams = 192 << 10", "kTwoTileSegmentExcess128 = 280 << 10",
                     "kTwoTileSegmentExcess64 = 224 << 10", "3LL * longest * units <= 4 * items", "rows < 2 * groups",
-                    "6 * excess <= load", "partition_size * key_bytes > 128 << 10"):
+                    "6 * excess <= load", "partition_size * key_bytes > 128 << 10", "if (items <= units) return 1;"):
         assert literal in src, literal
+
+
+def test_two_tile_rule_with_a_unit_for_every_partition():
+    """Leaving early changes nothing."""
+    rng, checked = random.Random(5), 0
+    while checked < 3000:
+        d, fp8, heads = rng.choice([64, 128]), rng.random() < 0.5, rng.choice([1, 2, 4, 5, 8, 16, 32])
+        size = rng.choice([64, 128, 256, 512, 1024, 4096])
+        hi = rng.choice([1, 100, 500, 2000, 9000, 40000])
+        lens = [rng.choice([0, rng.randint(0, hi), hi]) for _ in range(rng.randint(1, 64))]
+        items = sum(-(-n // size) for n in lens) * heads
+        if items == 0 or items > 256:
+            continue
+        checked += 1
+        slots = -(-max(lens) // size)
+        args = _two_tile_args(head_size=d, partition_size=size, max_num_partitions=slots, max_ctx=slots * size, num_kv_heads=heads,
+                              groups=rng.randint(items, 256), rows_apart=rng.random() < 0.5, partition_bytes=size * 2 * d * (1 if fp8 else 2),
+                              teams=rng.random() < 0.3)
+        assert P.two_tile_partitions_per_segment(lens, **args, leave_early=False) == 1, (lens, args)
 
 
 def test_two_tile_rows_stay_whole_only_where_the_deal_balances():
