@@ -186,10 +186,12 @@ constexpr bool short_rows_run_as_grid(int head_size, int num_seqs, int most_seqs
 constexpr int kReduceSingleWaveMinPairs = FA_REDUCE_1W_MIN_PAIRS;
 // After the segment kernel also:
 //  * sixteen for up to kReduceAheadMaxPairs pairs of up to kReduceAheadMaxPartitions slots: the launch lasts as long as its trips
-//    to memory follow one another, and sixteen wavefronts ask for a pair's first 64 rows of tmp_out together with the
-//    scalars that say which of them count (us a call, four wavefronts -> sixteen: 32 pairs of 59 slots 29.4 -> 25.6, 64 of 32
-//    25.4 -> 24.0, 128 of 16 24.8 -> 24.1; 256 of 8 24.2 both, 256 of 32 67.0 -> 67.2, 512 of 16 68.0 -> 69.1, and
-//    32 of 235, most of them beyond the first 64, 25.0 -> 26.0)
+//    to memory follow one another, and sixteen wavefronts ask for a pair's first 16 rows of tmp_out together with the
+//    scalars that say which of them count, and for all others as soon as the length has come (us a call, four wavefronts ->
+//    sixteen: 32 pairs of 59 slots 29.4 -> 25.8, 64 of 32 30.3 -> 28.1, 128 of 16 29.2 -> 28.1, with head size 64 32 of 86 17.5 -> 16.1,
+//    32 of 118 20.0 -> 18.2, 16 of 125 21.2 -> 13.6; 256 of 8 24.2 both, 256 of 32 67.0 -> 67.2, 512 of 16 68.0 -> 69.1).
+//    (Asking for the first 64 whatever the length gains 0.1 us more where all of them count, and costs 0.3 to 1.2 where the
+//    scratch arrays are wider than the rows: 80 pairs of 64 slots of which one counts 15.7 -> 16.6, 128 of which three do 15.2 -> 15.7)
 //  * where one wavefront takes a pair, kReducePairs of them in a work-group: thousands of work-groups of one wavefront, most of
 //    which find nothing to do, are launched more slowly than they run (12288 pairs 75.2 -> 74.2; 4, 8 and 16 alike)
 #ifndef FA_REDUCE_AHEAD_MAX_PAIRS
@@ -198,6 +200,7 @@ constexpr int kReduceSingleWaveMinPairs = FA_REDUCE_1W_MIN_PAIRS;
 constexpr int kReduceAheadMaxPairs = FA_REDUCE_AHEAD_MAX_PAIRS;
 constexpr int kReduceAheadMaxPartitions = 128;
 constexpr int kReduceAheadWaves = 16;
+static_assert(kReduceAheadMaxPartitions % 64 == 0, "whole groups of 64 slots in registers");
 #ifndef FA_REDUCE_PAIRS
 #define FA_REDUCE_PAIRS 8
 #endif

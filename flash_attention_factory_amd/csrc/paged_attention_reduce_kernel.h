@@ -193,14 +193,12 @@ __device__ __forceinline__ void reduce_marked_partials(const ReduceParams &p) {
   // the row turns out to have that many partitions, so that one wait covers both (slots past the
   // live ones are read and dropped: they lie inside the row).
   const int first_slots = min(p.max_num_partitions, 64);
-  // kAhead: so are the rows of tmp_out of those slots, whether or not they hold a partial
+  // kAhead: so are the rows of tmp_out of the first kReduceWaves slots, whether or not they hold a partial, and all others
+  // as soon as the length has come
   constexpr bool kAhead = kReduceWaves == kReduceAheadWaves;
-  constexpr int RA = kAhead ? 64 / kReduceWaves : 1;
+  constexpr int RA = kAhead ? kReduceAheadMaxPartitions / kReduceWaves : 1;
   float ahead[RA][EPL];
-  if constexpr (kAhead) {
-#pragma unroll
-    for (int u = 0; u < RA; ++u) load_row<EPL>(ahead[u], tmp + (int64_t)min(wave + kReduceWaves * u, first_slots - 1) * D);
-  }
+  if constexpr (kAhead) load_row<EPL>(ahead[0], tmp + (int64_t)min(wave, first_slots - 1) * D);
   const int my_slot = min(lane, first_slots - 1);  // (no branch around a load; a lane past the last slot drops what it reads)
   const float ml_first = ml[my_slot];
   const float es_first = es[my_slot];
@@ -215,6 +213,11 @@ __device__ __forceinline__ void reduce_marked_partials(const ReduceParams &p) {
     // one partial: the segment kernel has stored it into `out` as the row's result
     // (PagedAttnParams::final_out), and its tmp_out row holds nothing
     if (np == 1) return;
+  }
+  if constexpr (kAhead) {
+#pragma unroll
+    for (int u = 1; u < RA; ++u)
+      if (wave + kReduceWaves * u < np) load_row<EPL>(ahead[u], tmp + (int64_t)(wave + kReduceWaves * u) * D);  // wave-uniform
   }
 
   // Partitions are handled in groups of 64 (lane q of the wavefront holds the weight of
@@ -240,6 +243,29 @@ __device__ __forceinline__ void reduce_marked_partials(const ReduceParams &p) {
   for (int e = 0; e < EPL; ++e) acc[e] = 0.f;
   float W = 0.f;
   int nth = 0;  // partials met so far: wavefront w takes those with nth % kReduceWaves == w
+  if constexpr (kAhead) {
+#pragma unroll
+    for (int u0 = 0; u0 < RA; u0 += 64 / kReduceWaves) {
+      const int g0 = u0 * kReduceWaves, ql = g0 + lane;
+      if (g0 >= np) break;
+      const float m_q = g0 == 0 ? ml_first : (ql < np ? ml[ql] : -INFINITY);
+      const bool there = holds_partial(ql, m_q);
+      const float e_q = g0 == 0 ? es_first : (there ? es[ql] : 0.f);
+      const float w_lane = there ? e_q * __expf(m_q - M) : 0.f;
+      W += w_lane;
+      const unsigned long long todo = __ballot(there);
+#pragma unroll
+      for (int u = 0; u < 64 / kReduceWaves; ++u) {
+        const int q = wave + kReduceWaves * u;
+        if (todo >> q & 1) {  // wave-uniform; a row without a partial may hold anything
+          const float w = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(w_lane), q));
+#pragma unroll
+          for (int e = 0; e < EPL; ++e) acc[e] += w * ahead[u0 + u][e];
+        }
+      }
+    }
+    np = 0;  // nothing is left
+  }
   for (int g0 = 0; g0 < np; g0 += 64) {
     const int ql = g0 + lane;
     const float m_q = g0 == 0 ? ml_first : (ql < np ? ml[ql] : -INFINITY);
@@ -248,20 +274,6 @@ __device__ __forceinline__ void reduce_marked_partials(const ReduceParams &p) {
     const float w_lane = there ? e_q * __expf(m_q - M) : 0.f;
     W += w_lane;
     unsigned long long todo = __ballot(there);
-    if constexpr (kAhead) {
-      if (g0 == 0) {
-#pragma unroll
-        for (int u = 0; u < RA; ++u) {
-          const int q = wave + kReduceWaves * u;
-          if (todo >> q & 1) {  // wave-uniform; a row without a partial may hold anything
-            const float w = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(w_lane), q));
-#pragma unroll
-            for (int e = 0; e < EPL; ++e) acc[e] += w * ahead[u][e];
-          }
-        }
-        continue;
-      }
-    }
     while (todo) {  // wave-uniform: R rows of tmp_out per wavefront in flight at a time
       int slot[R];
       float v[R][EPL];
